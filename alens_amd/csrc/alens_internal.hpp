@@ -151,12 +151,13 @@ struct ZeroJobs {
 HipErr launch_zero_many(hipStream_t st, const ZeroJobs &z);
 // End of a captured step: the counts, clock readings, barrier abort word and solver reports gathered
 // into one buffer (read back with one copy): tail[0..4] = entries, pairs, adjacency slots, valid rows,
-// chunks; tail[5..8] = clock readings; tail[9] = abort word; tail[16 ..] = the FP64 reports (nrep
-// words), then the FP32 ones when out32 is given.
+// chunks; tail[5..8] = clock readings; tail[9] = abort word; tail[10] = resident plans that did
+// not fit (*plan, or 0); tail[16 ..] = the FP64 reports (nrep words), then the FP32 ones when out32
+// is given.
 constexpr int kTailHead = 16;
 HipErr launch_step_tail(hipStream_t st, const uint32_t *entries, const uint32_t *pairs, const uint32_t *slots,
                         const uint32_t *rows, const int32_t *chunks, const uint64_t *stamps, const uint32_t *abort_word,
-                        const double *out, const double *out32, int nrep, double *tail);
+                        const double *out, const double *out32, int nrep, const int32_t *plan, double *tail);
 HipErr launch_cell_ranges(hipStream_t st, const uint32_t *keys, int64_t E, uint32_t *cstart,
                           uint32_t *cend, const uint32_t *Ed = nullptr);
 HipErr launch_sweep(hipStream_t st, const RodsDev &r, const CfgDev &c, const uint32_t *keys, int64_t E,
@@ -205,7 +206,8 @@ constexpr int kSlice = 64;
 constexpr int kOrderWin = 1024;
 constexpr int kOrderWinPasses = 128;
 inline int slot_order_window(int64_t n, int ncu) { return n > (int64_t)ncu * kOrderWin ? kOrderWinPasses : kOrderWin; }
-HipErr launch_slot_order(hipStream_t st, int32_t n, const uint32_t *rowStart, const uint32_t *jStart,
+// A system's rods stay together: system s holds the positions of its rod range.
+HipErr launch_slot_order(hipStream_t st, int32_t n, const int32_t *rsys, const uint32_t *rowStart, const uint32_t *jStart,
                          const uint32_t *extStart, uint32_t *sord, uint32_t *spos, int win);
 HipErr launch_slice_sizes(hipStream_t st, int32_t n, const uint32_t *rowStart, const uint32_t *jStart,
                           const uint32_t *extStart, uint32_t *slice_len, const uint32_t *sord = nullptr);
@@ -316,7 +318,64 @@ constexpr int kBarXcc = 16;  // XCC id slots (the hardware field is 4 bits wide)
 // MI355X's last-level (Infinity) cache, which serves data that HBM has already sent once
 constexpr double kLastLevelCacheBytes = 256.0 * 1024 * 1024;
 constexpr int kBarXccArr = 2 + kBarGroups, kBarXccSize = kBarXccArr + kBarXcc, kBarSetup = kBarXccSize + kBarXcc;
-constexpr int kBarTotalWords = (kBarSetup + 1) * kBarWords;
+constexpr int kBarTicket = kBarSetup + 1;  // next share of a resident solve (k_resident.hip)
+constexpr int kBarTotalWords = (kBarTicket + 1) * kBarWords;
+
+// ---- solves whose operator stays on the chip (k_resident.hip) ----
+// LDS of a block: adjacency slots take their six weights; another part holds the slots' values and, at other
+// times, the velocities of the rods the block's rows touch.
+constexpr uint32_t kResidentPool = 160512;
+// Adjacency slots a block holds with g row groups.  With one group (and in FP32 two) the velocities of all
+// 1,024 g rods its rows can name fit beside them; with more, 784 of 2,048 (FP32: 1,560 of 4,096), else the rows
+// read them from memory.
+template <typename T>
+constexpr uint32_t resident_slots(int g) {
+    return sizeof(T) == 8 ? (g == 1 ? 2304 : 2560) : (g == 1 ? 3072 : (g == 2 ? 3584 : 4608));
+}
+// most 256-lane row groups (chunks) per block: with more, the rows' registers no longer fit
+template <typename T>
+constexpr int resident_groups() {
+    return sizeof(T) == 8 ? 2 : 4;
+}
+// A plan on the device: words 0..3 = {every share of the FP64 solve fits, its shares, the step's padded slots,
+// its chunks}, words 4..7 = {the FP32 solve's shares fit, its shares, wanted plans that do not fit (1: FP64, 2:
+// FP32), chunks}, then both solves' shares.
+struct ShareCut {
+    uint32_t sys, index, of;  // share `index` of the system's `of`
+    uint32_t p0, p1;          // its slice positions
+    uint32_t s0, slots;       // slots before the first of them, and its own
+    uint32_t pad;
+};
+constexpr int kPlanShares = 1 << 14;
+constexpr int kPlanHead = 4, kPlanUnfit = kPlanHead + 2;
+constexpr size_t kPlanWords = 2 * kPlanHead + 2 * (size_t)kPlanShares * (sizeof(ShareCut) / 4);
+struct ResidentPlanArgs {
+    int32_t nsys;
+    const SysDev *sys;
+    const uint32_t *sellStart;
+    uint32_t nslices;
+    uint32_t *con_off, *chunk_off;
+    int32_t *nchunks;
+    int gpb[2];               // row groups per block of the FP64 and the FP32 solve, 0 = not wanted
+    uint32_t max_shares[2];   // blocks of the launch: the most shares one system may take
+    uint32_t *mv;             // captured step: a plan that does not fit leaves no rows to solve
+    int32_t *plan;
+};
+HipErr launch_resident_plan(hipStream_t st, const ResidentPlanArgs &p);
+template <typename T>
+struct ResidentArgs {
+    SolveArgsT<T> s;
+    void *ex;                   // exchange memory, resident_exchange_bytes(m, n, nchunks)
+    const uint32_t *spos;       // slice position of each rod, NULL = identity
+    const int32_t *head;        // the plan's head and shares for this solve
+    const ShareCut *share;
+};
+// bytes of exchange memory (at most 4 GiB - 1) of a solve of m rows, n rods and nchunks chunks
+template <typename T>
+size_t resident_exchange_bytes(double m, double n, double nchunks);
+// one launch; keep_abort: an earlier launch of the same captured step may have set the abort word
+template <typename T>
+HipErr launch_resident(hipStream_t st, const ResidentArgs<T> &r, int gpb, int grid, bool keep_abort);
 
 // learned warm start (k_mlp.hip): 12 -> 64 -> 64 -> 64 -> 1; W1 stored 64 x 16 (columns 12..15 zero)
 constexpr int kMlpIn = 12;

@@ -66,6 +66,7 @@ struct alens_ctx {
     const uint32_t *sord_cur = nullptr, *spos_cur = nullptr;  // the last step's (NULL: identity)
     DBuf<double> sellW;
     uint64_t epad = 0;  // padded entry count of the sliced adjacency (component stride of sellW)
+    uint64_t slots = 0; // padded entries the last step used (epad of a captured step is a capacity)
 
     DBuf<double2> xg;
     DBuf<double> gamma, part, out;
@@ -120,6 +121,18 @@ struct alens_ctx {
     DBuf<double> pgam;
     uint32_t mprev = 0;
     bool have_prev = false;
+
+    // resident solves (k_resident.hip) of the current step buffers: row groups per block and blocks of the
+    // FP64 and the FP32 solve (0 groups: the general kernel), their device plan and exchange buffers
+    struct Route {
+        int gpb[2] = {0, 0}, grid[2] = {0, 0};
+        bool stream_nt[2] = {false, false};
+    };
+    Route route;
+    DBuf<SysDev> sys_one;                  // the one system of a stand-alone solve
+    DBuf<int32_t> plan;
+    DBuf<unsigned char> rex;
+    double resident_limit[2] = {1e300, 1e300};  // slots below which captures try a resident solve (lowered when it did not fit)
 
     int64_t m = 0, E = 0;
     int32_t nchunks_cur = 0, nsys_cur = 1;
@@ -274,6 +287,7 @@ void alens_destroy(alens_ctx *ctx) {
     rel(ctx->cImg); rel(ctx->delta0); rel(ctx->geo); rel(ctx->posI); rel(ctx->posJ); rel(ctx->b);
     rel(ctx->adjStart); rel(ctx->sellStart); rel(ctx->sellK); rel(ctx->slen); rel(ctx->sellW); rel(ctx->xg); rel(ctx->gamma); rel(ctx->part);
     rel(ctx->out); rel(ctx->bar); rel(ctx->pkey); rel(ctx->pgam);
+    rel(ctx->sys_one); rel(ctx->plan); rel(ctx->rex);
     rel(ctx->out32); rel(ctx->dword); rel(ctx->nch_dev); rel(ctx->step_dev);
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
@@ -293,6 +307,7 @@ alens_status alens_set_systems(alens_ctx *ctx, int32_t nsys, const int32_t *rod_
     if (ctx) {
         drop_graph(ctx);
         ctx->have_counts = false;
+        ctx->resident_limit[0] = ctx->resident_limit[1] = 1e300;
     }
     if (!ctx) return ALENS_E_ARG;
     if (nsys < 1 || nsys > kMaxSys || !rod_offset || !boxes || rod_offset[0] != 0)
@@ -691,7 +706,54 @@ struct SolveMem {
     uint32_t *bar;
     const uint32_t *con_off, *chunk_off;
     const int32_t *chunk_sys;
+    const int32_t *plan;  // the rows' resident plan, or NULL: the general kernel
 };
+
+// An explicit schedule in the environment names the general kernel, whose schedule it is.
+static bool schedule_named() {
+    for (const char *v : {"ALENS_SOLVER_MAX_BLOCKS", "ALENS_BARRIER_MODE", "ALENS_XCD_MAP", "ALENS_SOLVER_ENTRIES",
+                          "ALENS_GROUP_WIDTH", "ALENS_STREAM_HINT", "ALENS_SOLVER_SPLIT"})
+        if (getenv(v)) return true;
+    return false;
+}
+
+// Bytes of one iteration of the general kernel (per constraint 2 (9w + 8) + 5w, per rod 18w): its row streams
+// load non-temporally when they overflow the GPU's last-level cache, which otherwise keeps them between
+// iterations.
+static double general_iter_bytes(size_t w, double rows, double rods) {
+    return (double)w * (23.0 * rows + 18.0 * rods) + 16.0 * rows;
+}
+
+// Row groups (chunks) per block of a resident solve of T with `chunks` chunks on `blocks` blocks: the fewest
+// that give every chunk a group; with many systems, which need not run all at once, the most; 0 when one
+// system's chunks do not fit at all.
+template <typename T>
+static int resident_gpb(double chunks, int32_t nsys, int blocks) {
+    for (int g = 1; g <= resident_groups<T>(); g *= 2)
+        if (chunks <= (double)g * blocks) return g;
+    return nsys > 1 ? resident_groups<T>() : 0;
+}
+
+// The kernels for a step of `rows` rows and `slots` padded adjacency slots: resident where the operator fits
+// on the chip (the plan on the device has the last word; it fills a block's slots to 15/16), else general.  The
+// resident kernel is the faster one wherever it fits: per iteration 9.2 us against 13.7 at 800 rows, 11.4 against
+// 29 at 107k, in FP32 22.9 against 31 at 472k, near the largest it holds; a batch's systems, which then stop and
+// start one by one, 8.2 ms against 10.8 for 64 systems of 1.37M rows.
+static alens_ctx::Route want_route(const alens_ctx *ctx, double rows, double slots) {
+    alens_ctx::Route r;
+    r.stream_nt[0] = general_iter_bytes(8, rows, ctx->n) > kLastLevelCacheBytes;
+    r.stream_nt[1] = general_iter_bytes(4, rows, ctx->n) > kLastLevelCacheBytes;
+    if (schedule_named() || resident_exchange_bytes<double>(1.5 * rows + 4096, ctx->n, rows / kRedChunk * 1.5 + ctx->nsys + 8) >= 0xffffffffull)
+        return r;  // (offsets in the exchange memory are 32 bits)
+    const double chunks = std::ceil(rows / kRedChunk) + (ctx->nsys > 1 ? ctx->nsys : 0);
+    const bool one = ctx->nsys == 1;
+    if (!one || slots <= 0.937 * ctx->ncu * resident_slots<double>(resident_groups<double>()))
+        r.gpb[0] = resident_gpb<double>(chunks, ctx->nsys, ctx->ncu);
+    if (ctx->cfg.precision == 1 && (!one || slots <= 0.937 * ctx->ncu * resident_slots<float>(resident_groups<float>())))
+        r.gpb[1] = resident_gpb<float>(chunks, ctx->nsys, ctx->ncu);
+    for (int f = 0; f < 2; ++f) r.grid[f] = ctx->ncu;
+    return r;
+}
 
 template <typename T>
 static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem &mem, alens_solve_report *rep,
@@ -707,8 +769,12 @@ static alens_status run_bbpgd(alens_ctx *ctx, SolveArgsT<T> a, alens_solve_repor
     TRY_HIP(ctx->part.ensure((size_t)kRedQ * std::max<int32_t>(ctx->nchunks_cur, 1)));
     TRY_HIP(ctx->out.ensure(8 * (size_t)ns + 8));
     TRY_HIP(ctx->out32.ensure(8 * (size_t)ns + 8));
+    const bool res = ctx->route.gpb[sizeof(T) == 8 ? 0 : 1] > 0 && !ctx->tuning;
+    if (res) {
+        TRY_HIP(ctx->rex.ensure(resident_exchange_bytes<T>(a.m, a.n, ctx->nchunks_cur)));
+    }
     const SolveMem mem{ctx->part.p, sizeof(T) == 8 ? ctx->out.p : ctx->out32.p, ctx->bar.p,
-                       ctx->con_off.p, ctx->chunk_off.p, ctx->chunk_sys.p};
+                       ctx->con_off.p, ctx->chunk_off.p, ctx->chunk_sys.p, res ? ctx->plan.p : nullptr};
     return run_bbpgd_on<T>(ctx, a, mem, rep, ms_solve, per_sys);
 }
 
@@ -716,7 +782,12 @@ template <typename T>
 static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem &mem, alens_solve_report *rep,
                                  float *ms_solve, std::vector<alens_solve_report> *per_sys) {
     const int32_t ns = ctx->nsys_cur;
-    if (ctx->capture && ctx->bar_clean) {
+    constexpr int form = sizeof(T) == 8 ? 0 : 1;
+    // (in a captured step an abort of the FP32 launch must reach the step's tail past the FP64 one)
+    const bool keep_abort = ctx->capture && !ctx->bar_clean;
+    if (mem.plan) {
+        ctx->bar_clean = false;  // the resident launch clears the words it uses
+    } else if (ctx->capture && ctx->bar_clean) {
         ctx->bar_clean = false;  // the captured step zeroed them with its other counters
     } else if (ctx->capture) {
         // a later launch of the same captured step (the FP64 refinement after the FP32 solve): zero
@@ -765,13 +836,11 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
     const bool gw_band = !ctx->tuning && !getenv("ALENS_GROUP_WIDTH") && ctx->gw_rows > 0;
     a.gw_rows_lo = gw_band ? (uint32_t)(0.9 * ctx->gw_rows) : 0u;
     a.gw_rows_hi = gw_band ? (uint32_t)std::min(4294967295.0, 1.1 * ctx->gw_rows) : 0u;
-    // row streams of phase B: non-temporal when an iteration's bytes (per constraint 2 (9w + 8) + 5w,
-    // per rod 18w) overflow the GPU's last-level cache, which otherwise keeps them between iterations
+    // row streams of phase B: non-temporal when an iteration's bytes overflow the GPU's last-level cache
     // (a resident step's a.m is its row capacity; its last row count is the host's ctx->m)
     const int hint = env("ALENS_STREAM_HINT", ctx->stream_hint);
     const double rows = a.m_dev ? (double)ctx->m : (double)a.m;
-    const double iter_bytes = (double)sizeof(T) * (23.0 * rows + 18.0 * (double)a.n) + 16.0 * rows;
-    a.stream_nt = hint == 2 || (hint != 1 && iter_bytes > kLastLevelCacheBytes);
+    a.stream_nt = hint == 2 || (hint != 1 && general_iter_bytes(sizeof(T), rows, (double)a.n) > kLastLevelCacheBytes);
     const int entries = env("ALENS_SOLVER_ENTRIES", ctx->entries);
     // inside a graph the timing points are clock readings: stamp 2 before the first solver launch,
     // stamp 3 after each one (the last reading is the one read after the replay)
@@ -781,7 +850,15 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
         TRY_K(launch_stamp(ctx->st, ctx->stamps.p, 2));
         ctx->cap_solve_ev = true;
     }
-    if constexpr (sizeof(T) == 8)
+    if (mem.plan) {
+        ResidentArgs<T> ra{};
+        ra.s = a;
+        ra.ex = ctx->rex.p;
+        ra.head = mem.plan + form * kPlanHead;
+        ra.share = reinterpret_cast<const ShareCut *>(mem.plan + 2 * kPlanHead) + (size_t)form * kPlanShares;
+        ra.spos = ctx->spos_cur;
+        TRY_K(launch_resident<T>(ctx->st, ra, ctx->route.gpb[form], ctx->route.grid[form], keep_abort));
+    } else if constexpr (sizeof(T) == 8)
         TRY_K(launch_bbpgd64(ctx->st, a, max_blocks, entries, &ctx->grid_used));
     else
         TRY_K(launch_bbpgd32(ctx->st, a, max_blocks, entries, &ctx->grid_used));
@@ -888,6 +965,72 @@ static alens_status run_solver_mixed(alens_ctx *ctx, int32_t n, uint32_t m, bool
 }
 
 extern "C" {
+
+static void accept_plan(alens_ctx *ctx, const int32_t *head);
+
+// Enqueues the plan of the resident solves that ctx->route wants (k_resident_plan); mv: the row count of a
+// captured step, cleared when a plan does not fit.
+static alens_status launch_plan(alens_ctx *ctx, uint32_t *mv) {
+    TRY_HIP(ctx->plan.ensure(kPlanWords));
+    ResidentPlanArgs p{};
+    p.nsys = ctx->nsys;
+    p.sys = ctx->sysd.p;
+    p.sellStart = ctx->sellStart.p;
+    p.nslices = (uint32_t)(((int64_t)ctx->n + kSlice - 1) / kSlice);
+    p.con_off = ctx->con_off.p;
+    p.chunk_off = ctx->chunk_off.p;
+    p.nchunks = ctx->nch_dev.p;
+    for (int f = 0; f < 2; ++f) {
+        p.gpb[f] = ctx->route.gpb[f];
+        p.max_shares[f] = (uint32_t)ctx->route.grid[f];
+    }
+    p.mv = mv;
+    p.plan = ctx->plan.p;
+    TRY_K(launch_resident_plan(ctx->st, p));
+    return ALENS_OK;
+}
+
+// Plan for a stand-alone solve: one system of n rods in index order, its chunk table already on the device.
+static alens_status plan_one_system(alens_ctx *ctx, int32_t n, size_t nslices, uint64_t slots) {
+    ctx->route = alens_ctx::Route{};
+    if (schedule_named() || slots > (uint64_t)ctx->ncu * resident_slots<double>(resident_groups<double>())) return ALENS_OK;
+    ctx->route.gpb[0] = resident_gpb<double>(ctx->nchunks_cur, 1, ctx->ncu);
+    ctx->route.grid[0] = ctx->ncu;
+    if (!ctx->route.gpb[0]) return ALENS_OK;
+    SysDev one{};
+    one.rod_end = n;
+    TRY_HIP(ctx->sys_one.ensure(1));
+    TRY_HIP(ctx->plan.ensure(kPlanWords));
+    TRY_HIP(ctx->nch_dev.ensure(1));
+    TRY_HIP(hipMemcpyAsync(ctx->sys_one.p, &one, sizeof one, hipMemcpyHostToDevice, ctx->st));
+    TRY_HIP(hipMemcpyAsync(ctx->nch_dev.p, &ctx->nchunks_cur, sizeof(int32_t), hipMemcpyHostToDevice, ctx->st));
+    ResidentPlanArgs p{};
+    p.nsys = 1;
+    p.sys = ctx->sys_one.p;
+    p.sellStart = ctx->sellStart.p;
+    p.nslices = (uint32_t)nslices;
+    p.con_off = ctx->con_off.p;
+    p.chunk_off = ctx->chunk_off.p;
+    p.nchunks = ctx->nch_dev.p;
+    p.gpb[0] = ctx->route.gpb[0];
+    p.max_shares[0] = (uint32_t)ctx->ncu;
+    p.plan = ctx->plan.p;
+    TRY_K(launch_resident_plan(ctx->st, p));
+    int32_t head[2 * kPlanHead];
+    TRY_HIP(hipMemcpyAsync(head, ctx->plan.p, sizeof head, hipMemcpyDeviceToHost, ctx->st));
+    TRY_HIP(hipStreamSynchronize(ctx->st));
+    accept_plan(ctx, head);
+    return ALENS_OK;
+}
+
+// Takes a plan's heads as read back: a solve whose shares do not fit goes to the general kernel; one that fits
+// gets a block per share (or all blocks, which then take shares in turn).
+static void accept_plan(alens_ctx *ctx, const int32_t *head) {
+    for (int f = 0; f < 2; ++f) {
+        if (!head[f * kPlanHead]) ctx->route.gpb[f] = 0;
+        ctx->route.grid[f] = std::max(1, std::min(ctx->ncu, head[f * kPlanHead + 1]));
+    }
+}
 
 // One step with exact buffer sizes: the counts (cell entries, pairs, adjacency slots) are read back
 // between the phases.  Caller rows are supported here.
@@ -1067,29 +1210,38 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
         if (slot_order_on()) {
             TRY_HIP(ctx->sord.ensure((size_t)std::max(n, 1)));
             TRY_HIP(ctx->spos.ensure((size_t)std::max(n, 1)));
-            TRY_K(launch_slot_order(st, n, ctx->rowStart.p, ctx->jStart.p, xs, ctx->sord.p, ctx->spos.p,
+            TRY_K(launch_slot_order(st, n, ctx->rsys.p, ctx->rowStart.p, ctx->jStart.p, xs, ctx->sord.p, ctx->spos.p,
                                     slot_order_window(n, ctx->ncu)));
             ctx->sord_cur = ctx->sord.p;
             ctx->spos_cur = ctx->spos.p;
         }
         TRY_K(launch_slice_sizes(st, n, ctx->rowStart.p, ctx->jStart.p, xs, ctx->slen.p, ctx->sord_cur));
         TRY_K(exclusive_scan_u32(st, ctx->slen.p, ctx->sellStart.p, nsl, ctx->scan));
-        uint32_t ep = 0;
-        TRY_HIP(hipMemcpyAsync(&ep, ctx->sellStart.p + nsl, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        std::vector<uint32_t> coff((size_t)ctx->nsys + 1);
-        for (int32_t sy = 0; sy <= ctx->nsys; ++sy)
-            TRY_HIP(hipMemcpyAsync(&coff[sy], ctx->rowStart.p + ctx->rod_off[sy], sizeof(uint32_t),
-                                   hipMemcpyDeviceToHost, st));
+        // chunk table and resident plan on the device; one read-back of their sizes
+        const int32_t chcap = (int32_t)(M / kRedChunk) + ctx->nsys + 1;
+        TRY_HIP(ctx->con_off.ensure((size_t)ctx->nsys + 1));
+        TRY_HIP(ctx->chunk_off.ensure((size_t)ctx->nsys + 1));
+        TRY_HIP(ctx->chunk_sys.ensure((size_t)chcap));
+        TRY_HIP(ctx->nch_dev.ensure(1));
+        TRY_K(launch_chunk_table(st, ctx->nsys, n, ctx->sysd.p, ctx->rowStart.p, Me, ctx->con_off.p, ctx->chunk_off.p,
+                                 ctx->nch_dev.p, ctx->chunk_sys.p, chcap, nullptr));
+        ctx->route = want_route(ctx, M, 0.0);
+        alens_status ps = launch_plan(ctx, nullptr);
+        if (ps != ALENS_OK) return ps;
+        int32_t head[2 * kPlanHead];
+        TRY_HIP(hipMemcpyAsync(head, ctx->plan.p, sizeof head, hipMemcpyDeviceToHost, st));
         TRY_HIP(hipStreamSynchronize(st));
-        coff[ctx->nsys] += Me;
+        const uint32_t ep = (uint32_t)head[2];
         ctx->epad = ep;
+        ctx->slots = ep;
+        ctx->nchunks_cur = head[3];
+        ctx->nsys_cur = ctx->nsys;
+        accept_plan(ctx, head);
         TRY_HIP(ctx->sellK.ensure(std::max<size_t>(ep, 1)));
         TRY_HIP(ctx->sellW.ensure(6 * std::max<size_t>(ep, 1)));
         TRY_K(launch_adjacency(st, n, M, ctx->rowStart.p, ctx->jStart.p, ctx->jlist.p, xs, Me ? ctx->extEnt.p : nullptr,
                                Mcol, ctx->geo.p, ctx->sellStart.p, ctx->epad, ctx->adjStart.p, ctx->sellK.p,
                                ctx->sellW.p, ctx->spos_cur));
-        alens_status cs = set_chunk_table(ctx, coff);
-        if (cs != ALENS_OK) return cs;
     }
     TRY_HIP(hipEventRecord(ctx->ev[1], st));
     // solve: start point = 0 (cold), the previous step's gamma (warm_start 1) or the network's
@@ -1179,7 +1331,7 @@ static alens_status plan_resident(alens_ctx *ctx) {
     const double slack = hr ? 0.0 : 1.0;
     c.E = (uint32_t)std::min<double>(4294967295.0, (double)ctx->E * f + slack * 4096);
     c.M = (uint32_t)std::min<double>(2147483647.0, (double)ctx->m * f + slack * 4096);
-    c.epad = (uint32_t)std::min<double>(4294967295.0, (double)ctx->epad * f + slack * 4096);
+    c.epad = (uint32_t)std::min<double>(4294967295.0, (double)ctx->slots * f + slack * 4096);
     c.E = std::max<uint32_t>(c.E, 64);
     c.M = std::max<uint32_t>(c.M, 64);
     c.epad = std::max<uint32_t>(c.epad, 64);
@@ -1242,6 +1394,16 @@ static alens_status plan_resident(alens_ctx *ctx) {
         int khz = 0;
         TRY_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->dev));
         ctx->clock_khz = khz;
+    }
+    // resident solves with 4% of head room in the counts; a replay that outgrows the plan is redone plainly
+    ctx->route = want_route(ctx, 1.04 * (double)ctx->m, 1.04 * (double)ctx->slots);
+    for (int f = 0; f < 2; ++f)
+        if ((double)ctx->slots > ctx->resident_limit[f]) ctx->route.gpb[f] = 0;
+    for (int q = 0; q < 2; ++q)  // (the solve's launch decides from the same count)
+        ctx->route.stream_nt[q] = general_iter_bytes(q == 0 ? 8 : 4, (double)ctx->m, n) > kLastLevelCacheBytes;
+    TRY_HIP(ctx->plan.ensure(kPlanWords));
+    if (ctx->route.gpb[0] || ctx->route.gpb[1]) {
+        TRY_HIP(ctx->rex.ensure(resident_exchange_bytes<double>(c.M, n, c.nch)));
     }
     if (ctx->cfg.warm_start == 2) TRY_HIP(ctx->feat.ensure(16 * (size_t)c.M));
     if (ctx->cfg.precision == 1) {
@@ -1308,7 +1470,7 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
     const int64_t nsl = ((int64_t)n + kSlice - 1) / kSlice;
     ctx->sord_cur = ctx->spos_cur = nullptr;
     if (slot_order_on()) {
-        TRY_K(launch_slot_order(st, n, ctx->rowStart.p, ctx->jStart.p, nullptr, ctx->sord.p, ctx->spos.p,
+        TRY_K(launch_slot_order(st, n, ctx->rsys.p, ctx->rowStart.p, ctx->jStart.p, nullptr, ctx->sord.p, ctx->spos.p,
                                 slot_order_window(n, ctx->ncu)));
         ctx->sord_cur = ctx->sord.p;
         ctx->spos_cur = ctx->spos.p;
@@ -1320,6 +1482,11 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
                            ctx->sellStart.p, c.epad, ctx->adjStart.p, ctx->sellK.p, ctx->sellW.p, ctx->spos_cur));
     TRY_K(launch_chunk_table(st, ctx->nsys, n, ctx->sysd.p, ctx->rowStart.p, 0u, ctx->con_off.p, ctx->chunk_off.p,
                              ctx->nch_dev.p, ctx->chunk_sys.p, c.nch, Mv));
+    const bool planned = ctx->route.gpb[0] || ctx->route.gpb[1];
+    if (planned) {
+        alens_status ps = launch_plan(ctx, Mv);
+        if (ps != ALENS_OK) return ps;
+    }
     // start point and solve (the solver reads the row and chunk counts from the device)
     TRY_K(launch_stamp(st, ctx->stamps.p, 1));
     ctx->gstride = c.M;
@@ -1361,7 +1528,8 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
     // everything the host reads after a replay, in one buffer
     TRY_K(launch_step_tail(st, ctx->eoff.p + n, ctx->counter.p, ctx->sellStart.p + nsl, Mv, ctx->nch_dev.p,
                            ctx->stamps.p, ctx->bar.p + kBarWords, ctx->out.p,
-                           ctx->cfg.precision == 1 ? ctx->out32.p : nullptr, 8 * ctx->nsys, ctx->tail.p));
+                           ctx->cfg.precision == 1 ? ctx->out32.p : nullptr, 8 * ctx->nsys,
+                           planned ? ctx->plan.p + kPlanUnfit : nullptr, ctx->tail.p));
     return ALENS_OK;
 }
 
@@ -1406,10 +1574,13 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
     TRY_HIP(hipStreamSynchronize(st));
     uint32_t cnt[5];  // entries, pairs, slots, valid rows, chunks
     for (int q = 0; q < 5; ++q) cnt[q] = (uint32_t)tl[q];
-    if (cnt[0] > c.E || cnt[1] > c.M || cnt[2] > c.epad) {
+    const int unfit = (int)tl[10];
+    if (cnt[0] > c.E || cnt[1] > c.M || cnt[2] > c.epad || unfit) {
         // every overflow left zero valid rows downstream, so the replay wrote no impulse cache and
         // the plain redo starts from the same previous-step impulses
         drop_graph(ctx);
+        for (int f = 0; f < 2; ++f)
+            if (unfit & (1 << f)) ctx->resident_limit[f] = 0.9 * (double)cnt[2];
         ++ctx->graph_overflows;
         return step_plain(ctx, f_ext, rep_out);
     }
@@ -1432,6 +1603,7 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
     const double ms_collect = (double)(int64_t)(stamp[1] - stamp[0]) * tick_ms;
     const double ms_solve = (double)(int64_t)(stamp[3] - stamp[2]) * tick_ms;
     ctx->E = cnt[0];
+    ctx->slots = cnt[2];
     ctx->m = cnt[3];
     ctx->mcol = cnt[3];
     ctx->mext = 0;
@@ -1454,6 +1626,24 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
     return ALENS_OK;
 }
 
+// The captured step's kernels no longer suit the last step's counts: the solve would now fit on the chip, fewer
+// row groups per block would do, or the general kernel's row streams crossed the last-level cache's size (by
+// 5% either way).  The step is then captured again; a relaxing system does so once or twice in a run.
+static bool route_outdated(const alens_ctx *ctx) {
+    const double rows = (double)ctx->m, rods = (double)ctx->n;
+    alens_ctx::Route w = want_route(ctx, 1.04 * rows, 1.04 * (double)ctx->slots);
+    for (int f = 0; f < (ctx->cfg.precision == 1 ? 2 : 1); ++f) {
+        const int have = ctx->route.gpb[f];
+        if ((double)ctx->slots > ctx->resident_limit[f]) w.gpb[f] = 0;
+        if (w.gpb[f] > 0 && (have == 0 || w.gpb[f] < have)) return true;
+        if (have == 0 && !ctx->stream_hint) {
+            const double b = general_iter_bytes(f == 0 ? 8 : 4, rows, rods) / kLastLevelCacheBytes;
+            if (ctx->route.stream_nt[f] ? b < 0.95 : b > 1.05) return true;
+        }
+    }
+    return false;
+}
+
 alens_status alens_step_constraints(alens_ctx *ctx, const double *f_ext, alens_solve_report *rep_out) {
     if (!ctx) return ALENS_E_ARG;
     if (!ctx->have_rods) return fail(ctx, ALENS_E_STATE, "step_constraints before set_rods");
@@ -1462,6 +1652,7 @@ alens_status alens_step_constraints(alens_ctx *ctx, const double *f_ext, alens_s
     if (f_ext && !finite_all(f_ext, 6 * (size_t)ctx->n)) return fail(ctx, ALENS_E_NONFINITE, "non-finite f_ext");
     const bool fx = f_ext != nullptr;
     const bool warm_prev = ctx->cfg.warm_start >= 1 && ctx->have_prev;
+    if (ctx->gexec && route_outdated(ctx)) drop_graph(ctx);
     if (!ctx->gexec || ctx->graph_key != ((fx ? 1 : 0) | (warm_prev ? 2 : 0))) {
         // the first step sizes the buffers exactly; later ones plan capacities from the last counts
         // (the previous step's outputs are about to be replaced) and capture the resident step once
@@ -1827,6 +2018,8 @@ alens_status alens_bcqp_solve(alens_ctx *ctx, int32_t n, int64_t m, const int32_
     TRY_HIP(hipMemsetAsync(mono0.p, 0, sizeof(int32_t), st));
     alens_status cs = set_chunk_table(ctx, std::vector<uint32_t>{0u, (uint32_t)M});
     if (cs != ALENS_OK) return cs;
+    cs = plan_one_system(ctx, n, nsl, ep);
+    if (cs != ALENS_OK) return cs;
     float ms = 0.f;
     alens_status s = run_solver(ctx, n, (uint32_t)M, ctx->fext.p, x0 != nullptr, &rep, &ms, rs0.p, mono0.p, nullptr);
     rs0.release();
@@ -2016,7 +2209,7 @@ alens_status alens_bcqp_solve_static(alens_ctx *ctx, int32_t n, int64_t m, const
     ctx->cur_mdev = nullptr;
     ctx->cur_nchdev = nullptr;
     float ms = 0.f;
-    const SolveMem mem{part, out, bar, con_off, chunk_off, chunk_sys};
+    const SolveMem mem{part, out, bar, con_off, chunk_off, chunk_sys, nullptr};
     alens_status s = run_bbpgd_on<double>(ctx, a, mem, &rep, &ms, nullptr);
     ctx->nsys_cur = ns_keep;
     ctx->nchunks_cur = nch_keep;

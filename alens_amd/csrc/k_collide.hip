@@ -932,10 +932,11 @@ __device__ inline uint32_t rod_degree(const uint32_t *rowStart, const uint32_t *
     return deg;
 }
 
-// one block per window of W rods: a bitonic sort in LDS of the keys (descending degree,
-// then ascending index); rods past n sort last
+// one block per window of W rods: a bitonic sort in LDS of the keys (system, so that a system's rods keep
+// its range of positions; descending degree; ascending index); rods past n sort last
 template <int W>
-__global__ __launch_bounds__(W) void k_slot_order(int32_t n, const uint32_t *__restrict__ rowStart,
+__global__ __launch_bounds__(W) void k_slot_order(int32_t n, const int32_t *__restrict__ rsys,
+                                                  const uint32_t *__restrict__ rowStart,
                                                   const uint32_t *__restrict__ jStart,
                                                   const uint32_t *__restrict__ extStart, uint32_t *__restrict__ sord,
                                                   uint32_t *__restrict__ spos) {
@@ -943,7 +944,9 @@ __global__ __launch_bounds__(W) void k_slot_order(int32_t n, const uint32_t *__r
     const int32_t base = blockIdx.x * W;
     const int t = threadIdx.x;
     const int32_t i = base + t;
-    s_key[t] = i < n ? ((uint64_t)(0xffffffffu - rod_degree(rowStart, jStart, extStart, i)) << 32) | (uint32_t)t
+    static_assert(W <= 1 << 16 && kMaxSys <= 1 << 15, "key fields");
+    s_key[t] = i < n ? ((uint64_t)rsys[i] << 48) |
+                           ((uint64_t)(0xffffffffu - rod_degree(rowStart, jStart, extStart, i)) << 16) | (uint32_t)t
                      : ~0ull;
     __syncthreads();
     for (int k = 2; k <= W; k <<= 1) {
@@ -960,20 +963,20 @@ __global__ __launch_bounds__(W) void k_slot_order(int32_t n, const uint32_t *__r
         }
     }
     if (i < n) {
-        const uint32_t r = (uint32_t)base + (uint32_t)(s_key[t] & 0xffffffffu);
+        const uint32_t r = (uint32_t)base + (uint32_t)(s_key[t] & 0xffffu);
         sord[i] = r;         // position i holds rod r
         spos[r] = (uint32_t)i;
     }
 }
 
-HipErr launch_slot_order(hipStream_t st, int32_t n, const uint32_t *rowStart, const uint32_t *jStart,
+HipErr launch_slot_order(hipStream_t st, int32_t n, const int32_t *rsys, const uint32_t *rowStart, const uint32_t *jStart,
                          const uint32_t *extStart, uint32_t *sord, uint32_t *spos, int win) {
     if (n == 0) return hip_ok();
     if (win == kOrderWinPasses)
-        k_slot_order<kOrderWinPasses><<<nblk(n, kOrderWinPasses), kOrderWinPasses, 0, st>>>(n, rowStart, jStart,
-                                                                                         extStart, sord, spos);
+        k_slot_order<kOrderWinPasses><<<nblk(n, kOrderWinPasses), kOrderWinPasses, 0, st>>>(n, rsys, rowStart,
+                                                                                         jStart, extStart, sord, spos);
     else
-        k_slot_order<kOrderWin><<<nblk(n, kOrderWin), kOrderWin, 0, st>>>(n, rowStart, jStart, extStart, sord, spos);
+        k_slot_order<kOrderWin><<<nblk(n, kOrderWin), kOrderWin, 0, st>>>(n, rsys, rowStart, jStart, extStart, sord, spos);
     LAUNCH_CHECK();
     return hip_ok();
 }

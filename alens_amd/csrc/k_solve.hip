@@ -11,6 +11,7 @@
 // and stop together.
 #include "alens_dev.hpp"
 #include "alens_internal.hpp"
+#include "solve_dev.hpp"
 
 namespace alens {
 
@@ -25,8 +26,6 @@ static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / 
 constexpr uint32_t kSpinLimit = 1u << 26;  // barrier wait bound: sets the abort word, never hangs
 constexpr int kBlk = 1024;                  // threads per block: 4 reduction groups of 256
 constexpr int kGrp = kBlk / kRedThreads;
-
-enum : int { Q_SS = 0, Q_SY = 1, Q_YY = 2, Q_RMAX = 3, Q_NF = 4, Q_RC = 5, Q_NFC = 6 };
 
 // Grid barrier over co-resident blocks (cooperative launch).  Words (kBarWords apart, one cache
 // line each): bar[0] = arrivals, bar[kBarWords] = abort, bar[(2 + q) * kBarWords] = arrivals of
@@ -158,44 +157,6 @@ __device__ inline bool grid_barrier(uint32_t *bar, uint32_t &epoch, int *s_flag,
 // partial is already accumulated left to right; each wave folds by halving (lane l += lane l + h,
 // h = 32 .. 1); the group's four wave results are added (or compared) left to right, with one LDS
 // exchange for all of them.  Called by every thread of the block (all groups together).
-// Halving fold of one wave: lane l takes lane l + h for h = 32, 16, ..., 1 (sums: x + o; maxima:
-// o > x ? o : x) and the result is read from lane 0.  The partner values come from the gfx950 lane
-// swaps (h = 32 and 16) and DPP row shifts (h <= 8), register moves without the LDS round trip of a
-// general shuffle; lanes at or above h receive values that never reach lane 0.
-__device__ inline double lanes_up32(double x) {
-    const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
-    const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-    const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-    return __hiloint2double((int)b[1], (int)a[1]);
-}
-__device__ inline double lanes_up16(double x) {
-    const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
-    const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-    const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-    return __hiloint2double((int)b[1], (int)a[1]);
-}
-template <int H>
-__device__ inline double lanes_up_row(double x) {  // DPP row_shl:H (H < 16)
-    const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
-    return __hiloint2double((int)__builtin_amdgcn_update_dpp(0u, hi, 0x100 + H, 0xF, 0xF, true),
-                            (int)__builtin_amdgcn_update_dpp(0u, lo, 0x100 + H, 0xF, 0xF, true));
-}
-template <bool MAX>
-__device__ inline double fold_step(double x, double o) {
-    if (MAX) return o > x ? o : x;
-    return x + o;
-}
-template <bool MAX>
-__device__ inline double wave_fold(double x) {
-    x = fold_step<MAX>(x, lanes_up32(x));
-    x = fold_step<MAX>(x, lanes_up16(x));
-    x = fold_step<MAX>(x, lanes_up_row<8>(x));
-    x = fold_step<MAX>(x, lanes_up_row<4>(x));
-    x = fold_step<MAX>(x, lanes_up_row<2>(x));
-    x = fold_step<MAX>(x, lanes_up_row<1>(x));
-    return x;
-}
-
 template <int NS, int NX>
 __device__ inline void group_fold(const double (&vs)[NS], const double (&vx)[NX], double *sh /* kGrp * (NS + NX) * 4 */,
                                   double (&ts)[NS], double (&tx)[NX]) {
@@ -228,8 +189,6 @@ __device__ inline void group_fold(const double (&vs)[NS], const double (&vx)[NX]
 // group), lane c % 256 of the group accumulates the partials of the system's chunks c, c + 256, ...
 // left to right, then the group folds them (sums of slots S[], maxes of slots X[]).  Results land in
 // tot[q][s] (q < NS: sums, then the maxes) for every thread; systems not active are skipped.
-enum : int { S_ACTIVE = 0, S_CONVERGED = 1, S_NONFINITE = 2, S_NOCONV = 3 };
-
 // The same totals with one wave per system, for many small systems (replicas): lane l of the wave
 // holds the virtual lanes l, l + 64, l + 128 and l + 192 of the system's 256-lane group, accumulates
 // each one's chunks in order, folds each virtual wave by halving with shuffles and adds the four
@@ -354,19 +313,6 @@ __device__ inline void fold_systems(const double *part, int nchunks, const uint3
         }
     }
     __syncthreads();
-}
-
-enum : int { A_PROJ = 0, A_GRAD = 1 };
-
-template <typename T>
-__device__ inline typename Vec2<T>::type mk2(T x, T y);
-template <>
-__device__ inline double2 mk2<double>(double x, double y) {
-    return make_double2(x, y);
-}
-template <>
-__device__ inline float2 mk2<float>(float x, float y) {
-    return make_float2(x, y);
 }
 
 // adjacency entries a phase-A lane loads per step (their loads are in flight together): a template
@@ -604,8 +550,6 @@ __device__ inline T du_row(const SolveArgsT<T> &a, uint32_t k) {
     }
     return dt_row(gk, uI, uJ);
 }
-
-enum : int { B_INIT = 0, B_ALPHA0 = 1, B_ITER = 2 };
 
 // Phase-B reduction groups.  A 512-element chunk is reduced by GL lanes (GL = 256, or 128 when the
 // schedule asks for it); in the fixed order element e belongs to virtual lane e % 256 (pass
@@ -1319,7 +1263,8 @@ __global__ void k_step_tail(const uint32_t *__restrict__ entries, const uint32_t
                             const uint32_t *__restrict__ slots, const uint32_t *__restrict__ rows,
                             const int32_t *__restrict__ chunks, const uint64_t *__restrict__ stamps,
                             const uint32_t *__restrict__ abort_word, const double *__restrict__ out,
-                            const double *__restrict__ out32, int nrep, double *__restrict__ tail) {
+                            const double *__restrict__ out32, int nrep, const int32_t *__restrict__ plan,
+                            double *__restrict__ tail) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
         tail[0] = (double)*entries;
@@ -1329,6 +1274,7 @@ __global__ void k_step_tail(const uint32_t *__restrict__ entries, const uint32_t
         tail[4] = (double)*chunks;
         for (int q = 0; q < 4; ++q) tail[5 + q] = (double)stamps[q];
         tail[9] = (double)*abort_word;
+        tail[10] = plan ? (double)*plan : 0.0;
     }
     for (int i = t; i < nrep; i += gridDim.x * blockDim.x) {
         tail[kTailHead + i] = out[i];
@@ -1337,9 +1283,9 @@ __global__ void k_step_tail(const uint32_t *__restrict__ entries, const uint32_t
 }
 HipErr launch_step_tail(hipStream_t st, const uint32_t *entries, const uint32_t *pairs, const uint32_t *slots,
                         const uint32_t *rows, const int32_t *chunks, const uint64_t *stamps, const uint32_t *abort_word,
-                        const double *out, const double *out32, int nrep, double *tail) {
+                        const double *out, const double *out32, int nrep, const int32_t *plan, double *tail) {
     k_step_tail<<<nblk(nrep > 0 ? nrep : 1, 256), 256, 0, st>>>(entries, pairs, slots, rows, chunks, stamps, abort_word,
-                                                                out, out32, nrep, tail);
+                                                                out, out32, nrep, plan, tail);
     LAUNCH_CHECK();
     return hip_ok();
 }

@@ -383,11 +383,12 @@ constexpr int kPW1 = 0, kPB1 = 1024, kPW2 = 1088, kPB2 = 5184, kPW3 = 5248, kPB3
               kPB4 = 9472;
 constexpr int kMlpParams = 9473;
 constexpr int kMlpNorm = 2 * kMlpIn + 1;  // mean[12], 1/std[12], gamma scale
-struct MlpScratch {
-    float *XT, *Z1, *H1, *Z2, *H2, *Z3, *H3, *dO, *dZ1, *dZ2, *dZ3, *loss, *lossv;
-    float *kpart;  // K-slice partial products of the weight-gradient GEMMs (kMlpSplitFloats)
+// partial gradients (with the loss) of a batch, one per block
+constexpr int kMlpGradBlocks = 256, kMlpGradStride = 9476;
+constexpr size_t kMlpGradFloats = (size_t)kMlpGradBlocks * kMlpGradStride;
+struct AdamStep {
+    float lr, b1, b2, eps, c1, c2;  // c1, c2: 1 - b1^step, 1 - b2^step
 };
-constexpr size_t kMlpSplitFloats = 256 * 64 * 64;  // at most 256 K-slices of a 64 x 64 product
 HipErr launch_features(hipStream_t st, uint32_t m, uint32_t gs, const int32_t *cI, const int32_t *cJ, const double *delta0,
                        const double *geo, const double *posI, const double *posJ, const double *dir,
                        const double *length, const double *unc, const double2 *xprev, double dt, float *X,
@@ -396,13 +397,12 @@ HipErr launch_mlp_infer_f32(hipStream_t st, uint32_t m, const float *X, const fl
                             float *out);
 HipErr launch_mlp_infer_xg(hipStream_t st, uint32_t m, const float *X, const float *P, const float *norm,
                            double2 *xg, const uint32_t *md = nullptr);
-// part: K-slice partials (ksplit > 1), summed in order into C; NULL = one slice
-HipErr launch_gemm_bf16(hipStream_t st, int M, int N, int K, const float *A, int lda, int tA, const float *B,
-                        int ldb, int tB, float *C, int ldc, int ksplit, float *part);
-HipErr launch_gather_batch(hipStream_t st, int B, const int32_t *idx, const float *X, const float *t, float *XB,
-                           float *tB);
-HipErr mlp_gradient(hipStream_t st, int B, const float *X, const float *t, const float *P, const float *norm,
-                    MlpScratch &s, float *grad);
+// loss and gradient of B samples (a multiple of 16); part: kMlpGradFloats
+HipErr mlp_gradient(hipStream_t st, int B, const float *X, const float *t, const float *P, const float *norm, float *part,
+                    float *grad, float *loss);
+// one step of training on samples idx[0 .. B)
+HipErr mlp_train_batch(hipStream_t st, int B, const int32_t *idx, const float *X, const float *t, float *P,
+                       const float *norm, float *part, float *m1, float *m2, float lr, int step, float *loss);
 HipErr mlp_adam_step(hipStream_t st, float *P, const float *grad, float *m1, float *m2, float lr, int step);
 
 }  // namespace alens

@@ -2295,50 +2295,25 @@ alens_status alens_mlp_predict(alens_ctx *ctx, int64_t m, const float *X, float 
     return ALENS_OK;
 }
 
-namespace {
-struct TrainBufs {
-    DBuf<float> XT, Z1, H1, Z2, H2, Z3, H3, dO, dZ1, dZ2, dZ3, loss, lossv, kpart;
-    hipError_t ensure(int B) {
-        const size_t nb = (size_t)64 * B;
-        hipError_t e;
-        if ((e = XT.ensure(16 * (size_t)B)) != hipSuccess) return e;
-        for (auto *b : {&Z1, &H1, &Z2, &H2, &Z3, &H3, &dZ1, &dZ2, &dZ3})
-            if ((e = b->ensure(nb)) != hipSuccess) return e;
-        if ((e = dO.ensure((size_t)B)) != hipSuccess) return e;
-        if ((e = lossv.ensure((size_t)B)) != hipSuccess) return e;
-        if ((e = kpart.ensure(kMlpSplitFloats)) != hipSuccess) return e;
-        return loss.ensure(4);
-    }
-    MlpScratch view() {
-        return MlpScratch{XT.p, Z1.p, H1.p, Z2.p, H2.p, Z3.p, H3.p, dO.p, dZ1.p, dZ2.p, dZ3.p, loss.p, lossv.p, kpart.p};
-    }
-    void release() {
-        for (auto *b : {&XT, &Z1, &H1, &Z2, &H2, &Z3, &H3, &dO, &dZ1, &dZ2, &dZ3, &loss, &lossv, &kpart}) b->release();
-    }
-};
-}  // namespace
-
 alens_status alens_mlp_gradient(alens_ctx *ctx, int64_t m, const float *X, const float *target, float *grad,
                                 float *loss) {
     if (!ctx || m <= 0 || m % 16 || m > (1 << 26) || !X || !target || !grad) return ALENS_E_ARG;
     if (!ctx->mlp_ready) return fail(ctx, ALENS_E_STATE, "no network parameters");
     TRY_HIP(hipSetDevice(ctx->dev));
-    TrainBufs tb;
-    DBuf<float> dX, dT, dG;
-    TRY_HIP(tb.ensure((int)m));
+    DBuf<float> dX, dT, dG, part;
+    TRY_HIP(part.ensure(kMlpGradFloats));
     TRY_HIP(dX.ensure(16 * (size_t)m));
     TRY_HIP(dT.ensure((size_t)m));
-    TRY_HIP(dG.ensure(kMlpParams));
+    TRY_HIP(dG.ensure(kMlpParams + 1));  // and the loss
     TRY_HIP(hipMemcpyAsync(dX.p, X, sizeof(float) * 16 * m, hipMemcpyHostToDevice, ctx->st));
     TRY_HIP(hipMemcpyAsync(dT.p, target, sizeof(float) * m, hipMemcpyHostToDevice, ctx->st));
-    MlpScratch sv = tb.view();
-    TRY_K(mlp_gradient(ctx->st, (int)m, dX.p, dT.p, ctx->mlpP.p, ctx->mlpNorm.p, sv, dG.p));
+    TRY_K(mlp_gradient(ctx->st, (int)m, dX.p, dT.p, ctx->mlpP.p, ctx->mlpNorm.p, part.p, dG.p, dG.p + kMlpParams));
     TRY_HIP(hipMemcpyAsync(grad, dG.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->st));
     float l = 0.f;
-    TRY_HIP(hipMemcpyAsync(&l, tb.loss.p, sizeof(float), hipMemcpyDeviceToHost, ctx->st));
+    TRY_HIP(hipMemcpyAsync(&l, dG.p + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, ctx->st));
     TRY_HIP(hipStreamSynchronize(ctx->st));
     if (loss) *loss = l;
-    tb.release();
+    part.release();
     dX.release();
     dT.release();
     dG.release();
@@ -2399,16 +2374,12 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
     const float gs = norm[2 * kMlpIn];
     std::vector<float> t(m);
     for (int64_t i = 0; i < m; ++i) t[i] = gamma[i] / gs;
-    TrainBufs tb;
-    DBuf<float> dX, dT, dXB, dTB, dG, dM1, dM2, dL;
+    DBuf<float> dX, dT, part, dM1, dM2, dL;
     DBuf<int32_t> dIdx;
     const int64_t nb = m / batch;
-    TRY_HIP(tb.ensure(batch));
+    TRY_HIP(part.ensure(kMlpGradFloats));
     TRY_HIP(dX.ensure(16 * (size_t)m));
     TRY_HIP(dT.ensure((size_t)m));
-    TRY_HIP(dXB.ensure(16 * (size_t)batch));
-    TRY_HIP(dTB.ensure((size_t)batch));
-    TRY_HIP(dG.ensure(kMlpParams));
     TRY_HIP(dM1.ensure(kMlpParams));
     TRY_HIP(dM2.ensure(kMlpParams));
     TRY_HIP(dL.ensure((size_t)std::max<int64_t>(nb, 1)));
@@ -2419,7 +2390,6 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
     TRY_HIP(hipMemsetAsync(dM2.p, 0, sizeof(float) * kMlpParams, st));
     std::vector<int32_t> idx(m);
     std::vector<float> lh((size_t)std::max<int64_t>(nb, 1));
-    MlpScratch sv = tb.view();
     uint64_t rs = seed ^ 0xD1B54A32D192ED03ull;
     int step = 0;
     for (int ep = 0; ep < epochs; ++ep) {
@@ -2433,10 +2403,8 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
         }
         TRY_HIP(hipMemcpyAsync(dIdx.p, idx.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice, st));
         for (int64_t b = 0; b < nb; ++b) {
-            TRY_K(launch_gather_batch(st, batch, dIdx.p + b * batch, dX.p, dT.p, dXB.p, dTB.p));
-            TRY_K(mlp_gradient(st, batch, dXB.p, dTB.p, ctx->mlpP.p, ctx->mlpNorm.p, sv, dG.p));
-            TRY_K(mlp_adam_step(st, ctx->mlpP.p, dG.p, dM1.p, dM2.p, lr, ++step));
-            TRY_HIP(hipMemcpyAsync(dL.p + b, tb.loss.p, sizeof(float), hipMemcpyDeviceToDevice, st));
+            TRY_K(mlp_train_batch(st, batch, dIdx.p + b * batch, dX.p, dT.p, ctx->mlpP.p, ctx->mlpNorm.p, part.p, dM1.p,
+                                  dM2.p, lr, ++step, dL.p + b));
         }
         TRY_HIP(hipMemcpyAsync(lh.data(), dL.p, sizeof(float) * nb, hipMemcpyDeviceToHost, st));
         TRY_HIP(hipStreamSynchronize(st));
@@ -2444,8 +2412,7 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
         for (int64_t b = 0; b < nb; ++b) acc += lh[b];
         if (loss_per_epoch) loss_per_epoch[ep] = (float)(acc / std::max<int64_t>(nb, 1));
     }
-    tb.release();
-    for (auto *b : {&dX, &dT, &dXB, &dTB, &dG, &dM1, &dM2, &dL}) b->release();
+    for (auto *b : {&dX, &dT, &part, &dM1, &dM2, &dL}) b->release();
     dIdx.release();
     return ALENS_OK;
 }
@@ -2463,8 +2430,7 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
 // The solver's iterate buffer is overwritten; the step's outputs (gamma, velocities, rows) are not.
 namespace {
 struct EnergyBufs {
-    TrainBufs tb;
-    DBuf<float> X16, tgt, grad;
+    DBuf<float> X16, tgt, grad, part;
 };
 }  // namespace
 
@@ -2500,10 +2466,10 @@ static alens_status mlp_energy_eval(alens_ctx *ctx, double *energy, EnergyBufs *
     if (!std::isfinite(*energy)) return fail(ctx, ALENS_E_NONFINITE, "mlp energy: non-finite energy");
     if (!eb) return ALENS_OK;
     const int B = (int)((M + 15) / 16 * 16);
-    TRY_HIP(eb->tb.ensure(B));
+    TRY_HIP(eb->part.ensure(kMlpGradFloats));
     TRY_HIP(eb->X16.ensure(16 * (size_t)B));
     TRY_HIP(eb->tgt.ensure((size_t)B));
-    TRY_HIP(eb->grad.ensure(kMlpParams));
+    TRY_HIP(eb->grad.ensure(kMlpParams + 1));
     std::vector<float> t((size_t)B);
     const double half_b = 0.5 * (double)B;
     for (uint32_t k = 0; k < M; ++k) {
@@ -2515,8 +2481,8 @@ static alens_status mlp_energy_eval(alens_ctx *ctx, double *energy, EnergyBufs *
     for (int k = (int)M; k < B; ++k)
         TRY_HIP(hipMemcpyAsync(eb->X16.p + 16 * (size_t)k, ctx->feat.p, sizeof(float) * 16, hipMemcpyDeviceToDevice, st));
     TRY_HIP(hipMemcpyAsync(eb->tgt.p, t.data(), sizeof(float) * B, hipMemcpyHostToDevice, st));
-    MlpScratch sv = eb->tb.view();
-    TRY_K(mlp_gradient(st, B, eb->X16.p, eb->tgt.p, ctx->mlpP.p, ctx->mlpNorm.p, sv, eb->grad.p));
+    TRY_K(mlp_gradient(st, B, eb->X16.p, eb->tgt.p, ctx->mlpP.p, ctx->mlpNorm.p, eb->part.p, eb->grad.p,
+                       eb->grad.p + kMlpParams));
     return ALENS_OK;
 }
 

@@ -10,8 +10,11 @@
 // A[l % 16][4 (l / 16) + i], B[4 (l / 16) + i][l % 16] and D[4 (l / 16) + i][l % 16], i = 0..3.
 // Constraints run along N, so a layer's output tile (features along rows 4 (l / 16) + i, constraint
 // l % 16) is already laid out as the next layer's B operand and stays in registers from layer to layer.
-// MFMA, training GEMMs: gfx950's v_mfma_f32_16x16x32_bf16 where K is a multiple of 32 (lane l holds
-// A[l % 16][8 (l / 16) + i], B[8 (l / 16) + i][l % 16], i = 0..7, and D as above), else 16x16x16.
+// MFMA, layers of 64 inputs in training: gfx950's v_mfma_f32_16x16x32_bf16 (lane l holds A[l % 16][k] and
+// B[k][l % 16] for its eight k of 32, D as above).  Which k a lane's place holds is free as long as both operands
+// agree, so a lane's four values of two result tiles are its eight of the next operand.
+#include <algorithm>
+
 #include "alens_dev.hpp"
 #include "alens_internal.hpp"
 
@@ -29,13 +32,8 @@ typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline short f2bf(float f) {
-    // round to nearest even
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (short)(u >> 16);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (short)(u >> 16);
-}
+// round to nearest even
+__device__ inline short f2bf(float f) { return __builtin_bit_cast(short, (__bf16)f); }
 
 __device__ inline f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -43,13 +41,9 @@ __device__ inline f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
 __device__ inline f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ inline __bf16 f2bf16(float f) { return __builtin_bit_cast(__bf16, f2bf(f)); }
+__device__ inline __bf16 f2bf16(float f) { return (__bf16)f; }
 
 __device__ inline float silu(float z) { return z / (1.0f + __expf(-z)); }
-__device__ inline float silu_grad(float z) {
-    const float s = 1.0f / (1.0f + __expf(-z));
-    return s * (1.0f + z * (1.0f - s));
-}
 __device__ inline float softplus(float o) { return o > 20.0f ? o : log1pf(__expf(o)); }
 __device__ inline float sigmoidf(float o) { return 1.0f / (1.0f + __expf(-o)); }
 
@@ -214,247 +208,348 @@ HipErr launch_mlp_infer_xg(hipStream_t st, uint32_t m, const float *X, const flo
 }
 
 // ------------------------------------------------------------------------------------------------
-// training: generic BF16 MFMA GEMM  C (M x N) = op(A) (M x K) * op(B) (K x N), FP32 accumulate.
-// op(A)(m, k) = tA ? A[k * lda + m] : A[m * lda + k];  op(B)(k, n) = tB ? B[n * ldb + k] : B[k * ldb + n].
-// One wave per 16 x 16 tile of C and K-slice.  When the K range is split, slice y writes its tile to
-// part[y] and k_sum_slices adds the slices in order (the result does not depend on scheduling).
-// M, N, K are multiples of 16; K slices of a multiple of 32 use the 16x16x32 MFMA.
+// training: loss and gradient of a batch in one pass
+//
+// One wave takes 16 samples through forward and backward pass in registers; nothing of a sample goes to memory.
+// Every layer's result is wanted in two forms: samples along lanes (the next layer's operand) and units along
+// lanes (the operands of the weight gradients, which contract over samples).  The operands of an MFMA have the
+// same lane layout, so mfma(a, b) and mfma(b, a) are each other's transpose: the second form costs the same
+// products again, on matrix cores that are otherwise idle, and no transposition.  Weight gradients stay in
+// accumulators over all the wave's tiles; a block adds its four waves' in LDS and writes one partial gradient,
+// k_mlp_update adds the blocks' in order (the result does not depend on scheduling).
+//
+// A batch of 4,096 is bound by latency: loading the operands, the chain of six layers, two launches.  Layer by
+// layer through memory (35 launches, FP32 activations) it took 180 us, in this form 18 us and 4.5 us for the sum
+// over the blocks with the Adam step.
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_gemm_bf16(int M, int N, int K, const float *__restrict__ A, int lda, int tA,
-                                                  const float *__restrict__ B, int ldb, int tB, float *__restrict__ C,
-                                                  int ldc, int kslice, float *__restrict__ part) {
-    const int lane = threadIdx.x;
-    const int r16 = lane & 15, q = lane >> 4;
-    const int tilesN = N / 16;
-    const int tm = blockIdx.x / tilesN, tn = blockIdx.x % tilesN;
-    const int k0 = blockIdx.y * kslice;
-    int k1 = k0 + kslice;
-    if (k1 > K) k1 = K;
-    const int m = 16 * tm + r16, n = 16 * tn + r16;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    int k = k0;
-    for (; k + 32 <= k1; k += 32) {
-        bf16x8 a, b;
+// Sigmoid-weighted unit and its slope.  The quotients 1 / e and z / e share one reciprocal; a step of Newton each
+// (residual in one rounding) brings them to the precision of a division.  (e is capped where its reciprocal, below
+// the normal range, would be taken for 0.)
+__device__ inline void silu2(float z, float &h, float &g) {
+    const float e = fminf(1.0f + __expf(-z), 0x1p125f);
+    float s = __builtin_amdgcn_rcpf(e);
+    s = fmaf(fmaf(-e, s, 1.0f), s, s);
+    h = z * s;
+    h = fmaf(fmaf(-e, h, z), s, h);
+    g = s * (1.0f + z * (1.0f - s));
+}
+__device__ inline bf16x8 join(bf16x4 a, bf16x4 b) {
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+}
+
+constexpr int kGradWaves = 4, kGradLoss = kMlpParams;  // a partial gradient's last element: the loss
+static_assert(kMlpGradStride >= kMlpParams + 1, "a partial gradient and its loss");
+
+__global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32_t *__restrict__ idx,
+                                                              const float *__restrict__ X, const float *__restrict__ t,
+                                                              const float *__restrict__ P, const float *__restrict__ norm,
+                                                              float *__restrict__ part) {
+    // in the loop: the layers' weights in operand form, biases and output weights; then the waves' sums
+    __shared__ __align__(16) float sum[kGradWaves * kMlpGradStride];
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4, wv = threadIdx.x >> 6;
+    // operand rows: W2, W3 by output unit, then both by input unit; row 16 mt + r16, places i of pair kp: units
+    // 32 kp + 4 q + i, then those of the next tile of 16
+    bf16x8 *ops = reinterpret_cast<bf16x8 *>(sum);  // [matrix][mt][kp][lane]
+    float *vec = sum + 4 * 4 * 2 * 64 * 4;          // b1, b2, b3, w4
+#pragma unroll
+    for (int z = 0; z < 8; ++z) {
+        const int f = z * 4 + wv, mx = f >> 3, mt = (f >> 1) & 3, kp = f & 1, o = 16 * mt + r16;
+        const float *W = P + ((mx & 1) ? kPW3 : kPW2);
+        bf16x8 v;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int kk = k + 8 * q + i;
-            a[i] = f2bf16(tA ? A[(size_t)kk * lda + m] : A[(size_t)m * lda + kk]);
-            b[i] = f2bf16(tB ? B[(size_t)n * ldb + kk] : B[(size_t)kk * ldb + n]);
+            const int k = 32 * kp + 16 * (i >> 2) + 4 * q + (i & 3);
+            v[i] = f2bf16(mx < 2 ? W[o * 64 + k] : W[k * 64 + o]);
         }
-        acc = mfma32(a, b, acc);
+        ops[f * 64 + lane] = v;
     }
-    for (; k < k1; k += 16) {
-        bf16x4 a, b;
+    vec[threadIdx.x] = P[(wv == 0 ? kPB1 : wv == 1 ? kPB2 : wv == 2 ? kPB3 : kPW4) + lane];
+    bf16x4 a1[4];  // row = output unit 16 mt + r16
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a1[mt][i] = f2bf(P[kPW1 + (16 * mt + r16) * 16 + 4 * q + i]);
+    __syncthreads();
+    const float b4 = P[kPB4];
+    float mean[4], istd[4];  // of features 4 q + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        mean[i] = q < 3 ? norm[4 * q + i] : 0.0f;
+        istd[i] = q < 3 ? norm[kMlpIn + 4 * q + i] : 0.0f;
+    }
+    const float meanT = r16 < kMlpIn ? norm[r16] : 0.0f, istdT = r16 < kMlpIn ? norm[kMlpIn + r16] : 0.0f;
+
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 d1[4], d2[4][4], d3[4][4];  // weight gradients: rows 16 mt + 4 q + i, columns 16 nt + r16
+    float db1[4], db2[4], db3[4], dw4[4], db4 = 0.0f, loss = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+        d1[mt] = zero;
+        db1[mt] = db2[mt] = db3[mt] = dw4[mt] = 0.0f;
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) d2[mt][nt] = d3[mt][nt] = zero;
+    }
+    const int tiles = B / 16;
+    for (int tile = blockIdx.x * kGradWaves + wv; tile < tiles; tile += gridDim.x * kGradWaves) {
+        // (the lane index is formed anew for each tile, or the operands would be kept in registers across tiles)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        auto op = [&](int mx, int mt, int kp) { return ops[(mx * 8 + mt * 2 + kp) * 64 + ln]; };
+        auto along = [&](int v, int mt) { return *reinterpret_cast<const float4 *>(vec + v * 64 + 16 * mt + 4 * (ln >> 4)); };
+        auto vecT = [&](int v, int mt) { return vec[v * 64 + 16 * mt + (ln & 15)]; };
+        // inputs; a sample's 16 floats are one line of memory
+        const size_t s1 = (size_t)(idx ? idx[16 * tile + r16] : 16 * tile + r16);
+        const float4 x = *reinterpret_cast<const float4 *>(X + 16 * s1 + 4 * q);
+        const float tgt = t[s1];
+        bf16x4 bx, xT;
+        {
+            const float xi[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const size_t s2 = (size_t)(idx ? idx[16 * tile + 4 * q + i] : 16 * tile + 4 * q + i);
+                bx[i] = f2bf(q < 3 ? (xi[i] - mean[i]) * istd[i] : 0.0f);
+                xT[i] = f2bf(r16 < kMlpIn ? (X[16 * s2 + r16] - meanT) * istdT : 0.0f);
+            }
+        }
+        // forward: h (samples along lanes), hT (units along lanes) and the slopes the way back needs
+        bf16x4 h1[4], h1T[4], h2[4], h2T[4];
+        float g1T[4][4], g2[4][4], g2T[4][4], g3[4][4], g3T[4][4], h3T[4][4];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const f32x4 z = mfma16(a1[mt], bx, zero), zT = mfma16(bx, a1[mt], zero);
+            const float bT = vecT(0, mt);
+            const float4 b = along(0, mt);
+            const float bi[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float h, g;
+                silu2(z[i] + bi[i], h, g);
+                h1[mt][i] = f2bf(h);
+                silu2(zT[i] + bT, h, g1T[mt][i]);
+                h1T[mt][i] = f2bf(h);
+            }
+        }
+        bf16x8 o0 = join(h1[0], h1[1]), o1 = join(h1[2], h1[3]);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const bf16x8 w0 = op(0, mt, 0), w1 = op(0, mt, 1);
+            const f32x4 z = mfma32(w1, o1, mfma32(w0, o0, zero));
+            const f32x4 zT = mfma32(o1, w1, mfma32(o0, w0, zero));
+            const float bT = vecT(1, mt);
+            const float4 b = along(1, mt);
+            const float bi[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float h;
+                silu2(z[i] + bi[i], h, g2[mt][i]);
+                h2[mt][i] = f2bf(h);
+                silu2(zT[i] + bT, h, g2T[mt][i]);
+                h2T[mt][i] = f2bf(h);
+            }
+        }
+        o0 = join(h2[0], h2[1]);
+        o1 = join(h2[2], h2[3]);
+        float o = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const bf16x8 w0 = op(1, mt, 0), w1 = op(1, mt, 1);
+            const f32x4 z = mfma32(w1, o1, mfma32(w0, o0, zero));
+            const f32x4 zT = mfma32(o1, w1, mfma32(o0, w0, zero));
+            const float bT = vecT(2, mt);
+            const float4 b = along(2, mt);
+            const float bi[4] = {b.x, b.y, b.z, b.w};
+            const float4 w = along(3, mt);
+            const float wi[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float h;
+                silu2(z[i] + bi[i], h, g3[mt][i]);
+                o += wi[i] * h;
+                silu2(zT[i] + bT, h3T[mt][i], g3T[mt][i]);
+            }
+        }
+        // head: loss (y - t)^2 / B and dO = 2 (y - t) / B sigmoid(o) of sample r16
+        o += __shfl_xor(o, 16, 64);
+        o += __shfl_xor(o, 32, 64);
+        o += b4;
+        const float d = softplus(o) - tgt;
+        const float dO = 2.0f * d / (float)B * sigmoidf(o);
+        if (q == 0) {
+            loss += d * d / (float)B;
+            db4 += dO;
+        }
+        float dOT[4];  // of samples 4 q + i
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dOT[i] = __shfl(dO, 4 * q + i, 64);
+        // backward
+        bf16x4 e[4], eT[4];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const float wT = vecT(3, mt);
+            const float4 w = along(3, mt);
+            const float wi[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                e[mt][i] = f2bf(wi[i] * dO * g3[mt][i]);
+                const float dz = wT * dOT[i] * g3T[mt][i];
+                eT[mt][i] = f2bf(dz);
+                db3[mt] += dz;
+                dw4[mt] += h3T[mt][i] * dOT[i];
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) d3[mt][nt] = mfma16(eT[mt], h2T[nt], d3[mt][nt]);
+        o0 = join(e[0], e[1]);
+        o1 = join(e[2], e[3]);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const bf16x8 w0 = op(3, mt, 0), w1 = op(3, mt, 1);
+            const f32x4 z = mfma32(w1, o1, mfma32(w0, o0, zero));
+            const f32x4 zT = mfma32(o1, w1, mfma32(o0, w0, zero));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                e[mt][i] = f2bf(z[i] * g2[mt][i]);
+                const float dz = zT[i] * g2T[mt][i];
+                eT[mt][i] = f2bf(dz);
+                db2[mt] += dz;
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) d2[mt][nt] = mfma16(eT[mt], h1T[nt], d2[mt][nt]);
+        o0 = join(e[0], e[1]);
+        o1 = join(e[2], e[3]);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const f32x4 zT = mfma32(o1, op(2, mt, 1), mfma32(o0, op(2, mt, 0), zero));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dz = zT[i] * g1T[mt][i];
+                eT[mt][i] = f2bf(dz);
+                db1[mt] += dz;
+            }
+            d1[mt] = mfma16(eT[mt], xT, d1[mt]);
+        }
+    }
+    // the wave's sums into its part of LDS, the block's to memory
+    __syncthreads();
+    float *w = sum + wv * kMlpGradStride;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int kk = k + 4 * q + i;
-            a[i] = f2bf(tA ? A[(size_t)kk * lda + m] : A[(size_t)m * lda + kk]);
-            b[i] = f2bf(tB ? B[(size_t)n * ldb + kk] : B[(size_t)kk * ldb + n]);
+            const int row = 16 * mt + 4 * q + i;
+            w[kPW1 + row * 16 + r16] = d1[mt][i];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                w[kPW2 + row * 64 + 16 * nt + r16] = d2[mt][nt][i];
+                w[kPW3 + row * 64 + 16 * nt + r16] = d3[mt][nt][i];
+            }
         }
-        acc = mfma16(a, b, acc);
+        auto over_q = [](float v) {
+            v += __shfl_xor(v, 16, 64);
+            return v + __shfl_xor(v, 32, 64);
+        };
+        const float v1 = over_q(db1[mt]), v2 = over_q(db2[mt]), v3 = over_q(db3[mt]), v4 = over_q(dw4[mt]);
+        if (q == 0) {
+            const int unit = 16 * mt + r16;
+            w[kPB1 + unit] = v1;
+            w[kPB2 + unit] = v2;
+            w[kPB3 + unit] = v3;
+            w[kPW4 + unit] = v4;
+        }
     }
-    float *dst = part ? part + (size_t)blockIdx.y * M * N : C;
-    const int ld = part ? N : ldc;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[(size_t)(16 * tm + 4 * q + i) * ld + n] = acc[i];
-}
-
-// C[r][c] = part[0][r][c] + part[1][r][c] + ... (slices in order)
-__global__ void k_sum_slices(int M, int N, int ks, const float *__restrict__ part, float *__restrict__ C, int ldc) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= M * N) return;
-    float s = 0.0f;
-    for (int y = 0; y < ks; ++y) s += part[(size_t)y * M * N + idx];
-    C[(size_t)(idx / N) * ldc + idx % N] = s;
-}
-
-// K-slices of a split GEMM: a multiple of 32 at least 32 (the 16x16x32 MFMA), at most kMaxSplit slices
-constexpr int kMaxSplit = 256;
-static int gemm_kslice(int K, int ksplit) {
-    if (ksplit <= 1) return K;
-    int kslice = ((K / ksplit + 31) / 32) * 32;
-    if (kslice < 32) kslice = 32;
-    if ((K + kslice - 1) / kslice > kMaxSplit) kslice = ((K / kMaxSplit + 31) / 32 + 1) * 32;
-    return kslice;
-}
-
-HipErr launch_gemm_bf16(hipStream_t st, int M, int N, int K, const float *A, int lda, int tA, const float *B,
-                        int ldb, int tB, float *C, int ldc, int ksplit, float *part) {
-    if (M % 16 || N % 16 || K % 16) return HipErr{hipErrorInvalidValue, "gemm dims", __FILE__, __LINE__};
-    const int kslice = part ? gemm_kslice(K, ksplit) : K;
-    const int ks = (K + kslice - 1) / kslice;
-    dim3 grid((unsigned)((M / 16) * (N / 16)), (unsigned)ks);
-    k_gemm_bf16<<<grid, 64, 0, st>>>(M, N, K, A, lda, tA, B, ldb, tB, C, ldc, kslice, ks > 1 ? part : nullptr);
-    LAUNCH_CHECK();
-    if (ks > 1) {
-        k_sum_slices<<<nblk((int64_t)M * N, 256), 256, 0, st>>>(M, N, ks, part, C, ldc);
-        LAUNCH_CHECK();
+    for (int h = 32; h >= 1; h >>= 1) {
+        db4 += __shfl_xor(db4, h, 64);
+        loss += __shfl_xor(loss, h, 64);
     }
-    return hip_ok();
-}
-
-// standardised input, feature-major [16][B] (rows >= 12 zero)
-__global__ void k_mlp_input(int B, const float *__restrict__ X, const float *__restrict__ norm,
-                            float *__restrict__ XT) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= B) return;
-#pragma unroll
-    for (int f = 0; f < 16; ++f)
-        XT[(size_t)f * B + n] = f < kMlpIn ? (X[16 * (size_t)n + f] - norm[f]) * norm[kMlpIn + f] : 0.0f;
-}
-
-// Z (rows x B) += bias per row; H = SiLU(Z)
-__global__ void k_bias_silu(int rows, int B, float *__restrict__ Z, const float *__restrict__ bias,
-                            float *__restrict__ H) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)rows * B) return;
-    const int r = (int)(idx / B);
-    const float z = Z[idx] + bias[r];
-    Z[idx] = z;
-    H[idx] = silu(z);
-}
-
-// output layer: o = w4 . h3 + b4, y = softplus(o); per-sample loss (y - t)^2 / B and
-// dO = 2 (y - t) / B * sigmoid(o)
-__global__ void k_mlp_head(int B, const float *__restrict__ H3, const float *__restrict__ P,
-                           const float *__restrict__ t, float *__restrict__ dO, float *__restrict__ lossv) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= B) return;
-    float o = P[kPB4];
-    for (int r = 0; r < 64; ++r) o += P[kPW4 + r] * H3[(size_t)r * B + n];
-    const float y = softplus(o);
-    const float d = y - t[n];
-    dO[n] = 2.0f * d / (float)B * sigmoidf(o);
-    lossv[n] = d * d / (float)B;
-}
-
-// out[r] += sum_n M[r][n] * v[n] (one block per row); v = NULL sums the row
-__global__ void k_row_dot(int B, const float *__restrict__ Mx, const float *__restrict__ v, float *__restrict__ out) {
-    const int r = blockIdx.x;
-    float s = 0.0f;
-    for (int n = threadIdx.x; n < B; n += blockDim.x) s += Mx[(size_t)r * B + n] * (v ? v[n] : 1.0f);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    __shared__ float sh[4];
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    if (lane == 0) {
+        w[kPB4] = db4;
+        w[kGradLoss] = loss;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&out[r], ((sh[0] + sh[1]) + sh[2]) + sh[3]);
-}
-
-// dZ3 = (w4 dO) * SiLU'(Z3)
-__global__ void k_head_back(int B, const float *__restrict__ P, const float *__restrict__ dO,
-                            const float *__restrict__ Z, float *__restrict__ dZ) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)64 * B) return;
-    const int r = (int)(idx / B), n = (int)(idx % B);
-    dZ[idx] = P[kPW4 + r] * dO[n] * silu_grad(Z[idx]);
-}
-
-// dZ = dH * SiLU'(Z) in place on dH
-__global__ void k_silu_back(int64_t count, const float *__restrict__ Z, float *__restrict__ dH) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < count) dH[idx] = dH[idx] * silu_grad(Z[idx]);
+    float *dst = part + (size_t)blockIdx.x * kMlpGradStride;
+    for (int k = threadIdx.x; k <= kGradLoss; k += 64 * kGradWaves)
+        dst[k] = ((sum[k] + sum[kMlpGradStride + k]) + sum[2 * kMlpGradStride + k]) + sum[3 * kMlpGradStride + k];
 }
 
 // Adam (Kingma & Ba 2015); W1 columns >= 12 stay zero
-__global__ void k_adam(int np, float *__restrict__ P, const float *__restrict__ g, float *__restrict__ m1,
-                       float *__restrict__ m2, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
+__device__ inline void adam(int i, float gi, float *P, float *m1, float *m2, const AdamStep &s) {
     if (i < kPB1 && (i % 16) >= kMlpIn) {
         P[i] = 0.0f;
         return;
     }
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
+    const float a = s.b1 * m1[i] + (1.0f - s.b1) * gi;
+    const float b = s.b2 * m2[i] + (1.0f - s.b2) * gi * gi;
     m1[i] = a;
     m2[i] = b;
-    P[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+    P[i] -= s.lr * (a / s.c1) / (sqrtf(b / s.c2) + s.eps);
 }
 
-static HipErr fwd_bwd(hipStream_t st, int B, const float *X, const float *t, const float *P, const float *norm,
-                      MlpScratch &s, float *grad) {
-    const int64_t nb = (int64_t)64 * B;
-    k_mlp_input<<<nblk(B, 256), 256, 0, st>>>(B, X, norm, s.XT);
+// The gradient: blocks' partials added in a fixed order (64 elements a block, four lanes each take every fourth
+// partial); with P the Adam step that follows, else the gradient itself to grad.
+__global__ __launch_bounds__(256) void k_mlp_update(int np, const float *__restrict__ part, float *__restrict__ grad,
+                                                    float *__restrict__ loss, float *__restrict__ P,
+                                                    float *__restrict__ m1, float *__restrict__ m2, AdamStep s) {
+    __shared__ float sh[4][64];
+    const int e = threadIdx.x & 63, g = threadIdx.x >> 6, k = blockIdx.x * 64 + e;
+    float v = 0.0f;
+    if (k <= kGradLoss)
+#pragma unroll 8
+        for (int b = g; b < np; b += 4) v += part[(size_t)b * kMlpGradStride + k];
+    sh[g][e] = v;
+    __syncthreads();
+    if (g != 0 || k > kGradLoss) return;
+    v = ((sh[0][e] + sh[1][e]) + sh[2][e]) + sh[3][e];
+    if (k == kGradLoss)
+        *loss = v;
+    else if (P)
+        adam(k, v, P, m1, m2, s);
+    else
+        grad[k] = v;
+}
+
+__global__ void k_adam(float *__restrict__ P, const float *__restrict__ g, float *__restrict__ m1, float *__restrict__ m2,
+                       AdamStep s) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kMlpParams) adam(i, g[i], P, m1, m2, s);
+}
+
+static AdamStep adam_of(float lr, int step) {
+    const float b1 = 0.9f, b2 = 0.999f;
+    return AdamStep{lr, b1, b2, 1e-8f, 1.0f - powf(b1, (float)step), 1.0f - powf(b2, (float)step)};
+}
+
+// one wave per SIMD at most: a wave's operands and accumulators take most of a SIMD's registers
+static int grad_blocks(int B) { return std::max(1, std::min(kMlpGradBlocks, (B / 16 + kGradWaves - 1) / kGradWaves)); }
+
+HipErr mlp_gradient(hipStream_t st, int B, const float *X, const float *t, const float *P, const float *norm, float *part,
+                    float *grad, float *loss) {
+    const int nb = grad_blocks(B);
+    k_mlp_grad<<<nb, 64 * kGradWaves, 0, st>>>(B, nullptr, X, t, P, norm, part);
     LAUNCH_CHECK();
-    HipErr e;
-    // forward (feature-major activations: row = unit, column = sample)
-    e = launch_gemm_bf16(st, 64, B, 16, P + kPW1, 16, 0, s.XT, B, 0, s.Z1, B, 1, nullptr);
-    if (!e.ok()) return e;
-    k_bias_silu<<<nblk(nb, 256), 256, 0, st>>>(64, B, s.Z1, P + kPB1, s.H1);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, B, 64, P + kPW2, 64, 0, s.H1, B, 0, s.Z2, B, 1, nullptr);
-    if (!e.ok()) return e;
-    k_bias_silu<<<nblk(nb, 256), 256, 0, st>>>(64, B, s.Z2, P + kPB2, s.H2);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, B, 64, P + kPW3, 64, 0, s.H2, B, 0, s.Z3, B, 1, nullptr);
-    if (!e.ok()) return e;
-    k_bias_silu<<<nblk(nb, 256), 256, 0, st>>>(64, B, s.Z3, P + kPB3, s.H3);
-    LAUNCH_CHECK();
-    k_mlp_head<<<nblk(B, 256), 256, 0, st>>>(B, s.H3, P, t, s.dO, s.lossv);
-    LAUNCH_CHECK();
-    k_row_dot<<<64, 256, 0, st>>>(B, s.H3, s.dO, grad + kPW4);
-    LAUNCH_CHECK();
-    k_row_dot<<<1, 256, 0, st>>>(B, s.dO, nullptr, grad + kPB4);
-    LAUNCH_CHECK();
-    k_row_dot<<<1, 256, 0, st>>>(B, s.lossv, nullptr, s.loss);
-    LAUNCH_CHECK();
-    // backward
-    k_head_back<<<nblk(nb, 256), 256, 0, st>>>(B, P, s.dO, s.Z3, s.dZ3);
-    LAUNCH_CHECK();
-    const int ks = B / 1024 > 1 ? B / 1024 : 1;
-    e = launch_gemm_bf16(st, 64, 64, B, s.dZ3, B, 0, s.H2, B, 1, grad + kPW3, 64, ks, s.kpart);
-    if (!e.ok()) return e;
-    k_row_dot<<<64, 256, 0, st>>>(B, s.dZ3, nullptr, grad + kPB3);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, B, 64, P + kPW3, 64, 1, s.dZ3, B, 0, s.dZ2, B, 1, nullptr);
-    if (!e.ok()) return e;
-    k_silu_back<<<nblk(nb, 256), 256, 0, st>>>(nb, s.Z2, s.dZ2);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, 64, B, s.dZ2, B, 0, s.H1, B, 1, grad + kPW2, 64, ks, s.kpart);
-    if (!e.ok()) return e;
-    k_row_dot<<<64, 256, 0, st>>>(B, s.dZ2, nullptr, grad + kPB2);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, B, 64, P + kPW2, 64, 1, s.dZ2, B, 0, s.dZ1, B, 1, nullptr);
-    if (!e.ok()) return e;
-    k_silu_back<<<nblk(nb, 256), 256, 0, st>>>(nb, s.Z1, s.dZ1);
-    LAUNCH_CHECK();
-    e = launch_gemm_bf16(st, 64, 16, B, s.dZ1, B, 0, s.XT, B, 1, grad + kPW1, 16, ks, s.kpart);
-    if (!e.ok()) return e;
-    k_row_dot<<<64, 256, 0, st>>>(B, s.dZ1, nullptr, grad + kPB1);
+    k_mlp_update<<<nblk(kGradLoss + 1, 64), 256, 0, st>>>(nb, part, grad, loss, nullptr, nullptr, nullptr, AdamStep{});
     LAUNCH_CHECK();
     return hip_ok();
 }
 
-// minibatch gather: XB[b] = X[idx[b]], tB[b] = t[idx[b]] (idx < 0 -> zero row, zero weight)
-__global__ void k_gather_batch(int B, const int32_t *__restrict__ idx, const float *__restrict__ X,
-                               const float *__restrict__ t, float *__restrict__ XB, float *__restrict__ tB) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const int32_t s = idx[b];
-#pragma unroll
-    for (int f = 0; f < 16; ++f) XB[16 * (size_t)b + f] = X[16 * (size_t)s + f];
-    tB[b] = t[s];
-}
-HipErr launch_gather_batch(hipStream_t st, int B, const int32_t *idx, const float *X, const float *t, float *XB,
-                           float *tB) {
-    k_gather_batch<<<nblk(B, 256), 256, 0, st>>>(B, idx, X, t, XB, tB);
+HipErr mlp_train_batch(hipStream_t st, int B, const int32_t *idx, const float *X, const float *t, float *P,
+                       const float *norm, float *part, float *m1, float *m2, float lr, int step, float *loss) {
+    const int nb = grad_blocks(B);
+    k_mlp_grad<<<nb, 64 * kGradWaves, 0, st>>>(B, idx, X, t, P, norm, part);
+    LAUNCH_CHECK();
+    k_mlp_update<<<nblk(kGradLoss + 1, 64), 256, 0, st>>>(nb, part, nullptr, loss, P, m1, m2, adam_of(lr, step));
     LAUNCH_CHECK();
     return hip_ok();
-}
-
-HipErr mlp_gradient(hipStream_t st, int B, const float *X, const float *t, const float *P, const float *norm,
-                    MlpScratch &s, float *grad) {
-    ALENS_HIP_TRY(hipMemsetAsync(grad, 0, sizeof(float) * kMlpParams, st));
-    ALENS_HIP_TRY(hipMemsetAsync(s.loss, 0, sizeof(float), st));
-    return fwd_bwd(st, B, X, t, P, norm, s, grad);
 }
 
 HipErr mlp_adam_step(hipStream_t st, float *P, const float *grad, float *m1, float *m2, float lr, int step) {
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
-    k_adam<<<nblk(kMlpParams, 256), 256, 0, st>>>(kMlpParams, P, grad, m1, m2, lr, b1, b2, eps, c1, c2);
+    k_adam<<<nblk(kMlpParams, 256), 256, 0, st>>>(P, grad, m1, m2, adam_of(lr, step));
     LAUNCH_CHECK();
     return hip_ok();
 }

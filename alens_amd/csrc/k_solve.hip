@@ -1144,6 +1144,48 @@ __global__ void k_copy_gamma(const double2 *__restrict__ xg, double *__restrict_
     if (k < dcount(m, md)) gamma[k] = xg[k].x;
 }
 
+// gamma times the stress of a unit impulse, (lab_I - lab_J) (x) n, of rows [k0, k0 + count): nine words a row, in row
+// order, to the host's memory.  A block's words pass through LDS, so that the bus sees whole lines.
+__global__ __launch_bounds__(256) void k_row_stress(uint32_t k0, uint32_t count, uint32_t gs,
+                                                    const int32_t *__restrict__ cI, const int32_t *__restrict__ cJ,
+                                                    const uint32_t *__restrict__ img, const double *__restrict__ geo,
+                                                    const double *__restrict__ posI, const double *__restrict__ posJ,
+                                                    const double *__restrict__ center, const int32_t *__restrict__ rsys,
+                                                    const SysDev *__restrict__ sys, const double *__restrict__ gamma,
+                                                    double *__restrict__ out) {
+    __shared__ double sh[9 * 256];
+    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    if (e < count) {
+        const size_t k = (size_t)k0 + e;
+        const int32_t I = cI[k], J = cJ[k];
+        const SysDev &s = sys[rsys[I]];
+        const uint32_t im = img[k];
+        const double g = gamma[k];
+        double n[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) n[a] = geo[(size_t)a * gs + k];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const double cj = s.pbc[a] ? center[3 * (size_t)J + a] + (double)img_get(im, a) * s.len[a] : center[3 * (size_t)J + a];
+            const double d = (center[3 * (size_t)I + a] + posI[3 * k + a]) - (cj + posJ[3 * k + a]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sh[9 * threadIdx.x + 3 * a + c] = g * (d * n[c]);
+        }
+    }
+    __syncthreads();
+    const uint32_t b0 = 9 * 256 * blockIdx.x, words = 9 * count - b0 < 9 * 256 ? 9 * count - b0 : 9 * 256;
+    for (uint32_t w = threadIdx.x; w < words; w += 256) out[b0 + w] = sh[w];
+}
+
+HipErr launch_row_stress(hipStream_t st, uint32_t k0, uint32_t count, uint32_t gs, const int32_t *cI, const int32_t *cJ,
+                         const uint32_t *img, const double *geo, const double *posI, const double *posJ,
+                         const double *center, const int32_t *rsys, const SysDev *sys, const double *gamma, double *out) {
+    if (count == 0) return hip_ok();
+    k_row_stress<<<nblk(count, 256), 256, 0, st>>>(k0, count, gs, cI, cJ, img, geo, posI, posJ, center, rsys, sys, gamma, out);
+    LAUNCH_CHECK();
+    return hip_ok();
+}
+
 HipErr launch_writeback(hipStream_t st, int32_t n, const int32_t *rsys, const SysDev *sys, const uint32_t *adjStart,
                         const uint32_t *sellStart, const uint32_t *sellK, const double *sellW, uint64_t epad,
                         const double2 *xg, const double *mob, const double *unc, double *F, double *U,

@@ -222,6 +222,11 @@ HipErr launch_guard_pairs(hipStream_t st, const uint32_t *count, uint32_t cap, u
 // Chunk table on the device: con_off[s] = first row of system s (rows grouped by rod I; me caller rows
 // close the last system), chunk_off (scan of the systems' 512-row chunk counts), *nchunks, and
 // chunk_sys for the first chunk_cap chunks.
+// adjacency of rows in any order: entries (rod, row | side << 31), their starts per rod once sorted (none: as many
+// zeros), geometry from row-major vectors
+HipErr launch_row_entries(hipStream_t st, uint32_t m, const int32_t *cI, const int32_t *cJ, uint32_t *keys, uint32_t *vals);
+HipErr launch_entry_starts(hipStream_t st, int32_t n, uint32_t E, const uint32_t *keys, uint32_t *start, uint32_t *none);
+HipErr launch_row_geo(hipStream_t st, uint32_t m, const double *nrm, const double *rI, const double *rJ, double *geo);
 HipErr launch_chunk_table(hipStream_t st, int32_t nsys, int32_t n, const SysDev *sys, const uint32_t *rowStart,
                           uint32_t me, uint32_t *con_off, uint32_t *chunk_off, int32_t *nchunks, int32_t *chunk_sys,
                           int32_t chunk_cap, const uint32_t *mv);

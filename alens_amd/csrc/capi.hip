@@ -130,6 +130,7 @@ struct alens_ctx {
     };
     Route route;
     DBuf<SysDev> sys_one;                  // the one system of a stand-alone solve
+    DBuf<int32_t> zeros;                   // its rods' system
     DBuf<int32_t> plan;
     DBuf<unsigned char> rex;
     double resident_limit[2] = {1e300, 1e300};  // slots below which captures try a resident solve (lowered when it did not fit)
@@ -288,7 +289,7 @@ void alens_destroy(alens_ctx *ctx) {
     rel(ctx->cImg); rel(ctx->delta0); rel(ctx->geo); rel(ctx->posI); rel(ctx->posJ); rel(ctx->b);
     rel(ctx->adjStart); rel(ctx->sellStart); rel(ctx->sellK); rel(ctx->slen); rel(ctx->sellW); rel(ctx->xg); rel(ctx->gamma); rel(ctx->part);
     rel(ctx->out); rel(ctx->bar); rel(ctx->pkey); rel(ctx->pgam);
-    rel(ctx->sys_one); rel(ctx->plan); rel(ctx->rex);
+    rel(ctx->sys_one); rel(ctx->zeros); rel(ctx->plan); rel(ctx->rex);
     rel(ctx->out32); rel(ctx->dword); rel(ctx->nch_dev); rel(ctx->step_dev);
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
@@ -635,28 +636,6 @@ struct HostAdjacency {
     }
 };
 
-// Per-system constraint offsets -> reduction-chunk offsets and the chunk -> system table.
-static alens_status set_chunk_table(alens_ctx *ctx, const std::vector<uint32_t> &coff) {
-    const int32_t ns = (int32_t)coff.size() - 1;
-    std::vector<uint32_t> choff((size_t)ns + 1, 0);
-    for (int32_t sy = 0; sy < ns; ++sy)
-        choff[sy + 1] = choff[sy] + (coff[sy + 1] - coff[sy] + kRedChunk - 1) / kRedChunk;
-    std::vector<int32_t> csys(std::max<uint32_t>(choff[ns], 1));
-    for (int32_t sy = 0; sy < ns; ++sy)
-        for (uint32_t c = choff[sy]; c < choff[sy + 1]; ++c) csys[c] = sy;
-    TRY_HIP(ctx->con_off.ensure((size_t)ns + 1));
-    TRY_HIP(ctx->chunk_off.ensure((size_t)ns + 1));
-    TRY_HIP(ctx->chunk_sys.ensure(csys.size()));
-    TRY_HIP(hipMemcpyAsync(ctx->con_off.p, coff.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice, ctx->st));
-    TRY_HIP(hipMemcpyAsync(ctx->chunk_off.p, choff.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice,
-                           ctx->st));
-    TRY_HIP(hipMemcpyAsync(ctx->chunk_sys.p, csys.data(), sizeof(int32_t) * csys.size(), hipMemcpyHostToDevice,
-                           ctx->st));
-    TRY_HIP(hipStreamSynchronize(ctx->st));
-    ctx->nchunks_cur = (int32_t)choff[ns];
-    ctx->nsys_cur = ns;
-    return ALENS_OK;
-}
 
 // Per-system report words of a finished solve -> per-system reports and their aggregate (max
 // iterations / residuals, all converged, any fallback, worst status).
@@ -992,25 +971,29 @@ static alens_status launch_plan(alens_ctx *ctx, uint32_t *mv) {
     return ALENS_OK;
 }
 
-// Plan for a stand-alone solve: one system of n rods in index order, its chunk table already on the device.
-static alens_status plan_one_system(alens_ctx *ctx, int32_t n, size_t nslices, uint64_t slots) {
+// Chunk table and plan of a stand-alone solve (one system), made on the device; one read-back of their sizes.
+static alens_status plan_one_system(alens_ctx *ctx, int32_t n, uint32_t m) {
+    const int32_t nch = (int32_t)((m + kRedChunk - 1) / kRedChunk);
     ctx->route = alens_ctx::Route{};
-    if (schedule_named() || slots > (uint64_t)ctx->ncu * resident_slots<double>(resident_groups<double>())) return ALENS_OK;
-    ctx->route.gpb[0] = resident_gpb<double>(ctx->nchunks_cur, 1, ctx->ncu);
+    if (!schedule_named() && resident_exchange_bytes<double>(m, n, nch) < 0xffffffffull)
+        ctx->route.gpb[0] = resident_gpb<double>(nch, 1, ctx->ncu);
     ctx->route.grid[0] = ctx->ncu;
-    if (!ctx->route.gpb[0]) return ALENS_OK;
     SysDev one{};
     one.rod_end = n;
     TRY_HIP(ctx->sys_one.ensure(1));
     TRY_HIP(ctx->plan.ensure(kPlanWords));
     TRY_HIP(ctx->nch_dev.ensure(1));
+    TRY_HIP(ctx->con_off.ensure(2));
+    TRY_HIP(ctx->chunk_off.ensure(2));
+    TRY_HIP(ctx->chunk_sys.ensure((size_t)nch));
     TRY_HIP(hipMemcpyAsync(ctx->sys_one.p, &one, sizeof one, hipMemcpyHostToDevice, ctx->st));
-    TRY_HIP(hipMemcpyAsync(ctx->nch_dev.p, &ctx->nchunks_cur, sizeof(int32_t), hipMemcpyHostToDevice, ctx->st));
+    TRY_K(launch_chunk_table(ctx->st, 1, n, ctx->sys_one.p, ctx->rowStart.p, m, ctx->con_off.p, ctx->chunk_off.p,
+                             ctx->nch_dev.p, ctx->chunk_sys.p, nch, nullptr));
     ResidentPlanArgs p{};
     p.nsys = 1;
     p.sys = ctx->sys_one.p;
     p.sellStart = ctx->sellStart.p;
-    p.nslices = (uint32_t)nslices;
+    p.nslices = (uint32_t)(((int64_t)n + kSlice - 1) / kSlice);
     p.con_off = ctx->con_off.p;
     p.chunk_off = ctx->chunk_off.p;
     p.nchunks = ctx->nch_dev.p;
@@ -1021,6 +1004,9 @@ static alens_status plan_one_system(alens_ctx *ctx, int32_t n, size_t nslices, u
     int32_t head[2 * kPlanHead];
     TRY_HIP(hipMemcpyAsync(head, ctx->plan.p, sizeof head, hipMemcpyDeviceToHost, ctx->st));
     TRY_HIP(hipStreamSynchronize(ctx->st));
+    ctx->epad = (uint32_t)head[2];
+    ctx->nchunks_cur = head[3];
+    ctx->nsys_cur = 1;
     accept_plan(ctx, head);
     return ALENS_OK;
 }
@@ -1996,58 +1982,63 @@ alens_status alens_bcqp_solve(alens_ctx *ctx, int32_t n, int64_t m, const int32_
     ctx->gstride = (uint32_t)m;
     ctx->cur_mdev = nullptr;
     ctx->cur_nchdev = nullptr;
-    // rod-major adjacency in ascending constraint index, built on the host for arbitrary rows, in the
-    // sliced layout the solver reads (see launch_adjacency); geometry component-major
-    const size_t M = (size_t)m, N = (size_t)std::max(n, 1);
-    HostAdjacency h;
-    h.build(n, m, I, J, nrm, r_i, r_j);
-    const size_t nsl = h.sstart.size() - 1;
-    const uint64_t ep = h.ep;
-    std::vector<uint32_t> &start = h.start, &sstart = h.sstart, &sk = h.sk;
-    std::vector<double> &sw = h.sw, &geo = h.geo;
-    ctx->epad = ep;
-    ctx->sord_cur = ctx->spos_cur = nullptr;  // rods in index order in this layout
-    TRY_HIP(ctx->adjStart.ensure(N + 1));
-    TRY_HIP(ctx->sellStart.ensure(nsl + 1));
-    TRY_HIP(ctx->sellK.ensure(sk.size()));
-    TRY_HIP(ctx->sellW.ensure(sw.size()));
+    // rod-major adjacency in ascending constraint index, in the sliced layout the solver reads (see
+    // launch_adjacency), and component-major geometry, both made on the device: for 60,000 rows the host took 1.5 ms
+    // and sent twice the bytes
+    const size_t M = (size_t)m, N = (size_t)n;
+    const int64_t nsl = ((int64_t)n + kSlice - 1) / kSlice;
+    hipStream_t st = ctx->st;
+    for (auto *p : {&ctx->keys, &ctx->vals, &ctx->keys2, &ctx->vals2}) TRY_HIP(p->ensure(2 * M));
+    for (auto *p : {&ctx->adjStart, &ctx->extStart, &ctx->rowStart}) TRY_HIP(p->ensure(N + 1));
+    for (auto *p : {&ctx->sord, &ctx->spos}) TRY_HIP(p->ensure(N));
+    for (auto *p : {&ctx->posI, &ctx->posJ, &ctx->extNrm}) TRY_HIP(p->ensure(3 * M));
+    for (auto *p : {&ctx->b, &ctx->gamma, &ctx->delta0}) TRY_HIP(p->ensure(M));
+    for (auto *p : {&ctx->cI, &ctx->cJ}) TRY_HIP(p->ensure(M));
+    TRY_HIP(ctx->slen.ensure((size_t)nsl + 1));
+    TRY_HIP(ctx->sellStart.ensure((size_t)nsl + 1));
     TRY_HIP(ctx->geo.ensure(9 * M));
-    TRY_HIP(ctx->cI.ensure(M));
-    TRY_HIP(ctx->cJ.ensure(M));
-    TRY_HIP(ctx->b.ensure(M));
     TRY_HIP(ctx->xg.ensure(M));
-    TRY_HIP(ctx->gamma.ensure(M));
     TRY_HIP(ctx->Us.ensure(kUStride * N));
     TRY_HIP(ctx->fext.ensure(6 * N));
     TRY_HIP(ctx->bar.ensure(kBarTotalWords));
     TRY_HIP(ctx->out.ensure(16));
-    TRY_HIP(ctx->delta0.ensure(M));
-    hipStream_t st = ctx->st;
-    TRY_HIP(hipMemcpyAsync(ctx->adjStart.p, start.data(), sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, st));
-    TRY_HIP(hipMemcpyAsync(ctx->sellStart.p, sstart.data(), sizeof(uint32_t) * (nsl + 1), hipMemcpyHostToDevice, st));
-    TRY_HIP(hipMemcpyAsync(ctx->sellK.p, sk.data(), sizeof(uint32_t) * sk.size(), hipMemcpyHostToDevice, st));
-    TRY_HIP(hipMemcpyAsync(ctx->sellW.p, sw.data(), sizeof(double) * sw.size(), hipMemcpyHostToDevice, st));
-    TRY_HIP(hipMemcpyAsync(ctx->geo.p, geo.data(), sizeof(double) * 9 * M, hipMemcpyHostToDevice, st));
+    TRY_HIP(ctx->zeros.ensure(N));  // one system: every rod in system 0, no monolayer projection
     TRY_HIP(hipMemcpyAsync(ctx->cI.p, I, sizeof(int32_t) * M, hipMemcpyHostToDevice, st));
     TRY_HIP(hipMemcpyAsync(ctx->cJ.p, J, sizeof(int32_t) * M, hipMemcpyHostToDevice, st));
+    TRY_K(launch_row_entries(st, (uint32_t)M, ctx->cI.p, ctx->cJ.p, ctx->keys.p, ctx->vals.p));
+    TRY_K(launch_fill_u32(st, reinterpret_cast<uint32_t *>(ctx->zeros.p), 0u, n));
+    int bits = 1;
+    while (bits < 31 && ((n - 1) >> bits) != 0) ++bits;
+    bool alt = false;
+    TRY_K(radix_sort_pairs(st, ctx->keys.p, ctx->vals.p, ctx->keys2.p, ctx->vals2.p, 2 * (int64_t)M, bits, ctx->hist, ctx->scan,
+                           alt));
+    const uint32_t *ents = alt ? ctx->vals2.p : ctx->vals.p;
+    TRY_K(launch_entry_starts(st, n, (uint32_t)(2 * M), alt ? ctx->keys2.p : ctx->keys.p, ctx->extStart.p, ctx->rowStart.p));
+    ctx->sord_cur = ctx->spos_cur = nullptr;
+    if (slot_order_on()) {
+        TRY_K(launch_slot_order(st, n, ctx->zeros.p, ctx->rowStart.p, ctx->rowStart.p, ctx->extStart.p, ctx->sord.p,
+                                ctx->spos.p, slot_order_window(n, ctx->ncu)));
+        ctx->sord_cur = ctx->sord.p;
+        ctx->spos_cur = ctx->spos.p;
+    }
+    TRY_K(launch_slice_sizes(st, n, ctx->rowStart.p, ctx->rowStart.p, ctx->extStart.p, ctx->slen.p, ctx->sord_cur));
+    TRY_K(exclusive_scan_u32(st, ctx->slen.p, ctx->sellStart.p, nsl, ctx->scan));
+    TRY_HIP(hipMemcpyAsync(ctx->extNrm.p, nrm, sizeof(double) * 3 * M, hipMemcpyHostToDevice, st));
+    TRY_HIP(hipMemcpyAsync(ctx->posI.p, r_i, sizeof(double) * 3 * M, hipMemcpyHostToDevice, st));
+    TRY_HIP(hipMemcpyAsync(ctx->posJ.p, r_j, sizeof(double) * 3 * M, hipMemcpyHostToDevice, st));
     TRY_HIP(hipMemcpyAsync(ctx->b.p, b, sizeof(double) * M, hipMemcpyHostToDevice, st));
     TRY_HIP(hipMemcpyAsync(ctx->fext.p, mob, sizeof(double) * 6 * n, hipMemcpyHostToDevice, st));
     if (x0) TRY_HIP(hipMemcpyAsync(ctx->delta0.p, x0, sizeof(double) * M, hipMemcpyHostToDevice, st));
+    TRY_K(launch_row_geo(st, (uint32_t)M, ctx->extNrm.p, ctx->posI.p, ctx->posJ.p, ctx->geo.p));
     TRY_K(launch_init_xg(st, ctx->xg.p, x0 ? ctx->delta0.p : nullptr, (uint32_t)M));
-    // one system: every rod in system 0, no monolayer projection
-    DBuf<int32_t> rs0, mono0;
-    TRY_HIP(rs0.ensure(N));
-    TRY_HIP(mono0.ensure(1));
-    TRY_HIP(hipMemsetAsync(rs0.p, 0, sizeof(int32_t) * N, st));
-    TRY_HIP(hipMemsetAsync(mono0.p, 0, sizeof(int32_t), st));
-    alens_status cs = set_chunk_table(ctx, std::vector<uint32_t>{0u, (uint32_t)M});
+    alens_status cs = plan_one_system(ctx, n, (uint32_t)M);
     if (cs != ALENS_OK) return cs;
-    cs = plan_one_system(ctx, n, nsl, ep);
-    if (cs != ALENS_OK) return cs;
+    TRY_HIP(ctx->sellK.ensure((size_t)ctx->epad));
+    TRY_HIP(ctx->sellW.ensure(6 * (size_t)ctx->epad));
+    TRY_K(launch_adjacency(st, n, (uint32_t)M, ctx->rowStart.p, ctx->rowStart.p, nullptr, ctx->extStart.p, ents, 0u, ctx->geo.p,
+                           ctx->sellStart.p, ctx->epad, ctx->adjStart.p, ctx->sellK.p, ctx->sellW.p, ctx->spos_cur));
     float ms = 0.f;
-    alens_status s = run_solver(ctx, n, (uint32_t)M, ctx->fext.p, x0 != nullptr, &rep, &ms, rs0.p, mono0.p, nullptr);
-    rs0.release();
-    mono0.release();
+    alens_status s = run_solver(ctx, n, (uint32_t)M, ctx->fext.p, x0 != nullptr, &rep, &ms, ctx->zeros.p, ctx->zeros.p, nullptr);
     if (s != ALENS_OK) return s;
     TRY_K(launch_writeback(st, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, ctx->xg.p, nullptr, nullptr,
                            nullptr, nullptr, ctx->gamma.p, (uint32_t)M));

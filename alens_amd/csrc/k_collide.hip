@@ -995,6 +995,59 @@ __global__ void k_slice_sizes(int32_t n, const uint32_t *__restrict__ rowStart, 
     if ((threadIdx.x & 63) == 0 && p < n) slice_len[p >> 6] = deg * (uint32_t)kSlice;
 }
 
+// Rows a caller brings, in any order: an entry per row and side, (rod, row | side bit).  Sorted by rod (the sort is
+// stable, so a rod's rows ascend) they are the lists that slot order, slice sizes and k_adjacency take for caller rows.
+__global__ void k_row_entries(uint32_t m, const int32_t *__restrict__ cI, const int32_t *__restrict__ cJ,
+                              uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= m) return;
+    reinterpret_cast<uint2 *>(keys)[k] = make_uint2((uint32_t)cI[k], (uint32_t)cJ[k]);
+    reinterpret_cast<uint2 *>(vals)[k] = make_uint2(k, k | 0x80000000u);
+}
+// first sorted entry of each rod (and the end); no rows of its own grouping
+__global__ void k_entry_starts(int32_t n, uint32_t E, const uint32_t *__restrict__ keys, uint32_t *__restrict__ start,
+                               uint32_t *__restrict__ none) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i > n) return;
+    uint32_t lo = 0, hi = E;
+    while (lo < hi) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if ((int64_t)keys[mid] < i)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    start[i] = lo;
+    none[i] = 0u;
+}
+// row-major vectors to the component-major geometry
+__global__ void k_row_geo(uint32_t m, const double *__restrict__ nrm, const double *__restrict__ rI,
+                          const double *__restrict__ rJ, double *__restrict__ geo) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= m) return;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        geo[(size_t)a * m + k] = nrm[3 * (size_t)k + a];
+        geo[(size_t)(3 + a) * m + k] = rI[3 * (size_t)k + a];
+        geo[(size_t)(6 + a) * m + k] = rJ[3 * (size_t)k + a];
+    }
+}
+HipErr launch_row_entries(hipStream_t st, uint32_t m, const int32_t *cI, const int32_t *cJ, uint32_t *keys, uint32_t *vals) {
+    k_row_entries<<<nblk(m, 256), 256, 0, st>>>(m, cI, cJ, keys, vals);
+    LAUNCH_CHECK();
+    return hip_ok();
+}
+HipErr launch_entry_starts(hipStream_t st, int32_t n, uint32_t E, const uint32_t *keys, uint32_t *start, uint32_t *none) {
+    k_entry_starts<<<nblk((int64_t)n + 1, 256), 256, 0, st>>>(n, E, keys, start, none);
+    LAUNCH_CHECK();
+    return hip_ok();
+}
+HipErr launch_row_geo(hipStream_t st, uint32_t m, const double *nrm, const double *rI, const double *rJ, double *geo) {
+    k_row_geo<<<nblk(m, 256), 256, 0, st>>>(m, nrm, rI, rJ, geo);
+    LAUNCH_CHECK();
+    return hip_ok();
+}
+
 // Capacity guards between the phases of a step whose sizes are not read back: a count past its
 // capacity becomes 0 downstream (and the per-rod pair counts are cleared), so that no later kernel
 // indexes past a buffer; the host compares the raw counts with the capacities after the step.

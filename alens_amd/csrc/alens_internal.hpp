@@ -345,8 +345,8 @@ template <typename T>
 constexpr int resident_groups() {
     return sizeof(T) == 8 ? 2 : 4;
 }
-// A plan on the device: words 0..3 = {every share of the FP64 solve fits, its shares, the step's padded slots,
-// its chunks}, words 4..7 = {the FP32 solve's shares fit, its shares, wanted plans that do not fit (1: FP64, 2:
+// A plan on the device: words 0..3 = {how the FP64 solve runs, its shares, the step's padded slots,
+// its chunks}, words 4..7 = {how the FP32 solve runs, its shares, wanted plans that do not fit (1: FP64, 2:
 // FP32), chunks}, then both solves' shares.
 struct ShareCut {
     uint32_t sys, index, of;  // share `index` of the system's `of`
@@ -357,6 +357,15 @@ struct ShareCut {
 constexpr int kPlanShares = 1 << 14;
 constexpr int kPlanHead = 4, kPlanUnfit = kPlanHead + 2;
 constexpr size_t kPlanWords = 2 * kPlanHead + 2 * (size_t)kPlanShares * (sizeof(ShareCut) / 4);
+// words 0 and 4: how the solve runs
+enum { kPlanUnfitting = 0, kPlanShared = 1, kPlanAlone = 2 };
+// An FP64 solve of one system that one block holds whole (k_bbpgd_alone): at most kAloneRows rows, and LDS for the
+// slots' weights and rows, the rods' velocities and the rows' values.
+enum { kAloneNever = 0, kAloneTry = 1, kAloneOnly = 2 };
+constexpr uint32_t kAloneRows = 1024;
+__host__ __device__ inline uint64_t alone_bytes(uint64_t rows, uint64_t rods, uint64_t slots) {
+    return 50 * slots + 48 * rods + 8 * rows;
+}
 struct ResidentPlanArgs {
     int32_t nsys;
     const SysDev *sys;
@@ -365,6 +374,7 @@ struct ResidentPlanArgs {
     uint32_t *con_off, *chunk_off;
     int32_t *nchunks;
     int gpb[2];               // row groups per block of the FP64 and the FP32 solve, 0 = not wanted
+    int alone;                // one block for the FP64 solve: never, if it fits (else shares), or not at all otherwise
     uint32_t max_shares[2];   // blocks of the launch: the most shares one system may take
     uint32_t *mv;             // captured step: a plan that does not fit leaves no rows to solve
     int32_t *plan;
@@ -381,6 +391,7 @@ struct ResidentArgs {
 // bytes of exchange memory (at most 4 GiB - 1) of a solve of m rows, n rods and nchunks chunks
 template <typename T>
 size_t resident_exchange_bytes(double m, double n, double nchunks);
+HipErr launch_alone(hipStream_t st, const ResidentArgs<double> &r);
 // one launch; keep_abort: an earlier launch of the same captured step may have set the abort word
 template <typename T>
 HipErr launch_resident(hipStream_t st, const ResidentArgs<T> &r, int gpb, int grid, bool keep_abort);

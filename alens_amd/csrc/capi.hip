@@ -126,6 +126,7 @@ struct alens_ctx {
     // FP64 and the FP32 solve (0 groups: the general kernel), their device plan and exchange buffers
     struct Route {
         int gpb[2] = {0, 0}, grid[2] = {0, 0};
+        int alone = kAloneNever;  // the FP64 solve on one block
         bool stream_nt[2] = {false, false};
     };
     Route route;
@@ -733,6 +734,8 @@ static alens_ctx::Route want_route(const alens_ctx *ctx, double rows, double slo
     if (ctx->cfg.precision == 1 && (!one || slots <= 0.937 * ctx->ncu * resident_slots<float>(resident_groups<float>())))
         r.gpb[1] = resident_gpb<float>(chunks, ctx->nsys, ctx->ncu);
     for (int f = 0; f < 2; ++f) r.grid[f] = ctx->ncu;
+    if (one && rows <= kAloneRows && alone_bytes((uint64_t)rows, (uint64_t)ctx->n, (uint64_t)slots) <= kResidentPool)
+        r.alone = kAloneTry;
     return r;
 }
 
@@ -750,8 +753,9 @@ static alens_status run_bbpgd(alens_ctx *ctx, SolveArgsT<T> a, alens_solve_repor
     TRY_HIP(ctx->part.ensure((size_t)kRedQ * std::max<int32_t>(ctx->nchunks_cur, 1)));
     TRY_HIP(ctx->out.ensure(8 * (size_t)ns + 8));
     TRY_HIP(ctx->out32.ensure(8 * (size_t)ns + 8));
-    const bool res = ctx->route.gpb[sizeof(T) == 8 ? 0 : 1] > 0 && !ctx->tuning;
-    if (res) {
+    const bool alone = sizeof(T) == 8 && ctx->route.alone != kAloneNever;
+    const bool res = (alone || ctx->route.gpb[sizeof(T) == 8 ? 0 : 1] > 0) && !ctx->tuning;
+    if (res && !alone) {
         TRY_HIP(ctx->rex.ensure(resident_exchange_bytes<T>(a.m, a.n, ctx->nchunks_cur)));
     }
     const SolveMem mem{ctx->part.p, sizeof(T) == 8 ? ctx->out.p : ctx->out32.p, ctx->bar.p,
@@ -766,7 +770,8 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
     constexpr int form = sizeof(T) == 8 ? 0 : 1;
     // (in a captured step an abort of the FP32 launch must reach the step's tail past the FP64 one)
     const bool keep_abort = ctx->capture && !ctx->bar_clean;
-    if (mem.plan) {
+    const bool alone = mem.plan && form == 0 && ctx->route.alone != kAloneNever;
+    if (mem.plan && !alone) {
         ctx->bar_clean = false;  // the resident launch clears the words it uses
     } else if (ctx->capture && ctx->bar_clean) {
         ctx->bar_clean = false;  // the captured step zeroed them with its other counters
@@ -838,7 +843,14 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
         ra.head = mem.plan + form * kPlanHead;
         ra.share = reinterpret_cast<const ShareCut *>(mem.plan + 2 * kPlanHead) + (size_t)form * kPlanShares;
         ra.spos = ctx->spos_cur;
-        TRY_K(launch_resident<T>(ctx->st, ra, ctx->route.gpb[form], ctx->route.grid[form], keep_abort));
+        if constexpr (form == 0) {
+            if (alone)
+                TRY_K(launch_alone(ctx->st, ra));
+            else
+                TRY_K(launch_resident<T>(ctx->st, ra, ctx->route.gpb[form], ctx->route.grid[form], keep_abort));
+        } else {
+            TRY_K(launch_resident<T>(ctx->st, ra, ctx->route.gpb[form], ctx->route.grid[form], keep_abort));
+        }
     } else if constexpr (sizeof(T) == 8)
         TRY_K(launch_bbpgd64(ctx->st, a, max_blocks, entries, &ctx->grid_used));
     else
@@ -965,6 +977,7 @@ static alens_status launch_plan(alens_ctx *ctx, uint32_t *mv) {
         p.gpb[f] = ctx->route.gpb[f];
         p.max_shares[f] = (uint32_t)ctx->route.grid[f];
     }
+    p.alone = ctx->route.alone;
     p.mv = mv;
     p.plan = ctx->plan.p;
     TRY_K(launch_resident_plan(ctx->st, p));
@@ -977,6 +990,7 @@ static alens_status plan_one_system(alens_ctx *ctx, int32_t n, uint32_t m) {
     ctx->route = alens_ctx::Route{};
     if (!schedule_named() && resident_exchange_bytes<double>(m, n, nch) < 0xffffffffull)
         ctx->route.gpb[0] = resident_gpb<double>(nch, 1, ctx->ncu);
+    if (ctx->route.gpb[0] && m <= kAloneRows) ctx->route.alone = kAloneTry;
     ctx->route.grid[0] = ctx->ncu;
     SysDev one{};
     one.rod_end = n;
@@ -998,6 +1012,7 @@ static alens_status plan_one_system(alens_ctx *ctx, int32_t n, uint32_t m) {
     p.chunk_off = ctx->chunk_off.p;
     p.nchunks = ctx->nch_dev.p;
     p.gpb[0] = ctx->route.gpb[0];
+    p.alone = ctx->route.alone;
     p.max_shares[0] = (uint32_t)ctx->ncu;
     p.plan = ctx->plan.p;
     TRY_K(launch_resident_plan(ctx->st, p));
@@ -1015,9 +1030,10 @@ static alens_status plan_one_system(alens_ctx *ctx, int32_t n, uint32_t m) {
 // gets a block per share (or all blocks, which then take shares in turn).
 static void accept_plan(alens_ctx *ctx, const int32_t *head) {
     for (int f = 0; f < 2; ++f) {
-        if (!head[f * kPlanHead]) ctx->route.gpb[f] = 0;
+        if (head[f * kPlanHead] == kPlanUnfitting) ctx->route.gpb[f] = 0;
         ctx->route.grid[f] = std::max(1, std::min(ctx->ncu, head[f * kPlanHead + 1]));
     }
+    ctx->route.alone = head[0] == kPlanAlone ? kAloneOnly : kAloneNever;
 }
 
 // One step with exact buffer sizes: the counts (cell entries, pairs, adjacency slots) are read back
@@ -1387,6 +1403,7 @@ static alens_status plan_resident(alens_ctx *ctx) {
     ctx->route = want_route(ctx, 1.04 * (double)ctx->m, 1.04 * (double)ctx->slots);
     for (int f = 0; f < 2; ++f)
         if ((double)ctx->slots > ctx->resident_limit[f]) ctx->route.gpb[f] = 0;
+    if (ctx->route.alone != kAloneNever) ctx->route.alone = kAloneOnly;  // (the launch is fixed)
     for (int q = 0; q < 2; ++q)  // (the solve's launch decides from the same count)
         ctx->route.stream_nt[q] = general_iter_bytes(q == 0 ? 8 : 4, (double)ctx->m, n) > kLastLevelCacheBytes;
     TRY_HIP(ctx->plan.ensure(kPlanWords));
@@ -1470,7 +1487,7 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
                            ctx->sellStart.p, c.epad, ctx->adjStart.p, ctx->sellK.p, ctx->sellW.p, ctx->spos_cur));
     TRY_K(launch_chunk_table(st, ctx->nsys, n, ctx->sysd.p, ctx->rowStart.p, 0u, ctx->con_off.p, ctx->chunk_off.p,
                              ctx->nch_dev.p, ctx->chunk_sys.p, c.nch, Mv));
-    const bool planned = ctx->route.gpb[0] || ctx->route.gpb[1];
+    const bool planned = ctx->route.alone || ctx->route.gpb[0] || ctx->route.gpb[1];
     if (planned) {
         alens_status ps = launch_plan(ctx, Mv);
         if (ps != ALENS_OK) return ps;
@@ -1568,7 +1585,7 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
         // the plain redo starts from the same previous-step impulses
         drop_graph(ctx);
         for (int f = 0; f < 2; ++f)
-            if (unfit & (1 << f)) ctx->resident_limit[f] = 0.9 * (double)cnt[2];
+            if ((unfit & (1 << f)) && !(f == 0 && ctx->route.alone)) ctx->resident_limit[f] = 0.9 * (double)cnt[2];
         ++ctx->graph_overflows;
         return step_plain(ctx, f_ext, rep_out);
     }
@@ -1622,6 +1639,7 @@ static bool route_outdated(const alens_ctx *ctx) {
     alens_ctx::Route w = want_route(ctx, 1.04 * rows, 1.04 * (double)ctx->slots);
     for (int f = 0; f < (ctx->cfg.precision == 1 ? 2 : 1); ++f) {
         const int have = ctx->route.gpb[f];
+        if (f == 0 && w.alone != kAloneNever && ctx->route.alone == kAloneNever) return true;
         if ((double)ctx->slots > ctx->resident_limit[f]) w.gpb[f] = 0;
         if (w.gpb[f] > 0 && (have == 0 || w.gpb[f] < have)) return true;
         if (have == 0 && !ctx->stream_hint) {

@@ -207,10 +207,24 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
         const uint32_t scap = f == 0 ? resident_slots<double>((int)gpb) : resident_slots<float>((int)gpb);
         int32_t *head = a.plan + kPlanHead * f;
         ShareCut *share = reinterpret_cast<ShareCut *>(a.plan + 2 * kPlanHead) + (size_t)f * kPlanShares;
+        if (f == 0 && a.alone) {  // one block for the whole solve (one system)
+            const uint32_t rows = a.con_off[1] - a.con_off[0], p0 = (uint32_t)a.sys[0].rod_off, p1 = (uint32_t)a.sys[0].rod_end;
+            const uint32_t c0 = slots_before(a.sellStart, p0), slots = slots_before(a.sellStart, p1) - c0;
+            if (rows <= kAloneRows && alone_bytes(rows, p1 - p0, slots) <= kResidentPool) {
+                if (t == 0) {
+                    share[0] = ShareCut{0u, 0u, 1u, p0, p1, c0, slots, 0u};
+                    head[0] = kPlanAlone;
+                    head[1] = 1;
+                    head[2] = (int32_t)a.sellStart[a.nslices];
+                    head[3] = *a.nchunks;
+                }
+                continue;
+            }
+        }
         uint32_t nb = 0;
-        if (t == 0) s_bad = gpb == 0;
+        if (t == 0) s_bad = gpb == 0 || (f == 0 && a.alone == kAloneOnly);
         __syncthreads();
-        if (t < a.nsys && gpb > 0) {
+        if (t < a.nsys && gpb > 0 && !s_bad) {
             const uint32_t nch = a.chunk_off[t + 1] - a.chunk_off[t];
             const uint32_t slots = slots_before(a.sellStart, (uint32_t)a.sys[t].rod_end) -
                                    slots_before(a.sellStart, (uint32_t)a.sys[t].rod_off);
@@ -250,9 +264,9 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
         }
         __syncthreads();
         const bool bad = s_bad != 0;
-        if (gpb > 0 && bad) unfit |= 1 << f;
+        if ((gpb > 0 || (f == 0 && a.alone == kAloneOnly)) && bad) unfit |= 1 << f;
         if (t == 0) {
-            head[0] = bad ? 0 : 1;
+            head[0] = bad ? kPlanUnfitting : kPlanShared;
             head[1] = (int32_t)total;
             head[2] = f == 0 ? (int32_t)a.sellStart[a.nslices] : unfit;
             head[3] = *a.nchunks;
@@ -386,6 +400,20 @@ __device__ inline double wave_fold4(const double (&v)[4], bool sum2) {
 // where lane 16 r of wave_fold4 holds its result: quantity 0, 2, 1, 3
 __device__ inline int fold4_quantity(int r) { return r == 1 ? 2 : (r == 2 ? 1 : r); }
 
+// A system's report words.
+template <typename T>
+__device__ inline void report(const SolveArgsT<T> &a, int sy, int iters, int mv, int state, int fb, double res0, double res) {
+    double *o = a.out + 8 * (size_t)sy;
+    o[0] = (double)iters;
+    o[1] = (double)mv;
+    o[2] = state == S_CONVERGED ? 1.0 : 0.0;
+    o[3] = (double)fb;
+    o[4] = state == S_CONVERGED ? 0.0 : (state == S_NONFINITE ? (double)ALENS_E_NONFINITE : (double)ALENS_E_NOCONV);
+    o[5] = res0;
+    o[6] = res;
+    o[7] = (double)(a.con_off[sy + 1] - a.con_off[sy]);  // the system's rows
+}
+
 // EXT: the rows include caller rows (lower bounds and compliances other than 0).
 template <typename T, int GPB, bool EXT>
 __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r) {
@@ -407,7 +435,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
     __shared__ uint32_t s_cnt[NT / 64];
     __shared__ int s_abort;
     __shared__ uint32_t s_ticket;
-    if (r.head[0] == 0) return;  // a share does not fit: the host redoes the step
+    if (r.head[0] != kPlanShared) return;  // a share does not fit: the host redoes the step
     const int tid = threadIdx.x, grp = tid >> 8, gl = tid & 255, lane = tid & 63, wv = (tid >> 6) & 3;
     const uint32_t total = (uint32_t)r.head[1];
     const Regions rg = regions<T>(a.m, a.n, a.nchunks);
@@ -955,19 +983,261 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
             if (ok[q]) a.xg[kk[q]] = mk2<T>(xo[q], go[q]);
-        if (ib == 0 && tid == 0) {
-            double *o = a.out + 8 * (size_t)sy;
-            o[0] = (double)iters;
-            o[1] = (double)mv;
-            o[2] = state == S_CONVERGED ? 1.0 : 0.0;
-            o[3] = (double)fb;
-            o[4] = state == S_CONVERGED ? 0.0 : (state == S_NONFINITE ? (double)ALENS_E_NONFINITE : (double)ALENS_E_NOCONV);
-            o[5] = res0;
-            o[6] = res;
-            o[7] = (double)(a.con_off[sy + 1] - a.con_off[sy]);  // the system's rows
-        }
+        if (ib == 0 && tid == 0) report(a, sy, iters, mv, state, fb, res0, res);
         __syncthreads();
     }
+}
+
+// ------------------------------------------------------------------------------------------------
+// A solve that one block holds whole: nothing is exchanged but through LDS.  Groups of 256 lanes hold a chunk each,
+// two rows a lane; slot weights, the rows' values and the rods' velocities are in LDS.  An iteration is bound by LDS
+// reads (six weights and a value per slot, two velocities per row) and three block synchronisations.  Sums and their
+// order are the general kernel's.  Per iteration 2.1 us for 399 rows and 3.4 us for 793, against 7.6 and 9.2 us of the
+// shared form, whose one or two blocks spend three round trips past the L2: it is the faster one wherever it fits.
+// ------------------------------------------------------------------------------------------------
+template <bool EXT>
+__global__ __launch_bounds__(512) void k_bbpgd_alone(ResidentArgs<double> r) {
+    constexpr int NT = 512;
+    static_assert(kAloneRows == 2 * kRedChunk && kRedChunk == 2 * kRedThreads && kRedThreads == 256, "two groups, two rows a lane");
+    const SolveArgsT<double> &a = r.s;
+    __shared__ __align__(16) unsigned char pool[kResidentPool];
+    __shared__ double shG[2][2][4 * 4];
+    if (r.head[0] != kPlanAlone) return;  // does not fit: the host redoes the step
+    const int tid = threadIdx.x, grp = tid >> 8, gl = tid & 255, lane = tid & 63, wv = (tid >> 6) & 3;
+    const ShareCut cut = r.share[0];
+    const uint32_t p0 = cut.p0, p1 = cut.p1, S = cut.slots;
+    const uint32_t kb = a.con_off[0], R = a.con_off[1] - kb, nch = a.chunk_off[1] - a.chunk_off[0];
+    const int mono = a.smono[0];
+    const uint32_t oU = 48u * S, oV = oU + 48u * (p1 - p0), oE = oV + 8u * R;  // weights; velocities; values; slots' rows
+    // rows
+    uint32_t kk[2], pI[2], pJ[2];
+    bool ok[2];
+    double gk[2][9], bb[2], xo[2], go[2], lbk[2], ivk[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        kk[q] = (uint32_t)(grp * kRedChunk + gl + q * kRedThreads);
+        ok[q] = kk[q] < R;
+        lbk[q] = ivk[q] = 0.0;
+        const uint32_t k = kb + kk[q];
+        if (ok[q]) {
+#pragma unroll
+            for (int c = 0; c < 9; ++c) gk[q][c] = a.geo[(size_t)c * a.m + k];
+            const uint32_t I = (uint32_t)a.cI[k], J = (uint32_t)a.cJ[k];
+            pI[q] = oU + 48u * ((r.spos ? r.spos[I] : I) - p0);
+            pJ[q] = oU + 48u * ((r.spos ? r.spos[J] : J) - p0);
+            bb[q] = a.b[k];
+            if (EXT) {
+                lbk[q] = a.lb[k];
+                ivk[q] = a.invk[k];
+            }
+            const double2 xg = a.xg[k];
+            xo[q] = xg.x;
+            go[q] = xg.y;
+        }
+    }
+    // slots by component in slice order, a cut last slice packed; a rod: degree, first slot, distance of its slots
+    struct Rod {
+        uint32_t deg, at, step;
+    };
+    auto rod_index = [&](uint32_t p) { return a.sord ? (int)a.sord[p] : (int)p; };
+    auto rod_at = [&](uint32_t p) {
+        const int rod = rod_index(p);
+        const uint32_t c0 = p & ~(uint32_t)(kSlice - 1);
+        const uint32_t from = c0 > p0 ? c0 : p0, to = c0 + kSlice < p1 ? c0 + kSlice : p1;
+        return Rod{a.adjStart[rod + 1] - a.adjStart[rod], slots_before(a.sellStart, from) - cut.s0 + (p - from), to - from};
+    };
+    double *sW = reinterpret_cast<double *>(pool), *sV = reinterpret_cast<double *>(pool + oV);
+    uint16_t *sE = reinterpret_cast<uint16_t *>(pool + oE);
+    for (uint32_t p = p0 + tid; p < p1; p += NT) {
+        const Rod q = rod_at(p);
+        const size_t g0 = (size_t)a.sellStart[p / kSlice] + p % kSlice;
+        for (uint32_t j = 0; j < q.deg; j += 4) {
+            uint32_t K[4];
+            double w[4][6];
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+                const size_t ge = g0 + (size_t)(j + z < q.deg ? j + z : j) * kSlice;
+                K[z] = a.sellK[ge] & 0x7fffffffu;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) w[z][c] = a.sellW[c * a.epad + ge];
+            }
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+                if (j + z >= q.deg) break;
+                const uint32_t at = q.at + (j + z) * q.step;
+                sE[at] = (uint16_t)(K[z] - kb);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) sW[c * S + at] = w[z][c];
+            }
+        }
+    }
+    constexpr int NR = 2;  // a lane's first rods stay in registers, with their mobility
+    Rod rods[NR];
+    double rmob[NR][6];
+#pragma unroll
+    for (int z = 0; z < NR; ++z) {
+        const uint32_t p = p0 + tid + z * NT;
+        rods[z] = p < p1 ? rod_at(p) : Rod{0u, 0u, 0u};
+#pragma unroll
+        for (int c = 0; c < 6; ++c) rmob[z][c] = rods[z].deg ? a.mob[6 * (size_t)rod_index(p) + c] : 0.0;
+    }
+    const double dt = a.dt;
+    double alpha = 0.0;
+    auto walk = [&](const Rod &q, uint32_t p, const double (&mb)[6]) {
+        if (q.deg == 0) return;  // no row reads it
+        double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, u[6];
+        uint32_t at = q.at;
+        for (uint32_t j = 0; j < q.deg; ++j, at += q.step) {
+            const double v = sV[sE[at]];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) f[c] = f[c] + v * sW[c * S + at];
+        }
+        apply_M(mb, f, mono, u);
+        double2 *d = reinterpret_cast<double2 *>(pool + oU + 48u * (p - p0));
+#pragma unroll
+        for (int c = 0; c < 3; ++c) d[c] = make_double2(u[2 * c], u[2 * c + 1]);
+    };
+    int state = S_ACTIVE, iters = 0, mv = 0, fb = 0;
+    double res0 = 0.0, res = 0.0;
+    for (int it = -1; it <= a.max_ite; ++it) {
+        const bool odd = it & 1;
+        // v = P(x - alpha g) of every row (g itself for the first step); then one lane per rod: U = M F
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (ok[q]) sV[kk[q]] = it == 0 ? go[q] : proj(xo[q] - alpha * go[q], lbk[q]);
+        lds_sync();
+#pragma unroll
+        for (int z = 0; z < NR; ++z) walk(rods[z], p0 + tid + z * NT, rmob[z]);
+        for (uint32_t p = p0 + tid + NR * NT; p < p1; p += NT) {
+            double mb[6];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) mb[c] = a.mob[6 * (size_t)rod_index(p) + c];
+            walk(rod_at(p), p, mb);
+        }
+        lds_sync();
+        // rows: new (x, g), residual and products
+        double vs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, vx[2] = {0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (!ok[q]) continue;
+            double uI[6], uJ[6];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double2 wi = reinterpret_cast<const double2 *>(pool + pI[q])[c];
+                const double2 wj = reinterpret_cast<const double2 *>(pool + pJ[q])[c];
+                uI[2 * c] = wi.x;
+                uI[2 * c + 1] = wi.y;
+                uJ[2 * c] = wj.x;
+                uJ[2 * c + 1] = wj.y;
+            }
+            const double du = dt_row(gk[q], uI, uJ);
+            if (it == 0) {
+                double ag = dt * du;
+                if (EXT) ag = ag + ivk[q] * go[q];
+                vs[0] = vs[0] + go[q] * go[q];
+                vs[1] = vs[1] + go[q] * ag;
+                continue;
+            }
+            const double xn = proj(xo[q] - alpha * go[q], lbk[q]);
+            double gn = dt * du + bb[q];
+            if (EXT) gn = gn + ivk[q] * xn;
+            const double e = fabs(xn - proj(xn - gn, lbk[q]));
+            if (!isfinite(e))
+                vs[3] = vs[3] + 1.0;
+            else if (e > vx[0])
+                vx[0] = e;
+            if (it < 0) {
+                if (a.warm) {
+                    const double rc = fabs(0.0 - proj(0.0 - bb[q], lbk[q]));
+                    if (!isfinite(rc))
+                        vs[4] = vs[4] + 1.0;
+                    else if (rc > vx[1])
+                        vx[1] = rc;
+                }
+            } else {
+                const double sv = xn - xo[q], yv = gn - go[q];
+                vs[0] = vs[0] + sv * sv;
+                vs[1] = vs[1] + sv * yv;
+                vs[2] = vs[2] + yv * yv;
+            }
+            xo[q] = xn;
+            go[q] = gn;
+        }
+        // chunk partials as in k_bbpgd_resident, then the chunks' totals: sums first
+        const bool sum2 = it >= 0;
+        double v[4];
+        v[0] = it < 0 ? vs[3] : (it == 0 || odd ? vs[0] : vs[1]);
+        v[1] = it < 0 ? vs[4] : (it == 0 || odd ? vs[1] : vs[2]);
+        v[2] = it < 0 ? vx[0] : vs[3];
+        v[3] = it < 0 ? vx[1] : vx[0];
+        const double x = wave_fold4(v, sum2);
+        double *sg = shG[it & 1][grp];  // two in turn: one is read while the next is written
+        if ((lane & 15) == 0) sg[fold4_quantity(lane >> 4) * 4 + wv] = x;
+        lds_sync();
+        double tot[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool sum = q < 2 || (q == 2 && sum2);
+            double c[2] = {0.0, 0.0};
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h)
+                if (h < nch) {
+                    const double p = total4(shG[it & 1][h] + 4 * q, sum);
+                    c[h] = sum ? c[h] + p : (p > c[h] ? p : c[h]);
+                }
+            tot[q] = sum ? c[0] + c[1] : (c[1] > c[0] ? c[1] : c[0]);
+        }
+        ++mv;
+        if (it == 0) {
+            alpha = tot[0] / tot[1];
+            if (!(alpha > 0.0 && alpha < INFINITY)) alpha = 1.0;
+            continue;
+        }
+        double nf = tot[2], rm = tot[3];
+        if (it < 0) {
+            nf = tot[0];
+            rm = tot[2];
+            if (a.warm && (nf > 0.0 || rm > tot[3])) {  // the warm start raised the residual: x = 0, g = 0 + b
+                fb = 1;
+                nf = tot[1];
+                rm = tot[3];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    xo[q] = 0.0;
+                    go[q] = 0.0 + bb[q];
+                }
+            }
+            res0 = rm;
+        } else {
+            iters = it;
+        }
+        res = rm;
+        if (nf > 0.0) {
+            state = S_NONFINITE;
+            break;
+        }
+        if (rm <= a.tol) {
+            state = S_CONVERGED;
+            break;
+        }
+        if (it > 0) {
+            const double an = tot[0] / tot[1];  // s.s / s.y (odd) or s.y / y.y (even)
+            if (an > 0.0 && an < INFINITY) alpha = an;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (ok[q]) a.xg[kb + kk[q]] = make_double2(xo[q], go[q]);
+    if (tid == 0) report(a, 0, iters, mv, state, fb, res0, res);
+}
+
+HipErr launch_alone(hipStream_t st, const ResidentArgs<double> &r) {
+    if (r.s.lb)
+        k_bbpgd_alone<true><<<1, 512, 0, st>>>(r);
+    else
+        k_bbpgd_alone<false><<<1, 512, 0, st>>>(r);
+    LAUNCH_CHECK();
+    return hip_ok();
 }
 
 template <typename T, int GPB>

@@ -60,12 +60,12 @@ def comb():
     return rods, cfg
 
 
-@pytest.mark.parametrize("case", [("rows", m) for m in (1, 512, 513, 131072, 131073, 262144, 262145, 3000)] +
-                         [(kind, p) for kind in ("slab", "batch", "rows_of_the_caller") for p in (0, 1)] + [("comb", 0)],
+@pytest.mark.parametrize("case", [("rows", m) for m in (1, 512, 513, 1024, 1025, 131072, 131073, 262144, 262145, 3000)] +
+                         [(kind, p) for kind in ("slab", "batch", "small", "sparse", "rows_of_the_caller") for p in (0, 1)] + [("comb", 0)],
                          ids=lambda c: f"{c[0]}-{c[1]}")
 def test_resident_matches_general(monkeypatch, case):
     kind, v = case
-    if kind == "rows":  # the edges of a chunk, and of one and two row groups on each of 256 blocks
+    if kind == "rows":  # the edges of a chunk, of one block, and of one and two row groups on each of 256 blocks
         prob = rows_problem(v)
         x0 = np.random.default_rng(1).uniform(0.0, 0.1, v)
 
@@ -82,6 +82,8 @@ def test_resident_matches_general(monkeypatch, case):
         parts, cfg = systems.replicas(nsys=40, nmin=2000, nmax=14000, seed=31)
     elif kind == "comb":
         rods, cfg = comb()
+    elif kind in ("small", "sparse"):  # one block holds the solve; it holds the rows, but not so many rods
+        rods, cfg = systems.small_3d(n=800 if kind == "small" else 4000, box=3.8 if kind == "small" else 10.0, seed=35)
     elif kind == "slab":  # rods in random order: a block's rows touch more rods than its LDS keeps
         rods, cfg = systems.scaled("monolayer_slab", 60000, seed=32)
     else:

@@ -181,9 +181,22 @@ HipErr launch_order_J(hipStream_t st, int32_t n, uint32_t m, const int32_t *cJ,
 HipErr launch_rows(hipStream_t st, const RodsDev &r, const CfgDev &c, uint32_t m, uint32_t gs, const int32_t *cI,
                    const int32_t *cJ, const uint32_t *cImg, const double *unc, double *delta0,
                    double *geo, double *posI, double *posJ, double *b, const uint32_t *md = nullptr);
-HipErr launch_rows_ext(hipStream_t st, uint32_t me, uint32_t k0, uint32_t gs, const int32_t *cI, const int32_t *cJ,
-                       const double *nrm, const double *posI, const double *posJ, const double *delta0,
-                       const double *unc, double dt, double *geo, double *b);
+// Caller rows of a step, packed into one buffer of 13 m words, then 4 m + n + 1 half words: fields, rods, and the
+// rods' entries (row | side << 31) with their starts
+struct ExtRows {
+    const double *nrm, *posI, *posJ, *delta0, *x0, *lb, *invk;
+    const int32_t *I, *J;
+    const uint32_t *start, *ent;
+};
+inline ExtRows ext_rows(const double *p, size_t m, size_t n) {
+    if (m == 0) return ExtRows{};
+    const int32_t *i = reinterpret_cast<const int32_t *>(p + 13 * m);
+    const uint32_t *u = reinterpret_cast<const uint32_t *>(i + 2 * m);
+    return ExtRows{p, p + 3 * m, p + 6 * m, p + 9 * m, p + 10 * m, p + 11 * m, p + 12 * m, i, i + m, u, u + n + 1};
+}
+HipErr launch_rows_ext(hipStream_t st, uint32_t me, uint32_t k0, uint32_t gs, const ExtRows &x, const double *unc, double dt,
+                       int32_t *cI, int32_t *cJ, uint32_t *cImg, double *delta0, double *posI, double *posJ, double *geo,
+                       double *b, double *lb, double *invk, double2 *xg);
 
 // Rod-major adjacency (column blocks of D) in sliced, wave-interleaved form: rods are taken in
 // slices of kSlice consecutive indices; entry j of rod i (ascending constraint index, J-side entries
@@ -305,7 +318,6 @@ HipErr launch_writeback(hipStream_t st, int32_t n, const int32_t *rsys, const Sy
 HipErr launch_euler(hipStream_t st, int32_t n, const int32_t *rsys, const SysDev *sys, double *center, double *dir,
                     const double *u, const CfgDev &c);
 HipErr launch_init_xg(hipStream_t st, double2 *xg, const double *x0, uint32_t m);
-HipErr launch_set_x(hipStream_t st, double2 *xg, const double *x0, uint32_t me);
 HipErr launch_stamp(hipStream_t st, uint64_t *t, int idx);
 HipErr launch_warm_match(hipStream_t st, uint32_t m, const int32_t *cI, const int32_t *cJ,
                          const int32_t *gid, uint32_t mprev, const uint64_t *prev_key,

@@ -72,8 +72,8 @@ struct alens_ctx {
     DBuf<double> gamma, part, out;
     // caller rows (the constraint pool): pending for the next step, and those of the last step
     std::vector<alens_con_block> ext_pending, ext_step;
-    DBuf<uint32_t> extStart, extEnt;
-    DBuf<double> extNrm, extX0, lb, invk;
+    DBuf<uint32_t> extStart;
+    DBuf<double> ext, extNrm, lb, invk;
     DBuf<float> lb32, invk32;
     uint32_t mcol = 0, mext = 0;  // collision rows, caller rows of the last step
     // precision form: FP32 copies of the operator data and the FP32 iterate
@@ -294,7 +294,7 @@ void alens_destroy(alens_ctx *ctx) {
     rel(ctx->out32); rel(ctx->dword); rel(ctx->nch_dev); rel(ctx->step_dev);
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-    rel(ctx->extStart); rel(ctx->extEnt); rel(ctx->extNrm); rel(ctx->extX0); rel(ctx->lb); rel(ctx->invk);
+    rel(ctx->extStart); rel(ctx->ext); rel(ctx->extNrm); rel(ctx->lb); rel(ctx->invk);
     rel(ctx->lb32); rel(ctx->invk32); rel(ctx->geo32); rel(ctx->sellW32); rel(ctx->mob32); rel(ctx->b32); rel(ctx->U32); rel(ctx->xg32);
     rel(ctx->mlpP); rel(ctx->mlpNorm); rel(ctx->feat); rel(ctx->xprev);
     rel(ctx->sysd); rel(ctx->rsys); rel(ctx->smono); rel(ctx->chunk_sys); rel(ctx->con_off); rel(ctx->chunk_off);
@@ -676,7 +676,7 @@ static alens_status read_reports(alens_ctx *ctx, const double *out_dev, const ui
     std::vector<double> o(8 * (size_t)ctx->nsys_cur);
     uint32_t abort_word = 0;
     TRY_HIP(hipMemcpyAsync(o.data(), out_dev, sizeof(double) * o.size(), hipMemcpyDeviceToHost, ctx->st));
-    TRY_HIP(hipMemcpyAsync(&abort_word, bar + kBarWords, sizeof abort_word, hipMemcpyDeviceToHost, ctx->st));
+    if (bar) TRY_HIP(hipMemcpyAsync(&abort_word, bar + kBarWords, sizeof abort_word, hipMemcpyDeviceToHost, ctx->st));
     TRY_HIP(hipStreamSynchronize(ctx->st));
     return parse_reports(ctx, o.data(), abort_word, rep, per_sys);
 }
@@ -771,7 +771,9 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
     // (in a captured step an abort of the FP32 launch must reach the step's tail past the FP64 one)
     const bool keep_abort = ctx->capture && !ctx->bar_clean;
     const bool alone = mem.plan && form == 0 && ctx->route.alone != kAloneNever;
-    if (mem.plan && !alone) {
+    if (alone) {
+        // (no block waits for another: the words are neither used nor read)
+    } else if (mem.plan) {
         ctx->bar_clean = false;  // the resident launch clears the words it uses
     } else if (ctx->capture && ctx->bar_clean) {
         ctx->bar_clean = false;  // the captured step zeroed them with its other counters
@@ -861,7 +863,7 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
         return ALENS_OK;
     }
     TRY_HIP(hipEventRecord(ctx->ev[3], ctx->st));
-    alens_status s = read_reports(ctx, out, mem.bar, rep, per_sys);
+    alens_status s = read_reports(ctx, out, alone ? nullptr : mem.bar, rep, per_sys);
     if (s != ALENS_OK) return s;
     TRY_HIP(hipEventElapsedTime(ms_solve, ctx->ev[2], ctx->ev[3]));
     return ALENS_OK;
@@ -961,6 +963,21 @@ extern "C" {
 
 static void accept_plan(alens_ctx *ctx, const int32_t *head);
 
+// Every counter and cursor of a step, and the solver's barrier words, in one launch.
+static HipErr zero_counters(alens_ctx *ctx) {
+    ZeroJobs z{};
+    const int64_t n1 = (int64_t)ctx->n + 1;
+    uint32_t *bufs[8] = {ctx->cstart.p, ctx->cend.p, ctx->counter.p, ctx->cntI.p,
+                         ctx->cntJ.p,   ctx->cur.p,  ctx->cur2.p,    ctx->bar.p};
+    const int64_t lens[8] = {ctx->ncell, ctx->ncell, 1, n1, n1, n1, n1, kBarTotalWords};
+    for (int q = 0; q < 8; ++q) {
+        z.p[q] = bufs[q];
+        z.n[q] = lens[q];
+    }
+    z.count = 8;
+    return launch_zero_many(ctx->st, z);
+}
+
 // Enqueues the plan of the resident solves that ctx->route wants (k_resident_plan); mv: the row count of a
 // captured step, cleared when a plan does not fit.
 static alens_status launch_plan(alens_ctx *ctx, uint32_t *mv) {
@@ -1047,10 +1064,10 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     const RodsDev rd = make_rods(ctx);
     // caller rows: rods by gid, per-rod entry lists in ascending row order
     const uint32_t Me = (uint32_t)ctx->ext_pending.size();
-    std::vector<int32_t> eI(Me), eJ(Me);
-    std::vector<double> eD0(Me), eNrm(3 * (size_t)Me), ePI(3 * (size_t)Me), ePJ(3 * (size_t)Me), eX0(Me), eLb(Me),
-        eIk(Me);
-    std::vector<uint32_t> eStart, eEnt;
+    // (packed, so that they travel as one copy: the order of ExtRows)
+    const size_t ext_words = 13 * (size_t)Me + (4 * (size_t)Me + (size_t)n + 2) / 2;
+    std::vector<double> eblob(Me ? ext_words : 0);
+    const ExtRows eh = ext_rows(eblob.data(), Me, n);
     if (Me > 0) {
         if (ctx->nsys > 1) return fail(ctx, ALENS_E_STATE, "caller constraint blocks need a one-system context");
         if (!ctx->gid_index_ok) {
@@ -1059,7 +1076,11 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
             for (int32_t i = 0; i < n; ++i) ctx->gid_index[ctx->h_gid[i]] = i;
             ctx->gid_index_ok = true;
         }
-        eStart.assign((size_t)n + 1, 0);
+        double *eNrm = const_cast<double *>(eh.nrm), *ePI = const_cast<double *>(eh.posI), *ePJ = const_cast<double *>(eh.posJ);
+        double *eD0 = const_cast<double *>(eh.delta0), *eX0 = const_cast<double *>(eh.x0);
+        double *eLb = const_cast<double *>(eh.lb), *eIk = const_cast<double *>(eh.invk);
+        int32_t *eI = const_cast<int32_t *>(eh.I), *eJ = const_cast<int32_t *>(eh.J);
+        uint32_t *eStart = const_cast<uint32_t *>(eh.start), *eEnt = const_cast<uint32_t *>(eh.ent);
         for (uint32_t e = 0; e < Me; ++e) {
             const alens_con_block &cb = ctx->ext_pending[e];
             auto fi = ctx->gid_index.find(cb.gid_i), fj = ctx->gid_index.find(cb.gid_j);
@@ -1084,8 +1105,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
             eStart[(size_t)eJ[e] + 1]++;
         }
         for (int32_t i = 0; i < n; ++i) eStart[(size_t)i + 1] += eStart[i];
-        eEnt.resize(2 * (size_t)Me);
-        std::vector<uint32_t> cur(eStart.begin(), eStart.end() - 1);
+        std::vector<uint32_t> cur(eStart, eStart + n);
         for (uint32_t e = 0; e < Me; ++e) {
             eEnt[cur[eI[e]]++] = e;
             eEnt[cur[eJ[e]]++] = e | 0x80000000u;
@@ -1116,8 +1136,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
                            ctx->hist, ctx->scan, alt));
     const uint32_t *skeys = alt ? ctx->keys2.p : ctx->keys.p;
     const uint32_t *svals = alt ? ctx->vals2.p : ctx->vals.p;
-    TRY_HIP(hipMemsetAsync(ctx->cstart.p, 0, sizeof(uint32_t) * ctx->ncell, st));
-    TRY_HIP(hipMemsetAsync(ctx->cend.p, 0, sizeof(uint32_t) * ctx->ncell, st));
+    TRY_K(zero_counters(ctx));
     TRY_K(launch_cell_ranges(st, skeys, E, ctx->cstart.p, ctx->cend.p));
     // pair sweep (re-run once with a larger buffer if the pair buffer overflowed)
     if (ctx->pcap == 0) {
@@ -1129,9 +1148,11 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     }
     uint32_t M = 0;
     for (int attempt = 0; attempt < 2; ++attempt) {
-        TRY_HIP(hipMemsetAsync(ctx->counter.p, 0, sizeof(uint32_t), st));
-        TRY_HIP(hipMemsetAsync(ctx->cntI.p, 0, sizeof(uint32_t) * (n + 1), st));
-        TRY_HIP(hipMemsetAsync(ctx->cntJ.p, 0, sizeof(uint32_t) * (n + 1), st));
+        if (attempt > 0) {
+            TRY_HIP(hipMemsetAsync(ctx->counter.p, 0, sizeof(uint32_t), st));
+            TRY_HIP(hipMemsetAsync(ctx->cntI.p, 0, sizeof(uint32_t) * (n + 1), st));
+            TRY_HIP(hipMemsetAsync(ctx->cntJ.p, 0, sizeof(uint32_t) * (n + 1), st));
+        }
         TRY_K(launch_sweep(st, rd, cd, skeys, E, ctx->cstart.p, ctx->cend.p, svals, ctx->clo.p, ctx->blo.p, ctx->bhi.p,
                            ctx->counter.p, ctx->pcap, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->cntI.p,
                            ctx->cntJ.p));
@@ -1168,42 +1189,22 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     // canonical order + rows + adjacency
     TRY_K(exclusive_scan_u32(st, ctx->cntI.p, ctx->rowStart.p, n, ctx->scan));
     TRY_K(exclusive_scan_u32(st, ctx->cntJ.p, ctx->jStart.p, n, ctx->scan));
-    TRY_HIP(hipMemsetAsync(ctx->cur.p, 0, sizeof(uint32_t) * (n + 1), st));
     TRY_K(launch_order_I(st, n, Mcol, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->rowStart.p, ctx->cur.p, ctx->cI.p,
                          ctx->cJ.p, ctx->cImg.p));
-    TRY_HIP(hipMemsetAsync(ctx->cur.p, 0, sizeof(uint32_t) * (n + 1), st));
-    TRY_K(launch_order_J(st, n, Mcol, ctx->cJ.p, ctx->jStart.p, ctx->cur.p, ctx->jlist.p));
+    TRY_K(launch_order_J(st, n, Mcol, ctx->cJ.p, ctx->jStart.p, ctx->cur2.p, ctx->jlist.p));
     TRY_K(launch_rows(st, rd, cd, Mcol, M, ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->unc.p, ctx->delta0.p, ctx->geo.p,
                       ctx->posI.p, ctx->posJ.p, ctx->b.p));
+    ExtRows ed{};
     if (Me > 0) {
-        TRY_HIP(ctx->extStart.ensure((size_t)n + 1));
-        TRY_HIP(ctx->extEnt.ensure(2 * (size_t)Me));
-        TRY_HIP(ctx->extNrm.ensure(3 * (size_t)Me));
-        TRY_HIP(ctx->extX0.ensure(Me));
+        TRY_HIP(ctx->ext.ensure(ext_words));
         TRY_HIP(ctx->lb.ensure(Mc));
         TRY_HIP(ctx->invk.ensure(Mc));
-        TRY_HIP(hipMemcpyAsync(ctx->cI.p + Mcol, eI.data(), sizeof(int32_t) * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->cJ.p + Mcol, eJ.data(), sizeof(int32_t) * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemsetAsync(ctx->cImg.p + Mcol, 0, sizeof(uint32_t) * Me, st));
-        TRY_HIP(hipMemcpyAsync(ctx->delta0.p + Mcol, eD0.data(), sizeof(double) * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->posI.p + 3 * (size_t)Mcol, ePI.data(), sizeof(double) * 3 * Me,
-                               hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->posJ.p + 3 * (size_t)Mcol, ePJ.data(), sizeof(double) * 3 * Me,
-                               hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->extNrm.p, eNrm.data(), sizeof(double) * 3 * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->extX0.p, eX0.data(), sizeof(double) * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->extStart.p, eStart.data(), sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->extEnt.p, eEnt.data(), sizeof(uint32_t) * 2 * Me, hipMemcpyHostToDevice, st));
-        if (Mcol > 0) {
-            TRY_HIP(hipMemsetAsync(ctx->lb.p, 0, sizeof(double) * Mcol, st));  // 0.0 = all-zero bytes
-            TRY_HIP(hipMemsetAsync(ctx->invk.p, 0, sizeof(double) * Mcol, st));
-        }
-        TRY_HIP(hipMemcpyAsync(ctx->lb.p + Mcol, eLb.data(), sizeof(double) * Me, hipMemcpyHostToDevice, st));
-        TRY_HIP(hipMemcpyAsync(ctx->invk.p + Mcol, eIk.data(), sizeof(double) * Me, hipMemcpyHostToDevice, st));
-        TRY_K(launch_rows_ext(st, Me, Mcol, M, ctx->cI.p, ctx->cJ.p, ctx->extNrm.p, ctx->posI.p, ctx->posJ.p,
-                              ctx->delta0.p, ctx->unc.p, ctx->cfg.dt, ctx->geo.p, ctx->b.p));
+        TRY_HIP(hipMemcpyAsync(ctx->ext.p, eblob.data(), sizeof(double) * ext_words, hipMemcpyHostToDevice, st));
+        ed = ext_rows(ctx->ext.p, Me, n);
+        TRY_K(launch_rows_ext(st, Me, Mcol, M, ed, ctx->unc.p, ctx->cfg.dt, ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->delta0.p,
+                              ctx->posI.p, ctx->posJ.p, ctx->geo.p, ctx->b.p, ctx->lb.p, ctx->invk.p, ctx->xg.p));
     }
-    const uint32_t *xs = Me ? ctx->extStart.p : nullptr;
+    const uint32_t *xs = ed.start;
     {
         // sliced adjacency sizes; constraint range of each system = rowStart at its first rod (rows are
         // grouped by rod I; caller rows exist only with one system and close its range)
@@ -1243,7 +1244,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
         accept_plan(ctx, head);
         TRY_HIP(ctx->sellK.ensure(std::max<size_t>(ep, 1)));
         TRY_HIP(ctx->sellW.ensure(6 * std::max<size_t>(ep, 1)));
-        TRY_K(launch_adjacency(st, n, M, ctx->rowStart.p, ctx->jStart.p, ctx->jlist.p, xs, Me ? ctx->extEnt.p : nullptr,
+        TRY_K(launch_adjacency(st, n, M, ctx->rowStart.p, ctx->jStart.p, ctx->jlist.p, xs, ed.ent,
                                Mcol, ctx->geo.p, ctx->sellStart.p, ctx->epad, ctx->adjStart.p, ctx->sellK.p,
                                ctx->sellW.p, ctx->spos_cur));
     }
@@ -1276,10 +1277,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
             TRY_K(launch_mlp_infer_xg(st, Mcol, ctx->feat.p, ctx->mlpP.p, ctx->mlpNorm.p, ctx->xg.p));
             warm = true;
         }
-        if (Me > 0) {
-            TRY_K(launch_set_x(st, ctx->xg.p + Mcol, ctx->extX0.p, Me));
-            warm = true;
-        }
+        warm = warm || Me > 0;  // (the caller rows start from their blocks' gamma)
         alens_status s = ctx->cfg.precision == 1
                              ? run_solver_mixed(ctx, n, M, warm, &rep, &ms_solve)
                              : run_solver(ctx, n, M, ctx->mob.p, warm, &rep, &ms_solve, ctx->rsys.p, ctx->smono.p,
@@ -1446,21 +1444,8 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
                            ctx->scan, alt, Ee));
     const uint32_t *skeys = alt ? ctx->keys2.p : ctx->keys.p;
     const uint32_t *svals = alt ? ctx->vals2.p : ctx->vals.p;
-    {
-        // every counter and cursor of the step, and the solver's barrier words, in one launch
-        ZeroJobs z{};
-        uint32_t *bufs[8] = {ctx->cstart.p, ctx->cend.p, ctx->counter.p, ctx->cntI.p,
-                             ctx->cntJ.p,   ctx->cur.p,  ctx->cur2.p,    ctx->bar.p};
-        const int64_t lens[8] = {ctx->ncell, ctx->ncell, 1, (int64_t)n + 1, (int64_t)n + 1, (int64_t)n + 1,
-                                 (int64_t)n + 1, kBarTotalWords};
-        for (int q = 0; q < 8; ++q) {
-            z.p[q] = bufs[q];
-            z.n[q] = lens[q];
-        }
-        z.count = 8;
-        TRY_K(launch_zero_many(st, z));
-        ctx->bar_clean = true;
-    }
+    TRY_K(zero_counters(ctx));
+    ctx->bar_clean = true;
     TRY_K(launch_cell_ranges(st, skeys, c.E, ctx->cstart.p, ctx->cend.p, Ee));
     TRY_K(launch_sweep(st, rd, cd, skeys, c.E, ctx->cstart.p, ctx->cend.p, svals, ctx->clo.p, ctx->blo.p, ctx->bhi.p,
                        ctx->counter.p, c.M, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->cntI.p, ctx->cntJ.p, Ee));

@@ -882,18 +882,24 @@ HipErr launch_rows(hipStream_t st, const RodsDev &r, const CfgDev &c, uint32_t m
     return hip_ok();
 }
 
-// Caller-supplied rows k = k0 + e (the constraint pool): normal n = normI (uploaded into nrm),
-// arms posI / posJ given; rI = posI x n, rJ = posJ x n, b = delta0 + dt (D^T U_nc).
-__global__ void k_rows_ext(uint32_t me, uint32_t k0, uint32_t gs, const int32_t *__restrict__ cI,
-                           const int32_t *__restrict__ cJ, const double *__restrict__ nrm,
-                           const double *__restrict__ posI, const double *__restrict__ posJ,
-                           const double *__restrict__ delta0, const double *__restrict__ unc, double dt,
-                           double *__restrict__ geo, double *__restrict__ b) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= me) return;
-    const uint32_t k = k0 + e;
-    const double *nk = nrm + 3 * (size_t)e;
-    const double *pI = posI + 3 * (size_t)k, *pJ = posJ + 3 * (size_t)k;
+// Caller-supplied rows k = k0 + e (the constraint pool): normal n = normI, arms posI / posJ given; rI = posI x n,
+// rJ = posJ x n, b = delta0 + dt (D^T U_nc); start point x = the block's gamma.  The rows before them have lower
+// bound and compliance 0.
+__global__ void k_rows_ext(uint32_t me, uint32_t k0, uint32_t gs, ExtRows x, const double *__restrict__ unc, double dt,
+                           int32_t *__restrict__ cI, int32_t *__restrict__ cJ, uint32_t *__restrict__ cImg,
+                           double *__restrict__ delta0, double *__restrict__ posI, double *__restrict__ posJ,
+                           double *__restrict__ geo, double *__restrict__ b, double *__restrict__ lb,
+                           double *__restrict__ invk, double2 *__restrict__ xg) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= k0 + me) return;
+    if (k < k0) {
+        lb[k] = 0.0;
+        invk[k] = 0.0;
+        return;
+    }
+    const uint32_t e = k - k0;
+    const double *nk = x.nrm + 3 * (size_t)e;
+    const double *pI = x.posI + 3 * (size_t)e, *pJ = x.posJ + 3 * (size_t)e;
     double g9[9];
     g9[0] = nk[0];
     g9[1] = nk[1];
@@ -906,14 +912,28 @@ __global__ void k_rows_ext(uint32_t me, uint32_t k0, uint32_t gs, const int32_t 
     g9[8] = pJ[0] * nk[1] - pJ[1] * nk[0];
 #pragma unroll
     for (int a = 0; a < 9; ++a) geo[(size_t)a * gs + k] = g9[a];
-    b[k] = delta0[k] + dt * dt_row(g9, unc + 6 * (size_t)cI[k], unc + 6 * (size_t)cJ[k]);
+    const int32_t I = x.I[e], J = x.J[e];
+    b[k] = x.delta0[e] + dt * dt_row(g9, unc + 6 * (size_t)I, unc + 6 * (size_t)J);
+    cI[k] = I;
+    cJ[k] = J;
+    cImg[k] = 0u;
+    delta0[k] = x.delta0[e];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        posI[3 * (size_t)k + a] = pI[a];
+        posJ[3 * (size_t)k + a] = pJ[a];
+    }
+    lb[k] = x.lb[e];
+    invk[k] = x.invk[e];
+    xg[k] = make_double2(x.x0[e], 0.0);
 }
 
-HipErr launch_rows_ext(hipStream_t st, uint32_t me, uint32_t k0, uint32_t gs, const int32_t *cI, const int32_t *cJ,
-                       const double *nrm, const double *posI, const double *posJ, const double *delta0,
-                       const double *unc, double dt, double *geo, double *b) {
+HipErr launch_rows_ext(hipStream_t st, uint32_t me, uint32_t k0, uint32_t gs, const ExtRows &x, const double *unc, double dt,
+                       int32_t *cI, int32_t *cJ, uint32_t *cImg, double *delta0, double *posI, double *posJ, double *geo,
+                       double *b, double *lb, double *invk, double2 *xg) {
     if (me == 0) return hip_ok();
-    k_rows_ext<<<nblk(me, 256), 256, 0, st>>>(me, k0, gs, cI, cJ, nrm, posI, posJ, delta0, unc, dt, geo, b);
+    k_rows_ext<<<nblk((int64_t)k0 + me, 256), 256, 0, st>>>(me, k0, gs, x, unc, dt, cI, cJ, cImg, delta0, posI, posJ, geo, b, lb,
+                                                           invk, xg);
     LAUNCH_CHECK();
     return hip_ok();
 }

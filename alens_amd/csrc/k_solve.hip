@@ -1101,9 +1101,12 @@ __global__ void k_writeback(int32_t n, const int32_t *__restrict__ rsys, const S
                             const uint32_t *__restrict__ sellK, const double *__restrict__ sellW, uint64_t epad,
                             const double2 *__restrict__ xg,
                             const double *__restrict__ mob, const double *__restrict__ unc,
-                            double *__restrict__ F, double *__restrict__ U, const uint32_t *__restrict__ spos) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+                            double *__restrict__ F, double *__restrict__ U, const uint32_t *__restrict__ spos,
+                            double *__restrict__ gamma, uint32_t m, const uint32_t *__restrict__ md) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < dcount(m, md)) gamma[k] = xg[k].x;
+    if (k >= (uint32_t)n) return;
+    const int32_t i = (int32_t)k;
     const int mono = sys[rsys[i]].mono;
     double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const uint32_t deg = adjStart[i + 1] - adjStart[i];
@@ -1124,24 +1127,6 @@ __global__ void k_writeback(int32_t n, const int32_t *__restrict__ rsys, const S
         F[6 * (size_t)i + q] = f[q];
         U[6 * (size_t)i + q] = unc[6 * (size_t)i + q] + u[q];
     }
-}
-
-// start point of the caller rows k0 .. k0 + me: x = the blocks' gamma, g = 0
-__global__ void k_set_x(double2 *__restrict__ xg, const double *__restrict__ x0, uint32_t me) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < me) xg[e] = make_double2(x0[e], 0.0);
-}
-HipErr launch_set_x(hipStream_t st, double2 *xg, const double *x0, uint32_t me) {
-    if (me == 0) return hip_ok();
-    k_set_x<<<nblk(me, 256), 256, 0, st>>>(xg, x0, me);
-    LAUNCH_CHECK();
-    return hip_ok();
-}
-
-__global__ void k_copy_gamma(const double2 *__restrict__ xg, double *__restrict__ gamma, uint32_t m,
-                             const uint32_t *__restrict__ md) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < dcount(m, md)) gamma[k] = xg[k].x;
 }
 
 // gamma times the stress of a unit impulse, (lab_I - lab_J) (x) n, of rows [k0, k0 + count): nine words a row, in row
@@ -1190,13 +1175,10 @@ HipErr launch_writeback(hipStream_t st, int32_t n, const int32_t *rsys, const Sy
                         const uint32_t *sellStart, const uint32_t *sellK, const double *sellW, uint64_t epad,
                         const double2 *xg, const double *mob, const double *unc, double *F, double *U,
                         double *gamma, uint32_t m, const uint32_t *md, const uint32_t *spos) {
-    if (n > 0) {
-        k_writeback<<<nblk(n, 256), 256, 0, st>>>(n, rsys, sys, adjStart, sellStart, sellK, sellW, epad, xg, mob, unc,
-                                                  F, U, spos);
-        LAUNCH_CHECK();
-    }
-    if (m > 0) {
-        k_copy_gamma<<<nblk(m, 256), 256, 0, st>>>(xg, gamma, m, md);
+    const int64_t t = n > (int64_t)m ? n : (int64_t)m;
+    if (t > 0) {
+        k_writeback<<<nblk(t, 256), 256, 0, st>>>(n, rsys, sys, adjStart, sellStart, sellK, sellW, epad, xg, mob, unc, F, U,
+                                                  spos, gamma, m, md);
         LAUNCH_CHECK();
     }
     return hip_ok();

@@ -128,14 +128,23 @@ struct ScanScratch {
 // collide kernels (k_collide.hip)
 HipErr launch_mob_unc(hipStream_t st, const RodsDev &r, const double *length, const double *radius,
                       const uint8_t *immovable, const double *fext, const CfgDev &c, double *mob, double *unc);
-HipErr launch_aabb(hipStream_t st, const RodsDev &r, const CfgDev &c, int32_t *clo, int32_t *chi, double *blo,
-                   double *bhi, uint32_t *ecnt);
+// What the pair sweep reads of a rod, in one line each: its inflated box, the first cell of its box range and its
+// system; its segment (centre, direction, half length) and radius.
+struct alignas(16) RodBox {
+    double lo[3], hi[3];
+    int32_t cl[3], sys;
+};
+struct alignas(16) RodLine {
+    double c[3], t[3], h, r;
+};
+static_assert(sizeof(RodBox) == 64 && sizeof(RodLine) == 64, "a line each");
+HipErr launch_aabb(hipStream_t st, const RodsDev &r, int32_t *chi, RodBox *box, RodLine *line, uint32_t *ecnt);
 HipErr exclusive_scan_u32(hipStream_t st, const uint32_t *in, uint32_t *out, int64_t n,
                           ScanScratch &s);
 HipErr ensure_scan_scratch(ScanScratch &s, int64_t n);
 HipErr ensure_radix_scratch(DBuf<uint32_t> &hist, ScanScratch &s, int64_t n);
 // entries beyond ecap are not written (the count eoff[n] still tells how many there were)
-HipErr launch_fill_entries(hipStream_t st, const RodsDev &r, const int32_t *clo, const int32_t *chi,
+HipErr launch_fill_entries(hipStream_t st, const RodsDev &r, const RodBox *box, const int32_t *chi,
                            const uint32_t *eoff, uint32_t *keys, uint32_t *vals, uint32_t ecap);
 // n: capacity (grid); nd: device count or NULL
 HipErr radix_sort_pairs(hipStream_t st, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt,
@@ -161,8 +170,8 @@ HipErr launch_step_tail(hipStream_t st, const uint32_t *entries, const uint32_t 
 HipErr launch_cell_ranges(hipStream_t st, const uint32_t *keys, int64_t E, uint32_t *cstart,
                           uint32_t *cend, const uint32_t *Ed = nullptr);
 HipErr launch_sweep(hipStream_t st, const RodsDev &r, const CfgDev &c, const uint32_t *keys, int64_t E,
-                    const uint32_t *cstart, const uint32_t *cend, const uint32_t *vals, const int32_t *clo, const double *blo,
-                    const double *bhi, uint32_t *pair_count, uint32_t cap, uint32_t *pI, uint32_t *pJ,
+                    const uint32_t *cstart, const uint32_t *cend, const uint32_t *vals, const RodBox *box,
+                    const RodLine *line, uint32_t *pair_count, uint32_t cap, uint32_t *pI, uint32_t *pJ,
                     uint32_t *pImg, uint32_t *cntI, uint32_t *cntJ, const uint32_t *Ed = nullptr);
 HipErr launch_morton_keys(hipStream_t st, const RodsDev &r, int32_t i0, int32_t n, uint32_t *keys,
                           uint32_t *vals);
@@ -171,16 +180,16 @@ HipErr launch_permute_rods(hipStream_t st, int32_t n, const uint32_t *perm, cons
                            const double *hcol, const double *rcol, const uint8_t *immov, int32_t *gid2,
                            double *center2, double *dir2, double *length2, double *radius2, double *hcol2,
                            double *rcol2, uint8_t *immov2);
-HipErr launch_order_I(hipStream_t st, int32_t n, uint32_t m, const uint32_t *pI,
-                      const uint32_t *pJ, const uint32_t *pImg, const uint32_t *rowStart,
-                      uint32_t *cur, int32_t *cI, int32_t *cJ, uint32_t *cImg, const uint32_t *md = nullptr);
-HipErr launch_order_J(hipStream_t st, int32_t n, uint32_t m, const int32_t *cJ,
-                      const uint32_t *jStart, uint32_t *cur, uint32_t *jlist, const uint32_t *md = nullptr);
+// pairs into canonical order, and the J lists' rows (unsorted, in tmp: 16 B per row); launch_rows sorts the lists
+HipErr launch_order(hipStream_t st, uint32_t m, const uint32_t *pI, const uint32_t *pJ, const uint32_t *pImg,
+                    const uint32_t *rowStart, uint32_t *curI, const uint32_t *jStart, uint32_t *curJ, int32_t *cI,
+                    int32_t *cJ, uint32_t *cImg, void *tmp, const uint32_t *md = nullptr);
 // constraint geometry is stored component-major: geo[q * gs + k], q = 0..8 = {n, rI, rJ}, gs = the
 // step's total row count (collision rows first, then the caller's rows)
 HipErr launch_rows(hipStream_t st, const RodsDev &r, const CfgDev &c, uint32_t m, uint32_t gs, const int32_t *cI,
                    const int32_t *cJ, const uint32_t *cImg, const double *unc, double *delta0,
-                   double *geo, double *posI, double *posJ, double *b, const uint32_t *md = nullptr);
+                   double *geo, double *posI, double *posJ, double *b, const uint32_t *jStart, const void *tmp,
+                   uint32_t *jlist, const uint32_t *md = nullptr);
 // Caller rows of a step, packed into one buffer of 13 m words, then 4 m + n + 1 half words: fields, rods, and the
 // rods' entries (row | side << 31) with their starts
 struct ExtRows {

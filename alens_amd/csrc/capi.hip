@@ -51,8 +51,9 @@ struct alens_ctx {
     bool has_immov = false;
     DBuf<double> mob, unc, U, F, Us, fext;
 
-    DBuf<int32_t> clo, chi;
-    DBuf<double> blo, bhi;
+    DBuf<int32_t> chi;
+    DBuf<RodBox> rbox;
+    DBuf<RodLine> rline;
     DBuf<uint32_t> ecnt, eoff, keys, vals, keys2, vals2, cstart, cend, hist;
     ScanScratch scan;
 
@@ -281,7 +282,7 @@ void alens_destroy(alens_ctx *ctx) {
     auto rel = [](auto &b) { b.release(); };
     rel(ctx->gid); rel(ctx->center); rel(ctx->dir); rel(ctx->length); rel(ctx->radius); rel(ctx->hcol);
     rel(ctx->rcol); rel(ctx->immov); rel(ctx->mob); rel(ctx->unc); rel(ctx->U); rel(ctx->F); rel(ctx->Us);
-    rel(ctx->fext); rel(ctx->clo); rel(ctx->chi); rel(ctx->blo); rel(ctx->bhi); rel(ctx->ecnt);
+    rel(ctx->fext); rel(ctx->chi); rel(ctx->rbox); rel(ctx->rline); rel(ctx->ecnt);
     rel(ctx->eoff); rel(ctx->keys); rel(ctx->vals); rel(ctx->keys2); rel(ctx->vals2); rel(ctx->cstart);
     rel(ctx->cend); rel(ctx->hist);
     for (auto &l : ctx->scan.lvl) rel(l);
@@ -404,10 +405,9 @@ alens_status alens_set_systems(alens_ctx *ctx, int32_t nsys, const int32_t *rod_
     TRY_HIP(ctx->rsys.ensure(N));
     for (auto *bf : {&ctx->mob, &ctx->unc, &ctx->U, &ctx->F, &ctx->fext}) TRY_HIP(bf->ensure(6 * N));
     TRY_HIP(ctx->Us.ensure(kUStride * N));
-    TRY_HIP(ctx->clo.ensure(3 * N));
     TRY_HIP(ctx->chi.ensure(3 * N));
-    TRY_HIP(ctx->blo.ensure(3 * N));
-    TRY_HIP(ctx->bhi.ensure(3 * N));
+    TRY_HIP(ctx->rbox.ensure(N));
+    TRY_HIP(ctx->rline.ensure(N));
     TRY_HIP(ctx->ecnt.ensure(N + 1));
     TRY_HIP(ctx->eoff.ensure(N + 1));
     for (auto *bf : {&ctx->cntI, &ctx->cntJ, &ctx->rowStart, &ctx->jStart, &ctx->cur, &ctx->cur2, &ctx->adjStart})
@@ -1119,7 +1119,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     TRY_K(launch_mob_unc(st, rd, ctx->length.p, ctx->radius.p, ctx->has_immov ? ctx->immov.p : nullptr,
                          f_ext ? ctx->fext.p : nullptr, cd, ctx->mob.p, ctx->unc.p));
     // cell list
-    TRY_K(launch_aabb(st, rd, cd, ctx->clo.p, ctx->chi.p, ctx->blo.p, ctx->bhi.p, ctx->ecnt.p));
+    TRY_K(launch_aabb(st, rd, ctx->chi.p, ctx->rbox.p, ctx->rline.p, ctx->ecnt.p));
     TRY_K(exclusive_scan_u32(st, ctx->ecnt.p, ctx->eoff.p, n, ctx->scan));
     uint32_t E = 0;
     TRY_HIP(hipMemcpyAsync(&E, ctx->eoff.p + n, sizeof E, hipMemcpyDeviceToHost, st));
@@ -1130,7 +1130,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     TRY_HIP(ctx->vals.ensure(Ecap));
     TRY_HIP(ctx->keys2.ensure(Ecap));
     TRY_HIP(ctx->vals2.ensure(Ecap));
-    TRY_K(launch_fill_entries(st, rd, ctx->clo.p, ctx->chi.p, ctx->eoff.p, ctx->keys.p, ctx->vals.p, E));
+    TRY_K(launch_fill_entries(st, rd, ctx->rbox.p, ctx->chi.p, ctx->eoff.p, ctx->keys.p, ctx->vals.p, E));
     bool alt = false;
     TRY_K(radix_sort_pairs(st, ctx->keys.p, ctx->vals.p, ctx->keys2.p, ctx->vals2.p, E, ctx->keybits,
                            ctx->hist, ctx->scan, alt));
@@ -1153,7 +1153,7 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
             TRY_HIP(hipMemsetAsync(ctx->cntI.p, 0, sizeof(uint32_t) * (n + 1), st));
             TRY_HIP(hipMemsetAsync(ctx->cntJ.p, 0, sizeof(uint32_t) * (n + 1), st));
         }
-        TRY_K(launch_sweep(st, rd, cd, skeys, E, ctx->cstart.p, ctx->cend.p, svals, ctx->clo.p, ctx->blo.p, ctx->bhi.p,
+        TRY_K(launch_sweep(st, rd, cd, skeys, E, ctx->cstart.p, ctx->cend.p, svals, ctx->rbox.p, ctx->rline.p,
                            ctx->counter.p, ctx->pcap, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->cntI.p,
                            ctx->cntJ.p));
         TRY_HIP(hipMemcpyAsync(&M, ctx->counter.p, sizeof M, hipMemcpyDeviceToHost, st));
@@ -1189,11 +1189,11 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
     // canonical order + rows + adjacency
     TRY_K(exclusive_scan_u32(st, ctx->cntI.p, ctx->rowStart.p, n, ctx->scan));
     TRY_K(exclusive_scan_u32(st, ctx->cntJ.p, ctx->jStart.p, n, ctx->scan));
-    TRY_K(launch_order_I(st, n, Mcol, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->rowStart.p, ctx->cur.p, ctx->cI.p,
-                         ctx->cJ.p, ctx->cImg.p));
-    TRY_K(launch_order_J(st, n, Mcol, ctx->cJ.p, ctx->jStart.p, ctx->cur2.p, ctx->jlist.p));
+    // (the start points, set later, lend their memory)
+    TRY_K(launch_order(st, Mcol, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->rowStart.p, ctx->cur.p, ctx->jStart.p, ctx->cur2.p,
+                       ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->xg.p));
     TRY_K(launch_rows(st, rd, cd, Mcol, M, ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->unc.p, ctx->delta0.p, ctx->geo.p,
-                      ctx->posI.p, ctx->posJ.p, ctx->b.p));
+                      ctx->posI.p, ctx->posJ.p, ctx->b.p, ctx->jStart.p, ctx->xg.p, ctx->jlist.p));
     ExtRows ed{};
     if (Me > 0) {
         TRY_HIP(ctx->ext.ensure(ext_words));
@@ -1435,10 +1435,10 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
     TRY_K(launch_stamp(st, ctx->stamps.p, 0));
     TRY_K(launch_mob_unc(st, rd, ctx->length.p, ctx->radius.p, ctx->has_immov ? ctx->immov.p : nullptr,
                          fx ? ctx->fext.p : nullptr, cd, ctx->mob.p, ctx->unc.p));
-    TRY_K(launch_aabb(st, rd, cd, ctx->clo.p, ctx->chi.p, ctx->blo.p, ctx->bhi.p, ctx->ecnt.p));
+    TRY_K(launch_aabb(st, rd, ctx->chi.p, ctx->rbox.p, ctx->rline.p, ctx->ecnt.p));
     TRY_K(exclusive_scan_u32(st, ctx->ecnt.p, ctx->eoff.p, n, ctx->scan));
     TRY_K(launch_guard_entries(st, ctx->eoff.p + n, c.E, Ee));
-    TRY_K(launch_fill_entries(st, rd, ctx->clo.p, ctx->chi.p, ctx->eoff.p, ctx->keys.p, ctx->vals.p, c.E));
+    TRY_K(launch_fill_entries(st, rd, ctx->rbox.p, ctx->chi.p, ctx->eoff.p, ctx->keys.p, ctx->vals.p, c.E));
     bool alt = false;
     TRY_K(radix_sort_pairs(st, ctx->keys.p, ctx->vals.p, ctx->keys2.p, ctx->vals2.p, c.E, ctx->keybits, ctx->hist,
                            ctx->scan, alt, Ee));
@@ -1447,16 +1447,15 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
     TRY_K(zero_counters(ctx));
     ctx->bar_clean = true;
     TRY_K(launch_cell_ranges(st, skeys, c.E, ctx->cstart.p, ctx->cend.p, Ee));
-    TRY_K(launch_sweep(st, rd, cd, skeys, c.E, ctx->cstart.p, ctx->cend.p, svals, ctx->clo.p, ctx->blo.p, ctx->bhi.p,
+    TRY_K(launch_sweep(st, rd, cd, skeys, c.E, ctx->cstart.p, ctx->cend.p, svals, ctx->rbox.p, ctx->rline.p,
                        ctx->counter.p, c.M, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->cntI.p, ctx->cntJ.p, Ee));
     TRY_K(launch_guard_pairs(st, ctx->counter.p, c.M, Mv, ctx->cntI.p, ctx->cntJ.p, n));
     TRY_K(exclusive_scan_u32(st, ctx->cntI.p, ctx->rowStart.p, n, ctx->scan));
     TRY_K(exclusive_scan_u32(st, ctx->cntJ.p, ctx->jStart.p, n, ctx->scan));
-    TRY_K(launch_order_I(st, n, c.M, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->rowStart.p, ctx->cur.p, ctx->cI.p,
-                         ctx->cJ.p, ctx->cImg.p, Mv));
-    TRY_K(launch_order_J(st, n, c.M, ctx->cJ.p, ctx->jStart.p, ctx->cur2.p, ctx->jlist.p, Mv));
+    TRY_K(launch_order(st, c.M, ctx->pI.p, ctx->pJ.p, ctx->pImg.p, ctx->rowStart.p, ctx->cur.p, ctx->jStart.p, ctx->cur2.p,
+                       ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->xg.p, Mv));
     TRY_K(launch_rows(st, rd, cd, c.M, c.M, ctx->cI.p, ctx->cJ.p, ctx->cImg.p, ctx->unc.p, ctx->delta0.p,
-                      ctx->geo.p, ctx->posI.p, ctx->posJ.p, ctx->b.p, Mv));
+                      ctx->geo.p, ctx->posI.p, ctx->posJ.p, ctx->b.p, ctx->jStart.p, ctx->xg.p, ctx->jlist.p, Mv));
     const int64_t nsl = ((int64_t)n + kSlice - 1) / kSlice;
     ctx->sord_cur = ctx->spos_cur = nullptr;
     if (slot_order_on()) {

@@ -19,6 +19,9 @@ namespace alens {
     } while (0)
 
 static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+// Threads per block of kernels with one item per thread: waves of their own while that gives a CU no more than four
+// of 256 (a CU serves about one lane request per ns, so items spread over more CUs are served faster).
+static inline int blk(int64_t n) { return n <= 65536 ? 64 : 256; }
 
 // ------------------------------------------------------------------------------------------------
 // mobility + U_nc = M F_ext + U_B.  U_B = sqrt(2 kT/dt) M^{1/2} xi, xi from Philox4x32-10 keyed by
@@ -105,7 +108,7 @@ __global__ void k_mob_unc(int32_t n, const int32_t *__restrict__ rsys, const Sys
 HipErr launch_mob_unc(hipStream_t st, const RodsDev &r, const double *length, const double *radius,
                       const uint8_t *immovable, const double *fext, const CfgDev &c, double *mob, double *unc) {
     if (r.n == 0) return hip_ok();
-    k_mob_unc<<<nblk(r.n, 256), 256, 0, st>>>(r.n, r.rsys, r.sys, r.gid, r.dir, length, radius, immovable, fext, c,
+    k_mob_unc<<<nblk(r.n, blk(r.n)), blk(r.n), 0, st>>>(r.n, r.rsys, r.sys, r.gid, r.dir, length, radius, immovable, fext, c,
                                               mob, unc);
     LAUNCH_CHECK();
     return hip_ok();
@@ -139,13 +142,13 @@ __device__ inline bool slab_interval(const SysDev &S, int k, double ck, double t
     return s0 <= s1;
 }
 
-// Calls f(u) for the cells (unwrapped indices, inside the box range a..b) that the segment grown by
-// rho meets: for each (y, z) row, the parameter interval inside the row's grown slabs gives the
+// Calls f(ulo, uhi, uy, uz) for the rows of cells (unwrapped indices, inside the box range a..b) that the segment
+// grown by rho meets: for each (y, z) row, the parameter interval inside the row's grown slabs gives the
 // segment's x extent there, and the row's cells are those whose grown x range meets it.  A superset
 // of the cells within rho of the segment (rho carries a 1e-6 um margin, far above rounding).
 template <class F>
-__device__ inline void for_tube_cells(const SysDev &S, const double c[3], const double t[3], double hh,
-                                      const int a[3], const int b[3], double rho, F f) {
+__device__ inline void for_tube_rows(const SysDev &S, const double c[3], const double t[3], double hh,
+                                     const int a[3], const int b[3], double rho, F f) {
     int u[3];
     for (u[2] = a[2]; u[2] <= b[2]; ++u[2]) {
         double z0 = -hh, z1 = hh;
@@ -159,21 +162,22 @@ __device__ inline void for_tube_cells(const SysDev &S, const double c[3], const 
             int uhi = (int)floor((xhi + rho - S.box_lo[0]) / S.h[0]);
             ulo = ulo < a[0] ? a[0] : ulo;
             uhi = uhi > b[0] ? b[0] : uhi;
-            for (u[0] = ulo; u[0] <= uhi; ++u[0]) f(u);
+            if (ulo <= uhi) f(ulo, uhi, u[1], u[2]);
         }
     }
 }
 
-__global__ void k_aabb(RodsDev r, CfgDev c, int32_t *__restrict__ clo, int32_t *__restrict__ chi,
-                       double *__restrict__ blo, double *__restrict__ bhi, uint32_t *__restrict__ ecnt) {
+__global__ void k_aabb(RodsDev r, int32_t *__restrict__ chi, RodBox *__restrict__ box, RodLine *__restrict__ line,
+                       uint32_t *__restrict__ ecnt) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= r.n) return;
-    const SysDev &S = r.sys[r.rsys[i]];
+    RodBox bx;
+    bx.sys = r.rsys[i];
+    const SysDev &S = r.sys[bx.sys];
     const double hh = r.hcol[i];
     // one inflation per system (the largest radius): a contact's closest-point midpoint then lies
     // inside both rods' boxes and tubes, whatever their radii
     const double infl = S.infl;
-    (void)c;
     int a3[3], b3[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -186,25 +190,26 @@ __global__ void k_aabb(RodsDev r, CfgDev c, int32_t *__restrict__ clo, int32_t *
             a = a < 0 ? 0 : (a >= S.nc[k] ? S.nc[k] - 1 : a);
             b = b < 0 ? 0 : (b >= S.nc[k] ? S.nc[k] - 1 : b);
         }
-        clo[3 * i + k] = a;
         chi[3 * i + k] = b;
-        blo[3 * i + k] = lo;
-        bhi[3 * i + k] = hi;
+        bx.cl[k] = a;
+        bx.lo[k] = lo;
+        bx.hi[k] = hi;
         a3[k] = a;
         b3[k] = b;
     }
     // entries: the cells of the box range that the inflated segment meets
     const double ci[3] = {r.center[3 * i], r.center[3 * i + 1], r.center[3 * i + 2]};
     const double ti[3] = {r.dir[3 * i], r.dir[3 * i + 1], r.dir[3 * i + 2]};
+    box[i] = bx;
+    line[i] = RodLine{{ci[0], ci[1], ci[2]}, {ti[0], ti[1], ti[2]}, hh, r.rcol[i]};
     uint32_t cnt = 0;
-    for_tube_cells(S, ci, ti, hh, a3, b3, infl, [&](const int *) { ++cnt; });
+    for_tube_rows(S, ci, ti, hh, a3, b3, infl, [&](int ulo, int uhi, int, int) { cnt += (uint32_t)(uhi - ulo + 1); });
     ecnt[i] = cnt;
 }
 
-HipErr launch_aabb(hipStream_t st, const RodsDev &r, const CfgDev &c, int32_t *clo, int32_t *chi, double *blo,
-                   double *bhi, uint32_t *ecnt) {
+HipErr launch_aabb(hipStream_t st, const RodsDev &r, int32_t *chi, RodBox *box, RodLine *line, uint32_t *ecnt) {
     if (r.n == 0) return hip_ok();
-    k_aabb<<<nblk(r.n, 256), 256, 0, st>>>(r, c, clo, chi, blo, bhi, ecnt);
+    k_aabb<<<nblk(r.n, blk(r.n)), blk(r.n), 0, st>>>(r, chi, box, line, ecnt);
     LAUNCH_CHECK();
     return hip_ok();
 }
@@ -323,7 +328,7 @@ HipErr exclusive_scan_u32(hipStream_t st, const uint32_t *in, uint32_t *out, int
 // cell entries: rod i writes (wrapped cell id, i) for every cell of its range, rod-major, so the
 // stable sort below leaves each cell's rods in ascending index order.
 // ------------------------------------------------------------------------------------------------
-__global__ void k_fill_entries(RodsDev r, const int32_t *__restrict__ clo, const int32_t *__restrict__ chi,
+__global__ void k_fill_entries(RodsDev r, const RodBox *__restrict__ box, const int32_t *__restrict__ chi,
                                const uint32_t *__restrict__ eoff, uint32_t *__restrict__ keys,
                                uint32_t *__restrict__ vals, uint32_t ecap) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -334,24 +339,26 @@ __global__ void k_fill_entries(RodsDev r, const int32_t *__restrict__ clo, const
     const double ci[3] = {r.center[3 * i], r.center[3 * i + 1], r.center[3 * i + 2]};
     const double ti[3] = {r.dir[3 * i], r.dir[3 * i + 1], r.dir[3 * i + 2]};
     const double hh = r.hcol[i];
-    const int a3[3] = {clo[3 * i], clo[3 * i + 1], clo[3 * i + 2]};
+    const int a3[3] = {box[i].cl[0], box[i].cl[1], box[i].cl[2]};
     const int b3[3] = {chi[3 * i], chi[3 * i + 1], chi[3 * i + 2]};
     // the same cells, in the same order, as k_aabb counted (never more than its count)
-    for_tube_cells(g, ci, ti, hh, a3, b3, g.infl, [&](const int *u) {
-        if (w >= wend) return;
-        const uint32_t cx = (uint32_t)pmod_i(u[0], g.nc[0]);
-        const uint32_t cy = (uint32_t)pmod_i(u[1], g.nc[1]);
-        const uint32_t cz = (uint32_t)pmod_i(u[2], g.nc[2]);
-        keys[w] = g.cell_off + (cz * (uint32_t)g.nc[1] + cy) * (uint32_t)g.nc[0] + cx;
-        vals[w] = (uint32_t)i;
-        ++w;
+    // (wrapped once per row: integer remainders were most of the work, 351 -> 265 us for 10.1M entries)
+    for_tube_rows(g, ci, ti, hh, a3, b3, g.infl, [&](int ulo, int uhi, int uy, int uz) {
+        const uint32_t cy = (uint32_t)pmod_i(uy, g.nc[1]), cz = (uint32_t)pmod_i(uz, g.nc[2]);
+        const uint32_t row = g.cell_off + (cz * (uint32_t)g.nc[1] + cy) * (uint32_t)g.nc[0];
+        int cx = pmod_i(ulo, g.nc[0]);
+        for (int u = ulo; u <= uhi && w < wend; ++u, ++w) {
+            keys[w] = row + (uint32_t)cx;
+            vals[w] = (uint32_t)i;
+            cx = cx + 1 == g.nc[0] ? 0 : cx + 1;
+        }
     });
 }
 
-HipErr launch_fill_entries(hipStream_t st, const RodsDev &r, const int32_t *clo, const int32_t *chi,
+HipErr launch_fill_entries(hipStream_t st, const RodsDev &r, const RodBox *box, const int32_t *chi,
                            const uint32_t *eoff, uint32_t *keys, uint32_t *vals, uint32_t ecap) {
     if (r.n == 0) return hip_ok();
-    k_fill_entries<<<nblk(r.n, 256), 256, 0, st>>>(r, clo, chi, eoff, keys, vals, ecap);
+    k_fill_entries<<<nblk(r.n, blk(r.n)), blk(r.n), 0, st>>>(r, box, chi, eoff, keys, vals, ecap);
     LAUNCH_CHECK();
     return hip_ok();
 }
@@ -525,7 +532,8 @@ HipErr launch_cell_ranges(hipStream_t st, const uint32_t *keys, int64_t E, uint3
 // Found pairs are staged in LDS (an LDS counter per block) and reserved in the global list with one
 // atomic per block at the end; a block that fills its stage reserves the rest one by one.
 constexpr int kSweepT = 256;
-constexpr int kStage = 512;
+constexpr int kStage = 256;                            // pairs found, before they go to memory
+constexpr int kSweepQ = 128;                           // a wave's candidates: fewer than 64 wait, at most 64 come
 constexpr int kSweepPre = 64;                          // entries staged before the block's own
 constexpr int kSweepS = kSweepPre + kSweepT + 64;      // and after them
 
@@ -540,19 +548,30 @@ struct SweepBox {
     double lo[3], hi[3];
 };
 
+// d mod n where d is seldom a period away from its residue
+__device__ inline int near_pmod(int d, int n) {
+    d = d < 0 ? d + n : d;
+    return d >= 0 && d < n ? d : pmod_i(d, n);
+}
+
+// Bound by the vector units (FP64 distance tests) and, before, by lane requests: rods' boxes and segments are now a
+// line each instead of ten scattered words.  Pairs whose boxes meet wait in a queue of the wave until there is one
+// for every lane of the distance test.  10.1M entries 1,739 -> 1,505 us, 1.48M 195 -> 173 us.
 // four waves per SIMD (at most 128 VGPRs): measured faster than three with more registers, and than
 // five with spills
 __global__ __launch_bounds__(kSweepT) __attribute__((amdgpu_waves_per_eu(4)))
 void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int64_t E,
                      const uint32_t *__restrict__ cstart, const uint32_t *__restrict__ cend,
-                     const uint32_t *__restrict__ vals, const int32_t *__restrict__ clo,
-                     const double *__restrict__ blo, const double *__restrict__ bhi,
-                     uint32_t *__restrict__ pair_count, uint32_t cap, uint32_t *__restrict__ pI,
+                     const uint32_t *__restrict__ vals, const RodBox *__restrict__ box,
+                     const RodLine *__restrict__ line, uint32_t *__restrict__ pair_count, uint32_t cap, uint32_t *__restrict__ pI,
                      uint32_t *__restrict__ pJ, uint32_t *__restrict__ pImg, uint32_t *__restrict__ cntI,
                      uint32_t *__restrict__ cntJ, const uint32_t *__restrict__ Ed) {
     E = dcount((uint32_t)E, Ed);
     __shared__ uint32_t s_n, s_base;
     __shared__ uint32_t s_pi[kStage], s_pj[kStage], s_pm[kStage];
+    // candidates of each wave: rods, image and cell (i's frame) of pairs whose boxes meet
+    __shared__ uint32_t q_i[kSweepT / 64][kSweepQ], q_j[kSweepT / 64][kSweepQ], q_m[kSweepT / 64][kSweepQ];
+    __shared__ int q_u[3][kSweepT / 64][kSweepQ];
     // box data of entries e0 - kSweepPre .. e0 + kSweepT + 64, structure of arrays
     __shared__ uint32_t s_id[kSweepS];
     __shared__ int s_u[3][kSweepS];
@@ -564,26 +583,27 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
     const int64_t e = e0 + threadIdx.x;
     // cell coordinates of a cell id in its system's grid
     auto cell_xyz = [](uint32_t lc, const int (&n)[3], int (&x)[3]) {
-        x[0] = (int)(lc % (uint32_t)n[0]);
-        x[1] = (int)((lc / (uint32_t)n[0]) % (uint32_t)n[1]);
-        x[2] = (int)(lc / ((uint32_t)n[0] * (uint32_t)n[1]));
+        const uint32_t yz = lc / (uint32_t)n[0], z = yz / (uint32_t)n[1];
+        x[0] = (int)(lc - yz * (uint32_t)n[0]);
+        x[1] = (int)(yz - z * (uint32_t)n[1]);
+        x[2] = (int)z;
     };
     for (int q = threadIdx.x; q < kSweepS; q += blockDim.x) {
         const int64_t eq = es + q;
         if (eq < 0) continue;
         if (eq >= E) break;
         const uint32_t j = vals[eq];
-        const SysDev &g = r.sys[r.rsys[j]];
+        const RodBox bx = box[j];
+        const SysDev &g = r.sys[bx.sys];
         const int gn[3] = {g.nc[0], g.nc[1], g.nc[2]};
         int x[3];
         cell_xyz(keys[eq] - g.cell_off, gn, x);
         s_id[q] = j;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const int cl = clo[3 * j + k];
-            s_u[k][q] = g.pbc[k] ? cl + pmod_i(x[k] - cl, gn[k]) : x[k];
-            s_lo[k][q] = blo[3 * j + k];
-            s_hi[k][q] = bhi[3 * j + k];
+            s_u[k][q] = g.pbc[k] ? bx.cl[k] + near_pmod(x[k] - bx.cl[k], gn[k]) : x[k];
+            s_lo[k][q] = bx.lo[k];
+            s_hi[k][q] = bx.hi[k];
         }
     }
     if (threadIdx.x == 0) s_n = 0;
@@ -592,7 +612,7 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
     uint32_t cnt = 0, cs = 0, kc = 1, rr = 0;
     int cc[3] = {0, 0, 0};
     int pbc[3] = {0, 0, 0}, nc[3] = {1, 1, 1};
-    double len[3] = {0, 0, 0}, blo0[3] = {0, 0, 0}, hcell[3] = {1, 1, 1};
+    double len[3] = {0, 0, 0};
     // an entry of this lane's cell (its own, or a partner outside the stage)
     auto box_of = [&](int64_t ex) {
         SweepBox w;
@@ -607,12 +627,12 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
             }
         } else {
             w.id = vals[ex];
+            const RodBox bx = box[w.id];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const int cl = clo[3 * w.id + k];
-                w.u[k] = pbc[k] ? cl + pmod_i(cc[k] - cl, nc[k]) : cc[k];
-                w.lo[k] = blo[3 * w.id + k];
-                w.hi[k] = bhi[3 * w.id + k];
+                w.u[k] = pbc[k] ? bx.cl[k] + near_pmod(cc[k] - bx.cl[k], nc[k]) : cc[k];
+                w.lo[k] = bx.lo[k];
+                w.hi[k] = bx.hi[k];
             }
         }
         return w;
@@ -631,8 +651,6 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
             pbc[k] = g.pbc[k];
             nc[k] = g.nc[k];
             len[k] = g.len[k];
-            blo0[k] = g.box_lo[k];
-            hcell[k] = g.h[k];
         }
         cell_xyz(cell - g.cell_off, nc, cc);
     }
@@ -642,57 +660,81 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
         const uint32_t v = __shfl_xor(maxc, o, 64);
         maxc = v > maxc ? v : maxc;
     }
-    for (uint32_t t = 0; t < maxc; ++t) {
+    const int wv = threadIdx.x >> 6;
+    uint32_t t = 0, nq = 0;  // the wave's tests so far, its candidates
+    for (;;) {
+        if (t < maxc) {
+            // box test of one pair per lane; a pair that meets waits for the wave's distance test
+            bool meet = false;
+            uint32_t i = 0, j = 0;
+            int m[3] = {0, 0, 0}, ui[3] = {0, 0, 0};
+            if (t < cnt) {
+                uint32_t r2 = rr + 1u + t;
+                if (r2 >= kc) r2 -= kc;
+                const int64_t ep = (int64_t)cs + r2;
+                const SweepBox pw = box_of(ep);
+                // rod i is the pair's lower entry
+                const bool lo_own = e < ep;
+                const SweepBox &wi = lo_own ? own : pw;
+                const SweepBox &wj = lo_own ? pw : own;
+                i = wi.id;
+                j = wj.id;
+                meet = true;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    ui[k] = wi.u[k];
+                    const int du = ui[k] - wj.u[k];  // a whole number of periods (0 if not periodic)
+                    m[k] = du == 0 ? 0 : (du == nc[k] ? 1 : (du == -nc[k] ? -1 : du / nc[k]));
+                    const double sh = pbc[k] ? (double)m[k] * len[k] : 0.0;
+                    meet = meet && (wj.lo[k] + sh <= wi.hi[k]) && (wi.lo[k] <= wj.hi[k] + sh);
+                }
+            }
+            const uint64_t mm = __ballot(meet);
+            if (meet) {
+                const uint32_t q = nq + (uint32_t)__popcll(mm & lt);
+                q_i[wv][q] = i;
+                q_j[wv][q] = j;
+                q_m[wv][q] = img_pack(m[0], m[1], m[2]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) q_u[k][wv][q] = ui[k];
+            }
+            nq += (uint32_t)__popcll(mm);
+            ++t;
+        }
+        if (nq < 64u && t < maxc) continue;
+        if (nq == 0u) break;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes' candidates
+        // distance test of the last candidates, one per lane
+        const uint32_t take = nq < 64u ? nq : 64u;
+        nq -= take;
         bool pass = false;
-        uint32_t i = 0, j = 0;
-        int m[3] = {0, 0, 0};
-        if (t < cnt) {
-            uint32_t r2 = rr + 1u + t;
-            if (r2 >= kc) r2 -= kc;
-            const int64_t ep = (int64_t)cs + r2;
-            const SweepBox pw = box_of(ep);
-            // rod i is the pair's lower entry
-            const bool lo_own = e < ep;
-            const SweepBox &wi = lo_own ? own : pw;
-            const SweepBox &wj = lo_own ? pw : own;
-            i = wi.id;
-            j = wj.id;
-            int ui[3];
-            bool ok = true;
+        uint32_t i = 0, j = 0, im = 0;
+        if ((uint32_t)lane < take) {
+            const uint32_t q = nq + (uint32_t)lane;
+            i = q_i[wv][q];
+            j = q_j[wv][q];
+            im = q_m[wv][q];
+            const SysDev &g = r.sys[box[i].sys];
+            const RodLine li = line[i], lj = line[j];
+            const double *ci = li.c, *ti = li.t, *tj = lj.t;
+            double cj[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) cj[k] = g.pbc[k] ? lj.c[k] + (double)img_get(im, k) * g.len[k] : lj.c[k];
+            const SegRes sg = segseg(ci[0], ci[1], ci[2], ti[0], ti[1], ti[2], li.h, cj[0], cj[1], cj[2], tj[0], tj[1],
+                                     tj[2], lj.h);
+            const double d0 = (sg.dist - li.r) - lj.r;
+            pass = d0 < c.col_buf;
+            // the cell of the closest-point midpoint, in i's unwrapped frame
+            const double D[3] = {sg.D0, sg.D1, sg.D2};
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                ui[k] = wi.u[k];
-                const int du = ui[k] - wj.u[k];  // a whole number of periods (0 if not periodic)
-                m[k] = du == 0 ? 0 : du / nc[k];
-                const double sh = pbc[k] ? (double)m[k] * len[k] : 0.0;
-                ok = ok && (wj.lo[k] + sh <= wi.hi[k]) && (wi.lo[k] <= wj.hi[k] + sh);
-            }
-            if (ok) {
-                double ci[3], ti[3], cj[3], tj[3];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    ci[k] = r.center[3 * i + k];
-                    ti[k] = r.dir[3 * i + k];
-                    const double ck = r.center[3 * j + k];
-                    cj[k] = pbc[k] ? ck + (double)m[k] * len[k] : ck;
-                    tj[k] = r.dir[3 * j + k];
-                }
-                const double hi_ = r.hcol[i], ri = r.rcol[i], hj = r.hcol[j], rj = r.rcol[j];
-                const SegRes sg = segseg(ci[0], ci[1], ci[2], ti[0], ti[1], ti[2], hi_, cj[0], cj[1], cj[2], tj[0], tj[1],
-                                         tj[2], hj);
-                const double d0 = (sg.dist - ri) - rj;
-                pass = d0 < c.col_buf;
-                // the cell of the closest-point midpoint, in i's unwrapped frame
-                const double D[3] = {sg.D0, sg.D1, sg.D2};
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const double mk = (ci[k] + sg.s * ti[k]) - 0.5 * D[k];
-                    int um = (int)floor((mk - blo0[k]) / hcell[k]);
-                    if (!pbc[k]) um = um < 0 ? 0 : (um >= nc[k] ? nc[k] - 1 : um);
-                    pass = pass && um == ui[k];
-                }
+                const double mk = (ci[k] + sg.s * ti[k]) - 0.5 * D[k];
+                int um = (int)floor((mk - g.box_lo[k]) / g.h[k]);
+                if (!g.pbc[k]) um = um < 0 ? 0 : (um >= g.nc[k] ? g.nc[k] - 1 : um);
+                pass = pass && um == q_u[k][wv][q];
             }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read before the places are written again
         const uint64_t mask = __ballot(pass);
         if (mask) {
             const int leader = __ffsll((unsigned long long)mask) - 1;
@@ -701,7 +743,6 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
             base = __shfl(base, leader, 64);
             if (pass) {
                 const uint32_t q = base + (uint32_t)__popcll(mask & lt);
-                const uint32_t im = img_pack(m[0], m[1], m[2]);
                 if (q < (uint32_t)kStage) {
                     s_pi[q] = i;
                     s_pj[q] = j;
@@ -734,93 +775,63 @@ void k_sweep_entries(RodsDev r, CfgDev c, const uint32_t *__restrict__ keys, int
 }
 
 HipErr launch_sweep(hipStream_t st, const RodsDev &r, const CfgDev &c, const uint32_t *keys, int64_t E,
-                    const uint32_t *cstart, const uint32_t *cend, const uint32_t *vals, const int32_t *clo,
-                    const double *blo, const double *bhi, uint32_t *pair_count, uint32_t cap, uint32_t *pI,
+                    const uint32_t *cstart, const uint32_t *cend, const uint32_t *vals, const RodBox *box,
+                    const RodLine *line, uint32_t *pair_count, uint32_t cap, uint32_t *pI,
                     uint32_t *pJ, uint32_t *pImg, uint32_t *cntI, uint32_t *cntJ, const uint32_t *Ed) {
     if (E == 0) return hip_ok();
-    k_sweep_entries<<<nblk(E, kSweepT), kSweepT, 0, st>>>(r, c, keys, E, cstart, cend, vals, clo, blo, bhi, pair_count,
+    k_sweep_entries<<<nblk(E, kSweepT), kSweepT, 0, st>>>(r, c, keys, E, cstart, cend, vals, box, line, pair_count,
                                                           cap, pI, pJ, pImg, cntI, cntJ, Ed);
     LAUNCH_CHECK();
     return hip_ok();
 }
 
 // ------------------------------------------------------------------------------------------------
-// Canonical order: pairs grouped by I (scatter to rowStart[I] + atomic cursor), then each I-group
-// sorted by J by one thread (groups hold a handful of contacts).  The J-side lists hold constraint
-// indices, sorted ascending per rod.
+// Canonical order: pairs grouped by I (scatter to rowStart[I] + atomic cursor), each I-group sorted by J; the J-side
+// lists hold row indices, sorted ascending per rod.  A group's members (a handful) each count those before them and
+// go straight to their places: independent reads, where a thread per rod moved its members one by one (9.7k rods:
+// 16 + 12 us for both sorts; here 3 + 3 us, and k_rows does the second).  tmp: 16 B per row.
 // ------------------------------------------------------------------------------------------------
 __global__ void k_scatter_I(uint32_t m, const uint32_t *__restrict__ pI, const uint32_t *__restrict__ pJ,
                             const uint32_t *__restrict__ pImg, const uint32_t *__restrict__ rowStart,
                             uint32_t *__restrict__ cur, int32_t *__restrict__ cI,
-                            int32_t *__restrict__ cJ, uint32_t *__restrict__ cImg, const uint32_t *__restrict__ md) {
+                            uint2 *__restrict__ tmp, const uint32_t *__restrict__ md) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= dcount(m, md)) return;
     const uint32_t i = pI[p];
     const uint32_t pos = rowStart[i] + atomicAdd(&cur[i], 1u);
     cI[pos] = (int32_t)i;
-    cJ[pos] = (int32_t)pJ[p];
-    cImg[pos] = pImg[p];
+    tmp[pos] = make_uint2(pJ[p], pImg[p]);
 }
 
-__global__ void k_sort_I(int32_t n, const uint32_t *__restrict__ rowStart, int32_t *__restrict__ cJ,
-                         uint32_t *__restrict__ cImg) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+// row p of the scattered pairs to its place k; k into the list of its rod J (in any order)
+__global__ void k_rank_I(uint32_t m, const uint32_t *__restrict__ rowStart, const uint2 *__restrict__ tmp,
+                         const int32_t *__restrict__ cI, int32_t *__restrict__ cJ, uint32_t *__restrict__ cImg,
+                         const uint32_t *__restrict__ jStart, uint32_t *__restrict__ cur, uint32_t *__restrict__ jtmp,
+                         const uint32_t *__restrict__ md) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= dcount(m, md)) return;
+    const int32_t i = cI[p];
     const uint32_t s0 = rowStart[i], s1 = rowStart[i + 1];
-    for (uint32_t a = s0 + 1; a < s1; ++a) {
-        const int32_t kj = cJ[a];
-        const uint32_t km = cImg[a];
-        uint32_t b = a;
-        while (b > s0 && cJ[b - 1] > kj) {
-            cJ[b] = cJ[b - 1];
-            cImg[b] = cImg[b - 1];
-            --b;
-        }
-        cJ[b] = kj;
-        cImg[b] = km;
+    const uint2 me = tmp[p];
+    uint32_t k = s0;
+    for (uint32_t a = s0; a < s1; ++a) {
+        const uint32_t j = tmp[a].x;
+        k += j < me.x || (j == me.x && a < p);
     }
+    cJ[k] = (int32_t)me.x;
+    cImg[k] = me.y;
+    jtmp[jStart[me.x] + atomicAdd(&cur[me.x], 1u)] = k;
 }
 
-HipErr launch_order_I(hipStream_t st, int32_t n, uint32_t m, const uint32_t *pI,
-                      const uint32_t *pJ, const uint32_t *pImg, const uint32_t *rowStart,
-                      uint32_t *cur, int32_t *cI, int32_t *cJ, uint32_t *cImg, const uint32_t *md) {
+HipErr launch_order(hipStream_t st, uint32_t m, const uint32_t *pI, const uint32_t *pJ, const uint32_t *pImg,
+                    const uint32_t *rowStart, uint32_t *curI, const uint32_t *jStart, uint32_t *curJ, int32_t *cI,
+                    int32_t *cJ, uint32_t *cImg, void *tmp, const uint32_t *md) {
     if (m == 0) return hip_ok();
-    k_scatter_I<<<nblk(m, 256), 256, 0, st>>>(m, pI, pJ, pImg, rowStart, cur, cI, cJ, cImg, md);
+    uint2 *t = static_cast<uint2 *>(tmp);
+    k_scatter_I<<<nblk(m, blk(m)), blk(m), 0, st>>>(m, pI, pJ, pImg, rowStart, curI, cI, t, md);
     LAUNCH_CHECK();
-    k_sort_I<<<nblk(n, 256), 256, 0, st>>>(n, rowStart, cJ, cImg);
-    LAUNCH_CHECK();
-    return hip_ok();
-}
-
-__global__ void k_scatter_J(uint32_t m, const int32_t *__restrict__ cJ, const uint32_t *__restrict__ jStart,
-                            uint32_t *__restrict__ cur, uint32_t *__restrict__ jlist, const uint32_t *__restrict__ md) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= dcount(m, md)) return;
-    const uint32_t j = (uint32_t)cJ[k];
-    jlist[jStart[j] + atomicAdd(&cur[j], 1u)] = k;
-}
-
-__global__ void k_sort_J(int32_t n, const uint32_t *__restrict__ jStart, uint32_t *__restrict__ jlist) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t s0 = jStart[i], s1 = jStart[i + 1];
-    for (uint32_t a = s0 + 1; a < s1; ++a) {
-        const uint32_t v = jlist[a];
-        uint32_t b = a;
-        while (b > s0 && jlist[b - 1] > v) {
-            jlist[b] = jlist[b - 1];
-            --b;
-        }
-        jlist[b] = v;
-    }
-}
-
-HipErr launch_order_J(hipStream_t st, int32_t n, uint32_t m, const int32_t *cJ,
-                      const uint32_t *jStart, uint32_t *cur, uint32_t *jlist, const uint32_t *md) {
-    if (m == 0) return hip_ok();
-    k_scatter_J<<<nblk(m, 256), 256, 0, st>>>(m, cJ, jStart, cur, jlist, md);
-    LAUNCH_CHECK();
-    k_sort_J<<<nblk(n, 256), 256, 0, st>>>(n, jStart, jlist);
+    k_rank_I<<<nblk(m, blk(m)), blk(m), 0, st>>>(m, rowStart, t, cI, cJ, cImg, jStart, curJ, reinterpret_cast<uint32_t *>(t + m),
+                                                 md);
     LAUNCH_CHECK();
     return hip_ok();
 }
@@ -833,10 +844,14 @@ __global__ void k_rows(RodsDev r, CfgDev c, uint32_t m, uint32_t gs, const int32
                        const int32_t *__restrict__ cJ, const uint32_t *__restrict__ cImg,
                        const double *__restrict__ unc, double *__restrict__ delta0,
                        double *__restrict__ geo, double *__restrict__ posI,
-                       double *__restrict__ posJ, double *__restrict__ b, const uint32_t *__restrict__ md) {
+                       double *__restrict__ posJ, double *__restrict__ b, const uint32_t *__restrict__ jStart,
+                       const uint32_t *__restrict__ jtmp, uint32_t *__restrict__ jlist, const uint32_t *__restrict__ md) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= dcount(m, md)) return;
     const int32_t i = cI[k], j = cJ[k];
+    uint32_t at = jStart[j];  // the row's place in the list of rod J
+    for (uint32_t a = at, e = jStart[j + 1]; a < e; ++a) at += jtmp[a] < k;
+    jlist[at] = k;
     const uint32_t im = cImg[k];
     const SysDev &S = r.sys[r.rsys[i]];
     double cj[3];
@@ -875,9 +890,12 @@ __global__ void k_rows(RodsDev r, CfgDev c, uint32_t m, uint32_t gs, const int32
 
 HipErr launch_rows(hipStream_t st, const RodsDev &r, const CfgDev &c, uint32_t m, uint32_t gs, const int32_t *cI,
                    const int32_t *cJ, const uint32_t *cImg, const double *unc, double *delta0,
-                   double *geo, double *posI, double *posJ, double *b, const uint32_t *md) {
+                   double *geo, double *posI, double *posJ, double *b, const uint32_t *jStart, const void *tmp,
+                   uint32_t *jlist, const uint32_t *md) {
     if (m == 0) return hip_ok();
-    k_rows<<<nblk(m, 256), 256, 0, st>>>(r, c, m, gs, cI, cJ, cImg, unc, delta0, geo, posI, posJ, b, md);
+    const uint32_t *jtmp = reinterpret_cast<const uint32_t *>(static_cast<const uint2 *>(tmp) + m);
+    k_rows<<<nblk(m, blk(m)), blk(m), 0, st>>>(r, c, m, gs, cI, cJ, cImg, unc, delta0, geo, posI, posJ, b, jStart, jtmp, jlist,
+                                               md);
     LAUNCH_CHECK();
     return hip_ok();
 }
@@ -1163,7 +1181,7 @@ HipErr launch_slice_sizes(hipStream_t st, int32_t n, const uint32_t *rowStart, c
     static_assert(kSlice == 64, "one wave per slice");
     static_assert(kOrderWin % kSlice == 0 && kOrderWinPasses % kSlice == 0, "order windows hold whole slices");
     if (n == 0) return hip_ok();
-    k_slice_sizes<<<nblk(n, 256), 256, 0, st>>>(n, rowStart, jStart, extStart, slice_len, sord);
+    k_slice_sizes<<<nblk(n, blk(n)), blk(n), 0, st>>>(n, rowStart, jStart, extStart, slice_len, sord);
     LAUNCH_CHECK();
     return hip_ok();
 }
@@ -1226,7 +1244,7 @@ HipErr launch_adjacency(hipStream_t st, int32_t n, uint32_t m, const uint32_t *r
                         const uint32_t *jStart, const uint32_t *jlist, const uint32_t *extStart,
                         const uint32_t *extEnt, uint32_t mc, const double *geo, const uint32_t *sellStart,
                         uint64_t epad, uint32_t *adjStart, uint32_t *sellK, double *sellW, const uint32_t *spos) {
-    k_adjacency<<<nblk((int64_t)n + 1, 256), 256, 0, st>>>(n, m, rowStart, jStart, jlist, extStart, extEnt, mc, geo,
+    k_adjacency<<<nblk((int64_t)n + 1, blk(n)), blk(n), 0, st>>>(n, m, rowStart, jStart, jlist, extStart, extEnt, mc, geo,
                                                           sellStart, epad, adjStart, sellK, sellW, spos);
     LAUNCH_CHECK();
     return hip_ok();

@@ -1177,7 +1177,8 @@ HipErr launch_writeback(hipStream_t st, int32_t n, const int32_t *rsys, const Sy
                         double *gamma, uint32_t m, const uint32_t *md, const uint32_t *spos) {
     const int64_t t = n > (int64_t)m ? n : (int64_t)m;
     if (t > 0) {
-        k_writeback<<<nblk(t, 256), 256, 0, st>>>(n, rsys, sys, adjStart, sellStart, sellK, sellW, epad, xg, mob, unc, F, U,
+        const int b = t <= 65536 ? 64 : 256;  // small: items over more CUs
+        k_writeback<<<nblk(t, b), b, 0, st>>>(n, rsys, sys, adjStart, sellStart, sellK, sellW, epad, xg, mob, unc, F, U,
                                                   spos, gamma, m, md);
         LAUNCH_CHECK();
     }

@@ -354,12 +354,17 @@ constexpr int kBarTotalWords = (kBarTicket + 1) * kBarWords;
 // LDS of a block: adjacency slots take their six weights; another part holds the slots' values and, at other
 // times, the velocities of the rods the block's rows touch.
 constexpr uint32_t kResidentPool = 160512;
-// Adjacency slots a block holds with g row groups.  With one group (and in FP32 two) the velocities of all
-// 1,024 g rods its rows can name fit beside them; with more, 784 of 2,048 (FP32: 1,560 of 4,096), else the rows
-// read them from memory.
+// A block of the shared form with g row groups has 256 lanes a group, two rows a lane; with one group 512, a row a
+// lane: twice the waves hide each other's latencies (22.8k rows: 9.2 -> 8.1 us per iteration, 107k: 11.4 -> 10.6; with two groups the
+// 1,024 lanes' registers spill, 64 replicas 8.2 -> 17.8 ms, 183k rows in FP32 12.6 -> 16.6 us).  A group of 512 lanes
+// has 4 KB of the pool for half-folded partials.
+constexpr int resident_lanes(int g) { return g == 1 ? 512 : 256 * g; }
+constexpr uint32_t resident_pool(int g) { return kResidentPool - (g == 1 ? 4096u : 0u); }
+// Adjacency slots a block holds.  With one group (and in FP32 two) the velocities of all 1,024 g rods its rows can
+// name fit beside them; with more, 784 of 2,048 (FP32: 1,560 of 4,096), else the rows read them from memory.
 template <typename T>
 constexpr uint32_t resident_slots(int g) {
-    return sizeof(T) == 8 ? (g == 1 ? 2304 : 2560) : (g == 1 ? 3072 : (g == 2 ? 3584 : 4608));
+    return sizeof(T) == 8 ? (g == 1 ? 2208 : 2560) : (g == 1 ? 3072 : (g == 2 ? 3584 : 4608));
 }
 // most 256-lane row groups (chunks) per block: with more, the rows' registers no longer fit
 template <typename T>

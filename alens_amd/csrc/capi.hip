@@ -718,9 +718,9 @@ static int resident_gpb(double chunks, int32_t nsys, int blocks) {
 
 // The kernels for a step of `rows` rows and `slots` padded adjacency slots: resident where the operator fits
 // on the chip (the plan on the device has the last word; it fills a block's slots to 15/16), else general.  The
-// resident kernel is the faster one wherever it fits: per iteration 9.2 us against 13.7 at 800 rows, 11.4 against
-// 29 at 107k, in FP32 22.9 against 31 at 472k, near the largest it holds; a batch's systems, which then stop and
-// start one by one, 8.2 ms against 10.8 for 64 systems of 1.37M rows.
+// resident kernel is the faster one wherever it fits: per iteration 8.1 us against 29 at 22.8k rows, 10.6 against 29
+// at 107k, in FP32 22.9 against 31 at 472k, near the largest it holds; a batch's systems, which then stop and
+// start one by one, 8.1 ms against 10.8 for 64 systems of 1.37M rows.
 static alens_ctx::Route want_route(const alens_ctx *ctx, double rows, double slots) {
     alens_ctx::Route r;
     r.stream_nt[0] = general_iter_bytes(8, rows, ctx->n) > kLastLevelCacheBytes;

@@ -14,8 +14,8 @@
 //   phase A   v = P(x - alpha g) of every slot; then one lane per rod adds v_j w_j in the slots' order,
 //             U = M F, and stores U.
 //   phase B   the block polls the velocities of the rods its rows touch into LDS, each rod once; then one
-//             lane per two rows: new (x, g), residual and products, stored (x, g); the 256-lane group of
-//             a chunk folds its partials in the fixed order and stores them.
+//             lane per two rows: new (x, g), residual and products, stored (x, g); the lanes of
+//             a chunk fold its partials in the fixed order and stores them.
 //   fold      256 lanes poll the partials of the system's chunks and fold them in the fixed order, while the
 //             next gather is under way.  When they are all there, every block of the system has finished
 //             phase B.
@@ -31,8 +31,8 @@
 // the number of instructions.  So words travel 16 B at a time; velocities are held by slice position (a share's
 // are consecutive) and fetched once per block; strides of the LDS are constants; what only the start needs stays
 // out of the loop's registers.  Microseconds per iteration, general kernel -> here (slab and box systems in their
-// sorted order, FP64 unless noted): 800 rows 13.7 -> 9.2, 22.8k 29 -> 9.2, 107k 29 -> 11.4, 183k in FP32 33 -> 12.6,
-// 472k in FP32 31 -> 22.9; 64 systems of 1.37M rows together (each waits only for itself) 10.8 -> 8.2 ms.
+// sorted order, FP64 unless noted): 22.8k rows 29 -> 8.1, 107k 29 -> 10.6, 183k in FP32 33 -> 12.6, 472k in FP32
+// 31 -> 22.9; 64 systems of 1.37M rows together (each waits only for itself) 10.8 -> 8.1 ms.
 //
 // Systems do not meet each other at all: a block belongs to one system at a time, takes (system, share)
 // pairs from a counter in order, and so the blocks of the first unfinished system are always running.
@@ -375,16 +375,15 @@ __device__ inline void swap_rows16(double &a, double &b) {
     a = __hiloint2double((int)hi[0], (int)lo[0]);
     b = __hiloint2double((int)hi[1], (int)lo[1]);
 }
-__device__ inline double wave_fold4(const double (&v)[4], bool sum2) {
+__device__ inline double2 fold_passes(const double (&v)[4], bool sum2) {
     double a = v[0], b = v[1], c = v[2], d = v[3];
     swap_halves32(a, b);
-    a = a + b;
     swap_halves32(c, d);
+    const double s = c + d, m = d > c ? d : c;
+    return make_double2(a + b, sum2 && (threadIdx.x & 63) < 32 ? s : m);
+}
+__device__ inline double fold_rows(double a, double c, bool sum2) {
     const int l = threadIdx.x & 63;
-    {
-        const double s = c + d, m = d > c ? d : c;
-        c = sum2 && l < 32 ? s : m;
-    }
     swap_rows16(a, c);  // rows: v0, v2, v1, v3
     const bool sum = (l >> 4) == 0 || (l >> 4) == 2 || (sum2 && (l >> 4) == 1);
     auto step = [&](double x, double o) {
@@ -396,6 +395,15 @@ __device__ inline double wave_fold4(const double (&v)[4], bool sum2) {
     x = step(x, lanes_up_row<4>(x));
     x = step(x, lanes_up_row<2>(x));
     return step(x, lanes_up_row<1>(x));
+}
+__device__ inline double wave_fold4(const double (&v)[4], bool sum2) {
+    const double2 h = fold_passes(v, sum2);
+    return fold_rows(h.x, h.y, sum2);
+}
+// The same where a wave holds 32 virtual lanes in two passes (fold_passes folds those) and o has the 32 that follow.
+__device__ inline double fold_rest(double2 h, double2 o, bool sum2) {
+    const double s = h.y + o.y, m = o.y > h.y ? o.y : h.y;
+    return fold_rows(h.x + o.x, sum2 && (threadIdx.x & 63) < 32 ? s : m, sum2);
 }
 // where lane 16 r of wave_fold4 holds its result: quantity 0, 2, 1, 3
 __device__ inline int fold4_quantity(int r) { return r == 1 ? 2 : (r == 2 ? 1 : r); }
@@ -416,9 +424,10 @@ __device__ inline void report(const SolveArgsT<T> &a, int sy, int iters, int mv,
 
 // EXT: the rows include caller rows (lower bounds and compliances other than 0).
 template <typename T, int GPB, bool EXT>
-__global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r) {
+__global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(ResidentArgs<T> r) {
     using F = Form<T>;
-    constexpr int NT = 256 * GPB, NU = F::u16, W = (int)sizeof(T);
+    constexpr int NT = resident_lanes(GPB), NU = F::u16, W = (int)sizeof(T);
+    constexpr int LPC = NT / GPB, RPL = kRedChunk / LPC;  // lanes of a chunk, rows of a lane
     constexpr uint32_t kNone = 0xffffffffu;
     constexpr int NKEY = 1024 * GPB;  // rods named by the block's rows, with repeats
     // LDS: slot weights by component, then a part that holds the slots' values in phase A and the touched rods'
@@ -426,17 +435,21 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
     constexpr uint32_t SC = resident_slots<T>(GPB);
     constexpr int GW = (int)((SC + NT - 1) / NT);             // slots of a lane
     constexpr uint32_t oV = 6 * SC * W, B2 = 65536u;          // value part; second base of the immediate offsets
-    constexpr uint32_t UC = (kResidentPool - oV) / (16 * NU);  // velocities it holds
+    constexpr uint32_t UC = (resident_pool(GPB) - oV) / (16 * NU);  // velocities it holds
     constexpr int NB = (int)((UC * NU < 1024u * GPB * NU ? UC * NU : 1024u * GPB * NU) + NT - 1) / NT;  // words of a lane
-    static_assert(oV + GW * NT * W <= kResidentPool && oV >= 4 * W * SC && oV < 2 * B2, "LDS layout");
+    static_assert(oV + GW * NT * W <= resident_pool(GPB) && oV >= 4 * W * SC && oV < 2 * B2, "LDS layout");
     const SolveArgsT<T> &a = r.s;
-    __shared__ __align__(16) unsigned char pool[kResidentPool];
+    __shared__ __align__(16) unsigned char pool[resident_pool(GPB)];
     __shared__ double shG[GPB * 4 * 4], shF[4 * 4];
+    __shared__ double2 shH[RPL == 1 ? GPB * 4 * 64 : 1];  // the odd waves' half-folded partials
     __shared__ uint32_t s_cnt[NT / 64];
     __shared__ int s_abort;
     __shared__ uint32_t s_ticket;
     if (r.head[0] != kPlanShared) return;  // a share does not fit: the host redoes the step
-    const int tid = threadIdx.x, grp = tid >> 8, gl = tid & 255, lane = tid & 63, wv = (tid >> 6) & 3;
+    // A chunk's 256 virtual lanes of two passes: with two rows a lane they are the lanes; with one, a wave has 32 of
+    // them, pass 0 in its lower half, pass 1 in its upper one.
+    const int tid = threadIdx.x, grp = tid / LPC, gl = tid % LPC, lane = tid & 63, wv = gl >> 6;
+    const int first_row = RPL == 1 ? 32 * wv + (lane & 31) + (lane >> 5) * kRedThreads : gl;
     const uint32_t total = (uint32_t)r.head[1];
     const Regions rg = regions<T>(a.m, a.n, a.nchunks);
     const Exch ex(r.ex, rg.bytes());
@@ -463,12 +476,12 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
         const bool act = ch < ce;
         const uint32_t kb = a.con_off[sy] + ch * kRedChunk, kend = a.con_off[sy + 1];
         uint32_t *keys = reinterpret_cast<uint32_t *>(pool), *sP = keys + NKEY;
-        uint32_t kk[2], pIJ[2][2];
-        bool ok[2];
-        T gk[2][9], bb[2], xo[2], go[2], lbk[2], ivk[2];
+        uint32_t kk[RPL], pIJ[RPL][2];
+        bool ok[RPL];
+        T gk[RPL][9], bb[RPL], xo[RPL], go[RPL], lbk[RPL], ivk[RPL];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            kk[q] = kb + (uint32_t)(gl + q * kRedThreads);
+        for (int q = 0; q < RPL; ++q) {
+            kk[q] = kb + (uint32_t)(first_row + q * kRedThreads);
             ok[q] = act && kk[q] < kend;
             pIJ[q][0] = pIJ[q][1] = kNone;
             lbk[q] = ivk[q] = T(0);
@@ -487,17 +500,18 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
                 xo[q] = xg.x;
                 go[q] = xg.y;
             }
-            keys[4 * tid + 2 * q] = pIJ[q][0];
-            keys[4 * tid + 2 * q + 1] = pIJ[q][1];
+            keys[2 * RPL * tid + 2 * q] = pIJ[q][0];
+            keys[2 * RPL * tid + 2 * q + 1] = pIJ[q][1];
         }
         sort_keys<NKEY, NT>(keys);
         uint32_t un = 0;  // distinct rods
         {
-            uint32_t v[4], cnt = 0;
-            bool first[4];
+            constexpr int KPL = 2 * RPL;
+            uint32_t v[KPL], cnt = 0;
+            bool first[KPL];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int i = 4 * tid + q;
+            for (int q = 0; q < KPL; ++q) {
+                const int i = KPL * tid + q;
                 v[q] = keys[i];
                 first[q] = v[q] != kNone && (i == 0 || keys[i - 1] != v[q]);
                 cnt += first[q];
@@ -517,7 +531,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
                 un += s_cnt[w];
             }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < KPL; ++q)
                 if (first[q]) sP[at++] = v[q];
             __syncthreads();
         }
@@ -533,7 +547,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
             uat[z] = cached && un > 0 ? (sP[q / NU] * NU + q % NU) * 16u : 0u;
         }
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < RPL; ++q) {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 uint32_t at = ok[q] ? pIJ[q][e] : 0u;
@@ -602,7 +616,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
             if (EXT) lbs[q] = K < a.m ? a.lb[K] : T(0);
         }
         // a lane's first rods stay in registers, with their mobility (as many as leave the loop without spills)
-        constexpr int NR = GPB == 1 ? 3 : (W == 4 && GPB == 2 ? 2 : 1);
+        constexpr int NR = W == 4 && GPB <= 2 ? 2 : 1;
         Rod rods[NR];
         T rmob[NR][6];
 #pragma unroll
@@ -652,7 +666,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
             for (uint32_t q = t; q < (p1 - p0) * NU; q += NT) ex.unset16((p0 * NU + q) * 16u, rg.U(ue + 1));
             if (dst < 3) {
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
+                for (int q = 0; q < RPL; ++q) {
                     uint32_t kx = kk[q];
                     asm volatile("" : "+v"(kx));
                     if (ok[q]) F::unset(ex, kx * F::xg, rg.X(dst == 2 ? 0 : dst + 1));
@@ -769,7 +783,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
             stores_done();  // the resets of this exchange (their acknowledgement is long back)
             double vs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, vx[2] = {0.0, 0.0};
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+            for (int q = 0; q < RPL; ++q) {
                 if (!ok[q]) continue;
                 uint32_t pI = pIJ[q][0], pJ = pIJ[q][1], kx = kk[q];
                 T bq = bb[q];
@@ -853,8 +867,21 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
                 v[3] = mode == B_INIT ? vx[1] : 0.0;
             }
             double *sg = shG + grp * 4 * 4;
-            const double x = wave_fold4(v, mode != B_INIT);
-            if ((lane & 15) == 0) sg[fold4_quantity(lane >> 4) * 4 + wv] = x;
+            const bool sum2 = mode != B_INIT;
+            if constexpr (RPL == 2) {
+                const double x = wave_fold4(v, sum2);
+                if ((lane & 15) == 0) sg[fold4_quantity(lane >> 4) * 4 + wv] = x;
+            } else {
+                // passes, then the other wave's 32 virtual lanes, then within the wave
+                double2 h = fold_passes(v, sum2);
+                double2 *sh = shH + (grp * 4 + (wv >> 1)) * 64;
+                if (wv & 1) sh[lane] = h;
+                lds_sync();
+                if ((wv & 1) == 0) {
+                    const double x = fold_rest(h, sh[lane], sum2);
+                    if ((lane & 15) == 0) sg[fold4_quantity(lane >> 4) * 4 + (wv >> 1)] = x;
+                }
+            }
             lds_sync();
             const bool good = s_abort == 0;
             if (act && gl == 0 && good) {
@@ -943,7 +970,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
                         ex.unset16(rec + 16u, rg.P(pe == 2 ? 0 : pe + 1));
                     }
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) {
+                    for (int q = 0; q < RPL; ++q) {
                         if (!ok[q]) continue;
                         xo[q] = T(0);
                         go[q] = T(0) + bb[q];
@@ -981,7 +1008,7 @@ __global__ __launch_bounds__(256 * GPB) void k_bbpgd_resident(ResidentArgs<T> r)
             }
         }
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < RPL; ++q)
             if (ok[q]) a.xg[kk[q]] = mk2<T>(xo[q], go[q]);
         if (ib == 0 && tid == 0) report(a, sy, iters, mv, state, fb, res0, res);
         __syncthreads();
@@ -1244,7 +1271,7 @@ template <typename T, int GPB>
 static HipErr launch_resident_k(hipStream_t st, ResidentArgs<T> r, int grid) {
     void *args[] = {&r};
     const void *f = r.s.lb ? (const void *)k_bbpgd_resident<T, GPB, true> : (const void *)k_bbpgd_resident<T, GPB, false>;
-    ALENS_HIP_TRY(hipLaunchCooperativeKernel(f, dim3(grid), dim3(256 * GPB), args, 0, st));
+    ALENS_HIP_TRY(hipLaunchCooperativeKernel(f, dim3(grid), dim3(resident_lanes(GPB)), args, 0, st));
     return hip_ok();
 }
 

@@ -82,6 +82,8 @@ struct alens_ctx {
     DBuf<float2> xg32;
     // learned warm start: FP32 master parameters, normalisation, features of the step
     DBuf<float> mlpP, mlpNorm, feat;
+    DBuf<float> mlpX, mlpT, mlpPart, mlpG, mlpM1, mlpM2, mlpL;  // working memory of predict, gradient and train
+    DBuf<int32_t> mlpIdx;
     bool mlp_ready = false;
     DBuf<float> adam1, adam2;                // Adam moments of energy training (reset by alens_mlp_set)
     int adam_step = 0;
@@ -297,7 +299,8 @@ void alens_destroy(alens_ctx *ctx) {
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
     rel(ctx->extStart); rel(ctx->ext); rel(ctx->extNrm); rel(ctx->lb); rel(ctx->invk);
     rel(ctx->lb32); rel(ctx->invk32); rel(ctx->geo32); rel(ctx->sellW32); rel(ctx->mob32); rel(ctx->b32); rel(ctx->U32); rel(ctx->xg32);
-    rel(ctx->mlpP); rel(ctx->mlpNorm); rel(ctx->feat); rel(ctx->xprev);
+    rel(ctx->mlpP); rel(ctx->mlpNorm); rel(ctx->feat); rel(ctx->mlpX); rel(ctx->mlpT); rel(ctx->mlpPart); rel(ctx->mlpG);
+    rel(ctx->mlpM1); rel(ctx->mlpM2); rel(ctx->mlpL); rel(ctx->mlpIdx); rel(ctx->xprev);
     rel(ctx->sysd); rel(ctx->rsys); rel(ctx->smono); rel(ctx->chunk_sys); rel(ctx->con_off); rel(ctx->chunk_off);
     if (ctx->stress_host) (void)hipHostFree(ctx->stress_host);
     for (auto &e : ctx->ev)
@@ -2295,20 +2298,28 @@ alens_status alens_get_features(alens_ctx *ctx, float *X) {
     return ALENS_OK;
 }
 
+// The network calls keep their working memory for the next call, unless it is large: making and freeing it took
+// 50 us of a prediction of 250,000 rows (739 -> 690 us) and 110 us of an epoch over 120,000 (1,350 -> 1,243 us).
+static void trim_mlp(alens_ctx *ctx) {
+    constexpr size_t kKeep = (size_t)64 << 20;  // words
+    for (auto *b : {&ctx->mlpX, &ctx->mlpT, &ctx->mlpL})
+        if (b->cap > kKeep) b->release();
+    if (ctx->mlpIdx.cap > kKeep) ctx->mlpIdx.release();
+}
+
 alens_status alens_mlp_predict(alens_ctx *ctx, int64_t m, const float *X, float *gamma0) {
     if (!ctx || m < 0 || m > 0x7fffffff || (m > 0 && (!X || !gamma0))) return ALENS_E_ARG;
     if (!ctx->mlp_ready) return fail(ctx, ALENS_E_STATE, "no network parameters");
     if (m == 0) return ALENS_OK;
     TRY_HIP(hipSetDevice(ctx->dev));
-    DBuf<float> dX, dY;
+    DBuf<float> &dX = ctx->mlpX, &dY = ctx->mlpT;
     TRY_HIP(dX.ensure(16 * (size_t)m));
     TRY_HIP(dY.ensure((size_t)m));
     TRY_HIP(hipMemcpyAsync(dX.p, X, sizeof(float) * 16 * m, hipMemcpyHostToDevice, ctx->st));
     TRY_K(launch_mlp_infer_f32(ctx->st, (uint32_t)m, dX.p, ctx->mlpP.p, ctx->mlpNorm.p, dY.p));
     TRY_HIP(hipMemcpyAsync(gamma0, dY.p, sizeof(float) * m, hipMemcpyDeviceToHost, ctx->st));
     TRY_HIP(hipStreamSynchronize(ctx->st));
-    dX.release();
-    dY.release();
+    trim_mlp(ctx);
     return ALENS_OK;
 }
 
@@ -2317,7 +2328,7 @@ alens_status alens_mlp_gradient(alens_ctx *ctx, int64_t m, const float *X, const
     if (!ctx || m <= 0 || m % 16 || m > (1 << 26) || !X || !target || !grad) return ALENS_E_ARG;
     if (!ctx->mlp_ready) return fail(ctx, ALENS_E_STATE, "no network parameters");
     TRY_HIP(hipSetDevice(ctx->dev));
-    DBuf<float> dX, dT, dG, part;
+    DBuf<float> &dX = ctx->mlpX, &dT = ctx->mlpT, &dG = ctx->mlpG, &part = ctx->mlpPart;
     TRY_HIP(part.ensure(kMlpGradFloats));
     TRY_HIP(dX.ensure(16 * (size_t)m));
     TRY_HIP(dT.ensure((size_t)m));
@@ -2330,10 +2341,7 @@ alens_status alens_mlp_gradient(alens_ctx *ctx, int64_t m, const float *X, const
     TRY_HIP(hipMemcpyAsync(&l, dG.p + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, ctx->st));
     TRY_HIP(hipStreamSynchronize(ctx->st));
     if (loss) *loss = l;
-    part.release();
-    dX.release();
-    dT.release();
-    dG.release();
+    trim_mlp(ctx);
     return ALENS_OK;
 }
 
@@ -2391,8 +2399,8 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
     const float gs = norm[2 * kMlpIn];
     std::vector<float> t(m);
     for (int64_t i = 0; i < m; ++i) t[i] = gamma[i] / gs;
-    DBuf<float> dX, dT, part, dM1, dM2, dL;
-    DBuf<int32_t> dIdx;
+    DBuf<float> &dX = ctx->mlpX, &dT = ctx->mlpT, &part = ctx->mlpPart, &dM1 = ctx->mlpM1, &dM2 = ctx->mlpM2, &dL = ctx->mlpL;
+    DBuf<int32_t> &dIdx = ctx->mlpIdx;
     const int64_t nb = m / batch;
     TRY_HIP(part.ensure(kMlpGradFloats));
     TRY_HIP(dX.ensure(16 * (size_t)m));
@@ -2429,8 +2437,7 @@ alens_status alens_mlp_train(alens_ctx *ctx, int64_t m, const float *X, const fl
         for (int64_t b = 0; b < nb; ++b) acc += lh[b];
         if (loss_per_epoch) loss_per_epoch[ep] = (float)(acc / std::max<int64_t>(nb, 1));
     }
-    for (auto *b : {&dX, &dT, &part, &dM1, &dM2, &dL}) b->release();
-    dIdx.release();
+    trim_mlp(ctx);
     return ALENS_OK;
 }
 

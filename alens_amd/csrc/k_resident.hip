@@ -161,9 +161,9 @@ struct Form<float> {
 };
 
 // one more poll of a wait; false gives up (this wait was too long, or another block has set the abort word)
-__device__ inline bool spin_more(uint32_t &n, uint32_t *bar) {
+__device__ inline bool spin_more(uint32_t &n, uint32_t limit, uint32_t *bar) {
     reload();
-    if (++n > kResSpin) {
+    if (++n > limit) {
         __hip_atomic_store(&bar[kBarWords], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
     }
@@ -629,6 +629,9 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
         __syncthreads();
         __builtin_amdgcn_s_waitcnt(0);  // the share is loaded: nothing in the loop waits for it again
 
+        // where shares wait for blocks, the system's others may start only when earlier systems are done, however
+        // long those take; once its first exchange is complete all of them run
+        uint32_t limit = total > gridDim.x ? ~0u : kResSpin;
         const T dt = (T)a.dt;
         double alpha = 0.0;
         int odd = 0;              // parity of the iteration
@@ -684,7 +687,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                 for (int q = 0; q < GW; ++q)
                     if (q < nq) seen = F::seen(seen, wg[q]);
                 if (seen != 0u) break;
-                if (!spin_more(spins, a.bar)) {
+                if (!spin_more(spins, limit, a.bar)) {
                     s_abort = 1;
                     break;
                 }
@@ -764,7 +767,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                         for (int z = 0; z < NB; ++z)
                             if (z < nz) seen = F::seen_u(seen, w[z]);
                         if (seen != 0u) break;
-                        if (!spin_more(spins, a.bar)) {
+                        if (!spin_more(spins, limit, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -807,7 +810,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
 #pragma unroll
                         for (int c = 0; c < NU; ++c) seen = F::seen_u(F::seen_u(seen, wI[c]), wJ[c]);
                         if (seen != 0u) break;
-                        if (!spin_more(spins, a.bar)) {
+                        if (!spin_more(spins, limit, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -905,7 +908,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                     u32x4 w0 = ex.ld16(at, pr), w1 = ex.ld16(at + 16u, pr);
                     uint32_t spins = 0;
                     while (seen64(seen64(1u, w0), w1) == 0u) {
-                        if (!spin_more(spins, a.bar)) {
+                        if (!spin_more(spins, limit, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -948,6 +951,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
             }
             gather(rg.X(xs));
             if (!fold(it < 0 ? 2 : 3, tot)) return;
+            limit = kResSpin;
             ++ue;
             pe = pe == 2 ? 0 : pe + 1;
             ++mv;

@@ -201,7 +201,9 @@ alens_status alens_get_velocity(alens_ctx *ctx, double *u, double *u_nc, double 
  * Results are bit-identical under every schedule; only the time changes.  Needs a step with
  * constraints; leaves that step's outputs untouched.  Environment variables ALENS_SOLVER_ENTRIES,
  * ALENS_BARRIER_MODE, ALENS_XCD_MAP, ALENS_SOLVER_MAX_BLOCKS, ALENS_GROUP_WIDTH and ALENS_STREAM_HINT
- * override the choice outside tuning. */
+ * override the choice outside tuning.  The schedule is that of the kernel that streams its operator from
+ * memory.  A solve whose operator fits on the chip runs another kernel, to the same bits, which has no
+ * schedule to tune; naming a schedule in the environment selects the streaming kernel for every solve. */
 typedef struct {
     int32_t entries;     /* 0 = largest instantiated (3 in FP64, 4 in FP32), or 2 */
     int32_t bar_mode;    /* 0 flat, 1 grouped, 2 grouped with longer polls, 3 grouped by XCC with one

@@ -13,9 +13,9 @@
 //   gather    every slot of the block polls (x, g) of its row, all slots at once.
 //   phase A   v = P(x - alpha g) of every slot; then one lane per rod adds v_j w_j in the slots' order,
 //             U = M F, and stores U.
-//   phase B   the block polls the velocities of the rods its rows touch into LDS, each rod once; then one
-//             lane per two rows: new (x, g), residual and products, stored (x, g); the lanes of
-//             a chunk fold its partials in the fixed order and stores them.
+//   phase B   the block polls the velocities of the rods its rows touch into LDS, each rod once; then a lane per
+//             row or two: new (x, g), residual and products, stored (x, g); the lanes of a chunk fold its
+//             partials in the fixed order and store them.
 //   fold      256 lanes poll the partials of the system's chunks and fold them in the fixed order, while the
 //             next gather is under way.  When they are all there, every block of the system has finished
 //             phase B.

@@ -1481,6 +1481,7 @@ static alens_status enqueue_resident(alens_ctx *ctx, bool fx, bool warm_prev) {
     }
     // start point and solve (the solver reads the row and chunk counts from the device)
     TRY_K(launch_stamp(st, ctx->stamps.p, 1));
+    ctx->mext = 0;  // (the step before may have had caller rows: their bounds and compliances are not this one's)
     ctx->gstride = c.M;
     ctx->epad = c.epad;
     ctx->nchunks_cur = c.nch;

@@ -1642,7 +1642,12 @@ alens_status alens_step_constraints(alens_ctx *ctx, const double *f_ext, alens_s
     if (!ctx) return ALENS_E_ARG;
     if (!ctx->have_rods) return fail(ctx, ALENS_E_STATE, "step_constraints before set_rods");
     TRY_HIP(hipSetDevice(ctx->dev));
-    if (!ctx->graph_mode || !ctx->ext_pending.empty()) return step_plain(ctx, f_ext, rep_out);
+    if (!ctx->graph_mode || !ctx->ext_pending.empty()) {
+        // an exact-size step describes itself in the context (row stride, padded slots, route) and may reallocate
+        // buffers that a captured step writes: the next step without caller rows captures again
+        drop_graph(ctx);
+        return step_plain(ctx, f_ext, rep_out);
+    }
     if (f_ext && !finite_all(f_ext, 6 * (size_t)ctx->n)) return fail(ctx, ALENS_E_NONFINITE, "non-finite f_ext");
     const bool fx = f_ext != nullptr;
     const bool warm_prev = ctx->cfg.warm_start >= 1 && ctx->have_prev;

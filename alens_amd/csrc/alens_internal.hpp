@@ -371,9 +371,9 @@ template <typename T>
 constexpr int resident_groups() {
     return sizeof(T) == 8 ? 2 : 4;
 }
-// A plan on the device: words 0..3 = {how the FP64 solve runs, its shares, the step's padded slots,
-// its chunks}, words 4..7 = {how the FP32 solve runs, its shares, wanted plans that do not fit (1: FP64, 2:
-// FP32), chunks}, then both solves' shares.
+// A plan on the device: for the FP64 and for the FP32 solve a head {how it runs, its shares, 2, 3, row groups of a
+// block, most shares of one system}, with 2 and 3 {the step's padded slots, its chunks} in the first, {wanted plans
+// that do not fit (1: FP64, 2: FP32), chunks} in the second; then both solves' shares.
 struct ShareCut {
     uint32_t sys, index, of;  // share `index` of the system's `of`
     uint32_t p0, p1;          // its slice positions
@@ -381,9 +381,9 @@ struct ShareCut {
     uint32_t pad;
 };
 constexpr int kPlanShares = 1 << 14;
-constexpr int kPlanHead = 4, kPlanUnfit = kPlanHead + 2;
+constexpr int kPlanHead = 8, kPlanUnfit = kPlanHead + 2;
 constexpr size_t kPlanWords = 2 * kPlanHead + 2 * (size_t)kPlanShares * (sizeof(ShareCut) / 4);
-// words 0 and 4: how the solve runs
+// how a solve runs
 enum { kPlanUnfitting = 0, kPlanShared = 1, kPlanAlone = 2 };
 // An FP64 solve of one system that one block holds whole (k_bbpgd_alone): at most kAloneRows rows, and LDS for the
 // slots' weights and rows, the rods' velocities and the rows' values.
@@ -411,7 +411,7 @@ struct ResidentArgs {
     SolveArgsT<T> s;
     void *ex;                   // exchange memory, resident_exchange_bytes(m, n, nchunks)
     const uint32_t *spos;       // slice position of each rod, NULL = identity
-    const int32_t *head;        // the plan's head and shares for this solve
+    int32_t *head;              // the plan's head and shares for this solve
     const ShareCut *share;
 };
 // bytes of exchange memory (at most 4 GiB - 1) of a solve of m rows, n rods and nchunks chunks

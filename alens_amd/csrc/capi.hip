@@ -691,7 +691,7 @@ struct SolveMem {
     uint32_t *bar;
     const uint32_t *con_off, *chunk_off;
     const int32_t *chunk_sys;
-    const int32_t *plan;  // the rows' resident plan, or NULL: the general kernel
+    int32_t *plan;        // the rows' resident plan, or NULL: the general kernel
 };
 
 // An explicit schedule in the environment names the general kernel, whose schedule it is.

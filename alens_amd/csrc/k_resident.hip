@@ -160,14 +160,18 @@ struct Form<float> {
     }
 };
 
-// one more poll of a wait; false gives up (this wait was too long, or another block has set the abort word)
-__device__ inline bool spin_more(uint32_t &n, uint32_t limit, uint32_t *bar) {
+// One more poll of a wait; false gives up (this wait was too long, or another block has set the abort word).  need: 0,
+// or the ticket count at which every share of the system has a block.  Until then the wait is not counted: a share
+// without a block waits for systems before its own, and those end by themselves (tickets are taken in order, so all
+// their shares have blocks, whose waits are counted).
+__device__ inline bool spin_more(uint32_t &n, uint32_t need, uint32_t *bar) {
     reload();
-    if (++n > limit) {
-        __hip_atomic_store(&bar[kBarWords], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return false;
-    }
-    return (n & 255u) != 0 || __hip_atomic_load(&bar[kBarWords], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
+    if ((++n & 255u) != 0) return true;
+    if (__hip_atomic_load(&bar[kBarWords], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return false;
+    if (need != 0u && __hip_atomic_load(&bar[kBarTicket * kBarWords], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) n = 0;
+    if (n < kResSpin) return true;
+    __hip_atomic_store(&bar[kBarWords], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
 }
 
 // Slots before slice position p: whole slices, then p % 64 columns of its slice's depth.
@@ -200,6 +204,7 @@ __device__ inline uint32_t share_cut(const uint32_t *sellStart, uint32_t r0, uin
 __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
     __shared__ uint32_t s_off[kMaxSys + 1];
     __shared__ int s_bad;
+    __shared__ uint32_t s_most;
     const int t = threadIdx.x;
     int unfit = 0;
     for (int f = 0; f < 2; ++f) {
@@ -217,12 +222,16 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
                     head[1] = 1;
                     head[2] = (int32_t)a.sellStart[a.nslices];
                     head[3] = *a.nchunks;
+                    head[4] = head[5] = 1;
                 }
                 continue;
             }
         }
         uint32_t nb = 0;
-        if (t == 0) s_bad = gpb == 0 || (f == 0 && a.alone == kAloneOnly);
+        if (t == 0) {
+            s_bad = gpb == 0 || (f == 0 && a.alone == kAloneOnly);
+            s_most = 1;
+        }
         __syncthreads();
         if (t < a.nsys && gpb > 0 && !s_bad) {
             const uint32_t nch = a.chunk_off[t + 1] - a.chunk_off[t];
@@ -234,6 +243,7 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
             nb = nb < nch ? nb : nch;  // every share holds a chunk (its partials announce the share's writes)
             nb = nb > 0 ? nb : 1;
             if (nb > a.max_shares[f]) s_bad = 1;
+            atomicMax(&s_most, nb);
         }
         s_off[t + 1] = nb;
         if (t == 0) s_off[0] = 0;
@@ -270,6 +280,8 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
             head[1] = (int32_t)total;
             head[2] = f == 0 ? (int32_t)a.sellStart[a.nslices] : unfit;
             head[3] = *a.nchunks;
+            head[4] = (int32_t)gpb;
+            head[5] = (int32_t)s_most;
         }
         __syncthreads();
     }
@@ -311,10 +323,13 @@ template size_t resident_exchange_bytes<double>(double, double, double);
 template size_t resident_exchange_bytes<float>(double, double, double);
 
 // The exchange memory before a solve: the start point in the third (x, g) buffer, (0, 0) in the spare rows,
-// everything else unset; barrier words (the ticket among them) zero.
+// everything else unset; barrier words (the ticket among them) zero.  A plan is for launches with its number of row
+// groups and with a block for every share of a system at least: with another one (two groups' chunks on one, a share
+// that no block will take) the solve would leave rows out or wait for ever.  Such a plan is refused, with the abort word.
 template <typename T>
 __global__ void k_resident_reset(unsigned char *__restrict__ ex, Regions g, const typename Vec2<T>::type *__restrict__ xg,
-                                 uint32_t m, const uint32_t *__restrict__ md, uint32_t *__restrict__ bar, int keep_abort) {
+                                 uint32_t m, const uint32_t *__restrict__ md, uint32_t *__restrict__ bar, int keep_abort,
+                                 int32_t *__restrict__ head, int gpb, uint32_t grid) {
     using V2 = typename Vec2<T>::type;
     constexpr uint32_t xw = Form<T>::xg / 8;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -328,6 +343,10 @@ __global__ void k_resident_reset(unsigned char *__restrict__ ex, Regions g, cons
     }
     if (i < 3) reinterpret_cast<V2 *>(ex + g.X(i))[m] = mk2<T>(T(0), T(0));
     if (i < (uint32_t)kBarTotalWords && !(keep_abort && i == (uint32_t)kBarWords)) bar[i] = 0u;
+    if (i == (uint32_t)kBarWords && head[0] != kPlanUnfitting && (head[0] != kPlanShared || head[4] != gpb || (uint32_t)head[5] > grid)) {
+        head[0] = kPlanUnfitting;
+        bar[i] = 1u;
+    }
 }
 
 // Ascending bitonic sort of N keys in LDS by NT threads.
@@ -445,7 +464,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
     __shared__ uint32_t s_cnt[NT / 64];
     __shared__ int s_abort;
     __shared__ uint32_t s_ticket;
-    if (r.head[0] != kPlanShared) return;  // a share does not fit: the host redoes the step
+    if (r.head[0] != kPlanShared) return;  // a share does not fit (the host redoes the step), or the plan was refused
     // A chunk's 256 virtual lanes of two passes: with two rows a lane they are the lanes; with one, a wave has 32 of
     // them, pass 0 in its lower half, pass 1 in its upper one.
     const int tid = threadIdx.x, grp = tid / LPC, gl = tid % LPC, lane = tid & 63, wv = gl >> 6;
@@ -631,7 +650,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
 
         // where shares wait for blocks, the system's others may start only when earlier systems are done, however
         // long those take; once its first exchange is complete all of them run
-        uint32_t limit = total > gridDim.x ? ~0u : kResSpin;
+        uint32_t need = total > gridDim.x ? share - ib + nb : 0u;
         const T dt = (T)a.dt;
         double alpha = 0.0;
         int odd = 0;              // parity of the iteration
@@ -687,7 +706,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                 for (int q = 0; q < GW; ++q)
                     if (q < nq) seen = F::seen(seen, wg[q]);
                 if (seen != 0u) break;
-                if (!spin_more(spins, limit, a.bar)) {
+                if (!spin_more(spins, need, a.bar)) {
                     s_abort = 1;
                     break;
                 }
@@ -767,7 +786,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                         for (int z = 0; z < NB; ++z)
                             if (z < nz) seen = F::seen_u(seen, w[z]);
                         if (seen != 0u) break;
-                        if (!spin_more(spins, limit, a.bar)) {
+                        if (!spin_more(spins, need, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -810,7 +829,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
 #pragma unroll
                         for (int c = 0; c < NU; ++c) seen = F::seen_u(F::seen_u(seen, wI[c]), wJ[c]);
                         if (seen != 0u) break;
-                        if (!spin_more(spins, limit, a.bar)) {
+                        if (!spin_more(spins, need, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -908,7 +927,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
                     u32x4 w0 = ex.ld16(at, pr), w1 = ex.ld16(at + 16u, pr);
                     uint32_t spins = 0;
                     while (seen64(seen64(1u, w0), w1) == 0u) {
-                        if (!spin_more(spins, limit, a.bar)) {
+                        if (!spin_more(spins, need, a.bar)) {
                             s_abort = 1;
                             break;
                         }
@@ -951,7 +970,7 @@ __global__ __launch_bounds__(resident_lanes(GPB)) void k_bbpgd_resident(Resident
             }
             gather(rg.X(xs));
             if (!fold(it < 0 ? 2 : 3, tot)) return;
-            limit = kResSpin;
+            need = 0u;
             ++ue;
             pe = pe == 2 ? 0 : pe + 1;
             ++mv;
@@ -1284,7 +1303,7 @@ HipErr launch_resident(hipStream_t st, const ResidentArgs<T> &r, int gpb, int gr
     const Regions g = regions<T>(r.s.m, r.s.n, r.s.nchunks);
     const uint32_t mx = std::max(std::max((2 * g.u + 3 * g.p) / 8, r.s.m * (uint32_t)(Form<T>::xg / 8)), (uint32_t)kBarTotalWords);
     k_resident_reset<T><<<(mx + 255) / 256, 256, 0, st>>>(static_cast<unsigned char *>(r.ex), g, r.s.xg, r.s.m, r.s.m_dev,
-                                                          r.s.bar, keep_abort ? 1 : 0);
+                                                          r.s.bar, keep_abort ? 1 : 0, r.head, gpb, (uint32_t)grid);
     LAUNCH_CHECK();
     if constexpr (sizeof(T) == 4)
         if (gpb == 4) return launch_resident_k<T, 4>(st, r, grid);

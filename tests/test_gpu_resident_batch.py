@@ -1,0 +1,45 @@
+"""Batches on the chip whose shares wait for blocks, with systems that have nothing to solve among them (no rods, rods
+apart from each other) first, in between and last, and one of a single row: against the general kernel, to the bit."""
+import numpy as np
+import pytest
+
+from alens_amd import capi, systems
+
+from .test_gpu_parity import assert_bits
+from .test_gpu_resident import both_paths, steps
+
+pytestmark = pytest.mark.gpu
+
+
+def pair(gap, gid):
+    """Two parallel rods, their surfaces `gap` apart, in a box of their own."""
+    r = systems.RADIUS
+    rods = dict(gid=np.array([gid, gid + 1], np.int32), center=np.array([[2.0, 2.0, 2.0], [2.0, 2.0, 2.0 + 2 * r + gap]]),
+                dir=np.tile([1.0, 0.0, 0.0], (2, 1)), length=np.ones(2), radius=np.full(2, r), immovable=None)
+    return rods, dict(box_lo=(0, 0, 0), box_hi=(4, 4, 4), pbc=(0, 0, 0), monolayer=0)
+
+
+def nothing():
+    z = np.zeros
+    return (dict(gid=z(0, np.int32), center=z((0, 3)), dir=z((0, 3)), length=z(0), radius=z(0), immovable=None),
+            dict(box_lo=(0, 0, 0), box_hi=(4, 4, 4), pbc=(0, 0, 0), monolayer=0))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nsys,nmin,nmax", [(40, 2000, 14000), (2, 3000, 3001)])
+def test_systems_without_rows(monkeypatch, nsys, nmin, nmax, precision):
+    parts, cfg = systems.replicas(nsys=nsys, nmin=nmin, nmax=nmax, seed=51)
+    g = 10_000_000
+    parts = [pair(1.0, g), nothing()] + parts[:nsys // 2] + [nothing(), pair(1.0, g + 2), pair(0.01, g + 4)] + \
+        parts[nsys // 2:] + [pair(1.0, g + 6), nothing()]
+
+    def make():
+        c = capi.Context(**dict(cfg, precision=precision))
+        c.set_systems(parts)
+        return c
+    (got, info), (want, _) = both_paths(monkeypatch, lambda: steps(make, 4))
+    for s, (a, b) in enumerate(zip(got, want)):
+        assert a[:3] == b[:3] and a[0] + a[1] > 3, (s, a[:3], b[:3])
+        assert_bits(a[3], b[3], f"gamma, step {s}")
+        assert_bits(a[4], b[4], f"U, step {s}")
+    assert info["replays"] >= 1, info

@@ -55,7 +55,6 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // sentinel of an exchanged 8-byte word: a signalling NaN (as is its low half as a float)
 constexpr u64 kUnset = 0x7FF4A1E57FA1E5C0ull;
 constexpr unsigned kUnsetLo = (unsigned)kUnset, kUnsetHi = (unsigned)(kUnset >> 32);
-constexpr uint32_t kResSpin = 1u << 22;  // polls before a wait gives up (some seconds)
 
 // Agent-scope accesses of the exchange memory, 16 B wide where the data is (the sc1 bit takes a load or store
 // past the XCD's L2; a 16-byte access is two 8-byte words, each checked for itself).  One buffer holds every
@@ -169,7 +168,7 @@ __device__ inline bool spin_more(uint32_t &n, uint32_t need, uint32_t *bar) {
     if ((++n & 255u) != 0) return true;
     if (__hip_atomic_load(&bar[kBarWords], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return false;
     if (need != 0u && __hip_atomic_load(&bar[kBarTicket * kBarWords], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) n = 0;
-    if (n < kResSpin) return true;
+    if (n < kSpinLimit) return true;
     __hip_atomic_store(&bar[kBarWords], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return false;
 }

@@ -23,7 +23,6 @@ namespace alens {
 
 static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-constexpr uint32_t kSpinLimit = 1u << 26;  // barrier wait bound: sets the abort word, never hangs
 constexpr int kBlk = 1024;                  // threads per block: 4 reduction groups of 256
 constexpr int kGrp = kBlk / kRedThreads;
 

@@ -6,6 +6,10 @@
 
 namespace alens {
 
+// Polls before a wait of a solver kernel gives up, sets the abort word and leaves: a minute or so, since blocks may
+// start late beside other work on the GPU, or be held up by it.
+constexpr uint32_t kSpinLimit = 1u << 26;
+
 // partial sums of a chunk: s.s, s.y, y.y, max residual, non-finite count; cold-start residual and count
 enum : int { Q_SS = 0, Q_SY = 1, Q_YY = 2, Q_RMAX = 3, Q_NF = 4, Q_RC = 5, Q_NFC = 6 };
 // state of a system, and the modes of the two phases

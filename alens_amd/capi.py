@@ -24,7 +24,7 @@ EXPORTS = [
     "alens_set_step", "alens_get_step", "alens_step_constraints", "alens_step_euler",
     "alens_get_num_constraints", "alens_get_constraints", "alens_get_constraint_arrays", "alens_get_gamma",
     "alens_get_velocity", "alens_bcqp_solve", "alens_add_constraints", "alens_clear_constraints",
-    "alens_get_con_stress", "alens_autotune", "alens_set_graph", "alens_get_graph_info",
+    "alens_get_con_stress", "alens_autotune", "alens_set_graph", "alens_get_graph_info", "alens_get_route",
     "alens_mlp_set", "alens_mlp_get", "alens_get_features", "alens_mlp_predict", "alens_mlp_gradient",
     "alens_mlp_train", "alens_copy_probe", "alens_bcqp_solve_static", "alens_mlp_energy", "alens_mlp_train_energy",
 ]
@@ -91,6 +91,10 @@ class GraphInfo(ctypes.Structure):
         ("captures", ctypes.c_int64), ("capture_failures", ctypes.c_int64), ("overflows", ctypes.c_int64),
         ("last_failure", ctypes.c_char * 192),
     ]
+
+
+class RouteInfo(ctypes.Structure):
+    _fields_ = [("kernel", ctypes.c_int32 * 2), ("groups", ctypes.c_int32 * 2)]
 
 
 class Report(ctypes.Structure):
@@ -292,6 +296,13 @@ class Context:
         return dict(captured=g.captured, replays=g.replays, captures=g.captures,
                     capture_failures=g.capture_failures, overflows=g.overflows,
                     last_failure=g.last_failure.decode(errors="replace"))
+
+    def route(self):
+        """Kernel of the last FP64 and FP32 solve (alens_get_route): "stream", "chip1", "chip2" or "chip4" (on the
+        chip, by row groups of a block), "block", or None."""
+        r = RouteInfo()
+        self._check(lib().alens_get_route(self._h, ctypes.byref(r)))
+        return tuple((None, "stream", f"chip{g}", "block")[k] for k, g in zip(r.kernel, r.groups))
 
     def autotune(self):
         """Pick the solver schedule by timing the last step's solve under candidates (alens_autotune)."""

@@ -133,6 +133,7 @@ struct alens_ctx {
         bool stream_nt[2] = {false, false};
     };
     Route route;
+    alens_route_info ran{};                // the last solve's kernels
     DBuf<SysDev> sys_one;                  // the one system of a stand-alone solve
     DBuf<int32_t> zeros;                   // its rods' system
     DBuf<int32_t> plan;
@@ -742,6 +743,12 @@ static alens_ctx::Route want_route(const alens_ctx *ctx, double rows, double slo
     return r;
 }
 
+// the kernel of the last solve in FP64 (form 0) or FP32, for alens_get_route
+static void note_route(alens_ctx *ctx, int form, bool planned) {
+    ctx->ran.kernel[form] = !planned ? 1 : (form == 0 && ctx->route.alone != kAloneNever ? 3 : 2);
+    ctx->ran.groups[form] = ctx->ran.kernel[form] == 2 ? ctx->route.gpb[form] : 0;
+}
+
 template <typename T>
 static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem &mem, alens_solve_report *rep,
                                  float *ms_solve, std::vector<alens_solve_report> *per_sys);
@@ -774,6 +781,7 @@ static alens_status run_bbpgd_on(alens_ctx *ctx, SolveArgsT<T> a, const SolveMem
     // (in a captured step an abort of the FP32 launch must reach the step's tail past the FP64 one)
     const bool keep_abort = ctx->capture && !ctx->bar_clean;
     const bool alone = mem.plan && form == 0 && ctx->route.alone != kAloneNever;
+    note_route(ctx, form, mem.plan != nullptr);
     if (alone) {
         // (no block waits for another: the words are neither used nor read)
     } else if (mem.plan) {
@@ -1605,6 +1613,8 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
         ctx->mprev = cnt[3];
         ctx->have_prev = true;
     }
+    for (int f = 0; f <= ctx->cfg.precision; ++f)
+        note_route(ctx, f, ctx->route.gpb[f] || (f == 0 && ctx->route.alone != kAloneNever));
     ctx->ext_step.clear();
     ctx->have_step = true;
     ++ctx->graph_steps;
@@ -1685,6 +1695,12 @@ alens_status alens_get_graph_info(const alens_ctx *ctx, alens_graph_info *info) 
     info->capture_failures = ctx->graph_capfail;
     info->overflows = ctx->graph_overflows;
     snprintf(info->last_failure, sizeof info->last_failure, "%s", ctx->graph_err.c_str());
+    return ALENS_OK;
+}
+
+alens_status alens_get_route(const alens_ctx *ctx, alens_route_info *info) {
+    if (!ctx || !info) return ALENS_E_ARG;
+    *info = ctx->ran;
     return ALENS_OK;
 }
 

@@ -159,6 +159,14 @@ typedef struct {
 } alens_graph_info;
 alens_status alens_get_graph_info(const alens_ctx *ctx, alens_graph_info *info);
 
+/* Which kernel ran the last solve (of a step, a stand-alone call or the network's energy), [0] in FP64 and [1] in
+ * FP32; iterates and iteration counts do not depend on it. */
+typedef struct {
+    int32_t kernel[2]; /* 0 none yet, 1 operator streamed from memory, 2 operator on the chip, 3 one block */
+    int32_t groups[2]; /* kernel 2: row groups (512-row chunks) a block holds */
+} alens_route_info;
+alens_status alens_get_route(const alens_ctx *ctx, alens_route_info *info);
+
 /* One constraint step (rodSystem.runStep(), SRC/TubuleSystem.cpp:223): U_nc = M F_ext + U_B,
  * collision collection, BBPGD to tol, write-back F_con = D gamma, U = U_nc + M F_con.
  * f_ext is 6n (force, torque per rod) or NULL. */

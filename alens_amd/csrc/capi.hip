@@ -1412,12 +1412,18 @@ static alens_status plan_resident(alens_ctx *ctx) {
     ctx->route = want_route(ctx, 1.04 * (double)ctx->m, 1.04 * (double)ctx->slots);
     for (int f = 0; f < 2; ++f)
         if ((double)ctx->slots > ctx->resident_limit[f]) ctx->route.gpb[f] = 0;
+    const size_t exchange = resident_exchange_bytes<double>(c.M, n, c.nch);
+    for (int f = 0; f < 2; ++f)
+        if (ctx->route.gpb[f] && exchange >= 0xffffffffull) {  // its offsets are 32 bits; tried again with fewer slots
+            ctx->route.gpb[f] = 0;
+            ctx->resident_limit[f] = 0.9 * (double)ctx->slots;
+        }
     if (ctx->route.alone != kAloneNever) ctx->route.alone = kAloneOnly;  // (the launch is fixed)
     for (int q = 0; q < 2; ++q)  // (the solve's launch decides from the same count)
         ctx->route.stream_nt[q] = general_iter_bytes(q == 0 ? 8 : 4, (double)ctx->m, n) > kLastLevelCacheBytes;
     TRY_HIP(ctx->plan.ensure(kPlanWords));
     if (ctx->route.gpb[0] || ctx->route.gpb[1]) {
-        TRY_HIP(ctx->rex.ensure(resident_exchange_bytes<double>(c.M, n, c.nch)));
+        TRY_HIP(ctx->rex.ensure(exchange));
     }
     if (ctx->cfg.warm_start == 2) TRY_HIP(ctx->feat.ensure(16 * (size_t)c.M));
     if (ctx->cfg.precision == 1) {

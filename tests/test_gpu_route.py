@@ -55,3 +55,32 @@ def test_steps(kind, n, precision, want):
             seen.append(c.route())
             c.euler()
         assert seen[2:] == [want, want], (rows, seen)
+
+
+@pytest.mark.parametrize("headroom,want", [(None, "chip2"), ("8", "stream")])
+def test_exchange_memory_past_4_gib(monkeypatch, headroom, want):
+    """11 million rows in 256 systems: a captured step whose capacities need more exchange memory than 32-bit offsets
+    reach streams its operator; with less head room it runs on the chip.  The plain step before it has the same rows."""
+    if headroom:
+        monkeypatch.setenv("ALENS_GRAPH_HEADROOM", headroom)
+    parts, off = [], 0
+    for q in range(256):
+        rods, cfg = systems.scaled("monolayer_slab", 6500, seed=q)
+        parts.append((dict(rods, gid=rods["gid"] + off), {k: cfg[k] for k in ("box_lo", "box_hi", "pbc", "monolayer")}))
+        off += 6500
+    with capi.Context(**dict(systems.COMMON, max_ite=3)) as c:
+        c.set_systems(parts)
+        c.sort_rods()
+        c.set_graph(True)
+        reps, routes, gam = [], [], []
+        for _ in range(3):
+            reps.append(c.step())
+            routes.append(c.route()[0])
+            gam.append(c.gamma())
+        info = c.graph_info()
+    assert reps[0]["n_con"] * 8 * 48 + off * 96 > 1 << 32, reps[0]  # three (x, g) pairs a row, two velocities a rod
+    assert routes == ["chip2", want, want], routes
+    assert info["captures"] == 1 and info["replays"] == 2, info
+    for r, g in zip(reps[1:], gam[1:]):
+        assert (r["n_con"], r["iters"]) == (reps[0]["n_con"], reps[0]["iters"])
+        assert np.array_equal(g.view(np.uint64), gam[0].view(np.uint64))

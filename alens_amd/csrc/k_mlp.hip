@@ -231,13 +231,14 @@ HipErr launch_mlp_infer_xg(hipStream_t st, uint32_t m, const float *X, const flo
 // layer through memory (35 launches, FP32 activations) it took 180 us, in this form 19 us and 4.6 us for the sum
 // over the blocks with the Adam step.
 // ------------------------------------------------------------------------------------------------
-// Sigmoid-weighted unit and its slope.  The quotients 1 / e and z / e share one reciprocal; residuals in one
-// rounding bring each to the correctly rounded quotient.  (e is capped where its reciprocal, below the normal range,
-// would be taken for 0.)
+// Sigmoid-weighted unit and its slope.  The quotients 1 / e and z / e share one reciprocal, refined by Newton's
+// iteration; a residual step of its own then corrects each.  Far below zero, where the reciprocal leaves the normal
+// range, both are 0 (e is capped there, or its residuals would be undefined).
 __device__ inline void silu2(float z, float &h, float &g) {
     const float e = fminf(1.0f + __expf(-z), 0x1p125f);
     float r = __builtin_amdgcn_rcpf(e);
     r = fmaf(fmaf(-e, r, 1.0f), r, r);
+    r = z < -86.5f ? 0.0f : r;
     float s = fmaf(fmaf(-e, r, 1.0f), r, r);
     s = fmaf(fmaf(-e, s, 1.0f), r, s);
     h = z * r;

@@ -721,10 +721,12 @@ static int resident_gpb(double chunks, int32_t nsys, int blocks) {
 }
 
 // The kernels for a step of `rows` rows and `slots` padded adjacency slots: resident where the operator fits
-// on the chip (the plan on the device has the last word; it fills a block's slots to 15/16), else general.  The
-// resident kernel is the faster one wherever it fits: per iteration 8.1 us against 29 at 22.8k rows, 10.6 against 29
-// at 107k, in FP32 22.9 against 31 at 472k, near the largest it holds; a batch's systems, which then stop and
-// start one by one, 8.1 ms against 10.8 for 64 systems of 1.37M rows.
+// on the chip (the plan on the device has the last word; it fills a block's slots to 15/16), else general.  For one
+// system the resident kernel is the faster one wherever it fits.  Per iteration, relaxed slabs: 8.1 us against 29 at
+// 22.8k rows, 10.6 against 29 at 107k, in FP32 22.9 against 31 at 472k; first steps of slabs and boxes: 14.0 against 54
+// at 206k rows, 18.7 against 43 at 198k, in FP32 20 against 51 at 309k and 22 against 38 at 296k, near the
+// largest it holds; rows with a rod of 64 to 2,000 rows among them: 0.17 to 0.36 of the general kernel's time.  Batches,
+// whose systems may have to take turns: see k_resident_plan.
 static alens_ctx::Route want_route(const alens_ctx *ctx, double rows, double slots) {
     alens_ctx::Route r;
     r.stream_nt[0] = general_iter_bytes(8, rows, ctx->n) > kLastLevelCacheBytes;
@@ -1252,6 +1254,9 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
         ctx->slots = ep;
         ctx->nchunks_cur = head[3];
         ctx->nsys_cur = ctx->nsys;
+        if (ctx->nsys > 1)  // (a batch's captured steps would find the same)
+            for (int f = 0; f < 2; ++f)
+                if (ctx->route.gpb[f] && head[f * kPlanHead] == kPlanUnfitting) ctx->resident_limit[f] = 0.9 * (double)ep;
         accept_plan(ctx, head);
         TRY_HIP(ctx->sellK.ensure(std::max<size_t>(ep, 1)));
         TRY_HIP(ctx->sellW.ensure(6 * std::max<size_t>(ep, 1)));

@@ -198,12 +198,32 @@ __device__ inline uint32_t share_cut(const uint32_t *sellStart, uint32_t r0, uin
 
 // How the systems are cut into shares, one per block, for the FP64 and the FP32 solve: a system takes as
 // many shares as its chunks need, or its slots at 15/16 of the LDS.  The plan fits when every share does (slots
-// in LDS, chunks in the block's lanes) and no system has more shares than the launch has blocks.  In a captured
-// step a wanted plan that does not fit clears the step's rows, and the host redoes the step.
+// in LDS, chunks in the block's lanes), no system has more shares than the launch has blocks and the systems do not
+// take too many turns (turns_ok).  In a captured step a wanted plan that does not fit clears the step's rows, and the
+// host redoes the step.
+//
+// Systems whose shares do not all have blocks take turns, and in a turn the blocks that are left over wait; the general
+// kernel takes all systems at once.  Whether the turns are shorter depends on how they fill the blocks and on how
+// the systems' iterations differ.  Solve times here over those of the general kernel, at three states of a relaxing
+// batch each (rods per system; boxes, slabs, or both in turn):
+//   FP64  up to 3 turns               3 boxes of 40,000 0.45-0.70, 6 boxes of 40,000 0.71-0.96, 12 slabs of 16,000 0.55-0.62
+//         more, 3 systems at a time   64 of 2,000-20,000 0.56-0.86, 100 of 4,000 0.49-0.67, 24 boxes of 16,000 0.70-1.00,
+//                                     64 of 2,000-50,000 0.98-1.05
+//         more, fewer at a time       8 boxes of 30,000 1.02-1.13, of 34,000 1.15-1.29; 12 boxes of 22,000 0.82-1.07
+//   FP32  1 turn                      5 boxes of 26,000 0.50-0.55, 4 slabs of 30,000 0.53-0.65
+//         2 turns, 3 at a time        12 boxes of 16,000 0.54-0.85, 8 slabs of 30,000 0.78-0.90, 8 boxes of 30,000 0.85-1.02
+//         2 turns, fewer at a time    4 boxes of 60,000 1.03-1.09, 3 slabs of 80,000 0.93-1.13
+//         more                        8 boxes of 34,000 1.23-1.52, 24 boxes of 16,000 0.81-1.20, 64 of 2,000-50,000 1.27-1.42
+__device__ inline bool turns_ok(int f, int turns, int solving) {
+    const bool three = 3 * turns <= solving;
+    return f == 0 ? turns <= 3 || three : turns == 1 || (turns == 2 && three);
+}
+
 __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
     __shared__ uint32_t s_off[kMaxSys + 1];
     __shared__ int s_bad;
     __shared__ uint32_t s_most;
+    __shared__ int s_next[kMaxSys], s_solving;
     const int t = threadIdx.x;
     int unfit = 0;
     for (int f = 0; f < 2; ++f) {
@@ -230,6 +250,7 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
         if (t == 0) {
             s_bad = gpb == 0 || (f == 0 && a.alone == kAloneOnly);
             s_most = 1;
+            s_solving = 0;
         }
         __syncthreads();
         if (t < a.nsys && gpb > 0 && !s_bad) {
@@ -255,6 +276,23 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
         }
         const uint32_t total = s_off[a.nsys];
         if (t == 0 && total > (uint32_t)kPlanShares) s_bad = 1;
+        if (total > a.max_shares[f]) {
+            if (t < a.nsys) {  // the system that starts the turn after the one that system t starts
+                int lo = t + 1, hi = a.nsys;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_off[mid] - s_off[t] <= a.max_shares[f]) lo = mid; else hi = mid - 1;
+                }
+                s_next[t] = lo;
+                if (a.chunk_off[t + 1] > a.chunk_off[t]) atomicAdd(&s_solving, 1);
+            }
+            __syncthreads();
+            if (t == 0) {
+                int turns = 0;
+                for (int q = 0; q < a.nsys; q = s_next[q]) ++turns;
+                if (!turns_ok(f, turns, s_solving)) s_bad = 1;
+            }
+        }
         __syncthreads();
         if (!s_bad) {
             for (uint32_t v = t; v < total; v += 256) {

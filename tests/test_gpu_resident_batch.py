@@ -43,3 +43,39 @@ def test_systems_without_rows(monkeypatch, nsys, nmin, nmax, precision):
         assert_bits(a[3], b[3], f"gamma, step {s}")
         assert_bits(a[4], b[4], f"U, step {s}")
     assert info["replays"] >= 1, info
+
+
+@pytest.mark.parametrize("kind,nsys,n,precision,want", [
+    ("monolayer_slab", 5, 9000, 0, ("chip2", None)),       # two turns
+    ("lognormal_3d", 6, 38000, 0, ("chip2", None)),        # three, two systems at a time
+    ("lognormal_3d", 8, 34000, 0, ("stream", None)),       # eight, one at a time
+    ("lognormal_3d", 24, 16000, 0, ("chip2", None)),       # eight, three at a time
+    ("monolayer_slab", 5, 4000, 1, ("chip2", "chip2")),    # FP32: one turn
+    ("lognormal_3d", 12, 16000, 1, ("chip2", "chip4")),    # two, nine at a time
+    ("lognormal_3d", 4, 60000, 1, ("stream", "stream")),   # two, two at a time
+    ("lognormal_3d", 24, 16000, 1, ("chip2", "stream"))])  # four
+def test_turns(monkeypatch, kind, nsys, n, precision, want):
+    """Batches that take turns on the chip, or too many of them: the kernel, the bits, and no captured step in vain."""
+    parts, first = [], 0
+    for q in range(nsys):
+        rods, cfg = systems.scaled(kind, n, seed=7 * q + 1)
+        parts.append((dict(rods, gid=rods["gid"] + first), {k: cfg[k] for k in ("box_lo", "box_hi", "pbc", "monolayer")}))
+        first += n
+
+    def run():
+        out = []
+        with capi.Context(**dict(systems.COMMON, precision=precision, max_ite=40)) as c:
+            c.set_systems(parts)
+            c.sort_rods()
+            c.set_graph(True)
+            for _ in range(3):  # an exact-size step, then captured ones, of the same rods
+                r = c.step()
+                out.append((r["n_con"], r["iters"], r["iters_fp32"], c.gamma(), c.velocity()["u"], c.route()))
+            return out, c.graph_info()
+    (got, info), (ref, _) = both_paths(monkeypatch, run)
+    for s, (a, b) in enumerate(zip(got, ref)):
+        assert a[:3] == b[:3], (s, a[:3], b[:3])
+        assert_bits(a[3], b[3], f"gamma, step {s}")
+        assert_bits(a[4], b[4], f"U, step {s}")
+    assert [a[5] for a in got] == [want] * 3 and ref[0][5][0] == "stream", [a[5] for a in got]
+    assert info["replays"] == 2 and info["captures"] == 1 and info["overflows"] == 0, info

@@ -323,6 +323,8 @@ __global__ __launch_bounds__(256) void k_resident_plan(ResidentPlanArgs a) {
         __syncthreads();
     }
     if (a.mv && unfit) {
+        // (nor may the other form's solve start: its shares name rows that would never come)
+        if (t < 2) a.plan[kPlanHead * t] = kPlanUnfitting;
         for (int q = t; q <= a.nsys; q += 256) a.con_off[q] = a.chunk_off[q] = 0u;
         if (t == 0) {
             *a.mv = 0u;

@@ -79,3 +79,45 @@ def test_turns(monkeypatch, kind, nsys, n, precision, want):
         assert_bits(a[4], b[4], f"U, step {s}")
     assert [a[5] for a in got] == [want] * 3 and ref[0][5][0] == "stream", [a[5] for a in got]
     assert info["replays"] == 2 and info["captures"] == 1 and info["overflows"] == 0, info
+
+
+@pytest.mark.parametrize("case", ["batch", "grown"])
+def test_plan_that_suits_one_form(monkeypatch, case):
+    """Captured steps in the FP32 form where one form's plan suits and the other's does not: the step is redone, and
+    neither solve runs on the cleared one.  batch: FP64 takes turns on the chip, FP32 would take too many.  grown: the
+    rows outgrow the one block that held the FP64 solve, the FP32 solve still fits."""
+    if case == "batch":
+        parts, first = [], 0
+        for q in range(24):
+            rods, cfg = systems.scaled("monolayer_slab", 20000, seed=7 * q + 1)
+            parts.append((dict(rods, gid=rods["gid"] + first), {k: cfg[k] for k in ("box_lo", "box_hi", "pbc", "monolayer")}))
+            first += 20000
+        cfg = dict(systems.COMMON, max_ite=25)
+    else:
+        rods, cfg = systems.small_3d(n=1000, box=3.8, seed=35)
+        cfg["max_ite"] = 200
+        parts = None
+        z = rods["center"][:, 2]
+        push = np.zeros((1000, 6))
+        push[:, 2] = np.where(z > np.median(z), -400.0, 400.0)
+
+    def run():
+        out = []
+        with capi.Context(**dict(cfg, precision=1)) as c:
+            c.set_systems(parts) if parts else c.set_rods(rods)
+            c.sort_rods()
+            c.set_graph(True)
+            for s in range(5 if parts else 14):
+                r = c.step(f_ext=None if parts else push if s >= 2 else 0 * push)
+                out.append((r["n_con"], r["iters"], r["iters_fp32"], c.gamma(), c.velocity()["u"], c.route()))
+                c.euler()
+            return out, c.graph_info()
+    (got, info), (ref, _) = both_paths(monkeypatch, run)
+    for s, (a, b) in enumerate(zip(got, ref)):
+        assert a[:3] == b[:3], (s, a[:3], b[:3])
+        assert_bits(a[3], b[3], f"gamma, step {s}")
+        assert_bits(a[4], b[4], f"U, step {s}")
+    seen = [(a[0], a[5]) for a in got]
+    assert info["overflows"] >= 1 and info["replays"] >= 1, (info, seen)
+    want = ("chip2", "stream") if parts else ("block", "chip1")
+    assert {want, ("stream", "stream") if parts else ("chip1", "chip1")} <= {r for _, r in seen}, (info, seen)

@@ -695,6 +695,10 @@ struct SolveMem {
     int32_t *plan;        // the rows' resident plan, or NULL: the general kernel
 };
 
+// Slots below which captures try the chip again after a plan that did not suit `slots` of them: a try in vain costs a
+// step, and a batch's turns change less with its slots than whether one system fits.
+static double retry_slots(const alens_ctx *ctx, double slots) { return (ctx->nsys > 1 ? 0.8 : 0.9) * slots; }
+
 // An explicit schedule in the environment names the general kernel, whose schedule it is.
 static bool schedule_named() {
     for (const char *v : {"ALENS_SOLVER_MAX_BLOCKS", "ALENS_BARRIER_MODE", "ALENS_XCD_MAP", "ALENS_SOLVER_ENTRIES",
@@ -1256,7 +1260,8 @@ static alens_status step_plain(alens_ctx *ctx, const double *f_ext, alens_solve_
         ctx->nsys_cur = ctx->nsys;
         if (ctx->nsys > 1)  // (a batch's captured steps would find the same)
             for (int f = 0; f < 2; ++f)
-                if (ctx->route.gpb[f] && head[f * kPlanHead] == kPlanUnfitting) ctx->resident_limit[f] = 0.9 * (double)ep;
+                if (ctx->route.gpb[f] && head[f * kPlanHead] == kPlanUnfitting)
+                    ctx->resident_limit[f] = std::min(ctx->resident_limit[f], retry_slots(ctx, (double)ep));
         accept_plan(ctx, head);
         TRY_HIP(ctx->sellK.ensure(std::max<size_t>(ep, 1)));
         TRY_HIP(ctx->sellW.ensure(6 * std::max<size_t>(ep, 1)));
@@ -1421,7 +1426,7 @@ static alens_status plan_resident(alens_ctx *ctx) {
     for (int f = 0; f < 2; ++f)
         if (ctx->route.gpb[f] && exchange >= 0xffffffffull) {  // its offsets are 32 bits; tried again with fewer slots
             ctx->route.gpb[f] = 0;
-            ctx->resident_limit[f] = 0.9 * (double)ctx->slots;
+            ctx->resident_limit[f] = retry_slots(ctx, (double)ctx->slots);
         }
     if (ctx->route.alone != kAloneNever) ctx->route.alone = kAloneOnly;  // (the launch is fixed)
     for (int q = 0; q < 2; ++q)  // (the solve's launch decides from the same count)
@@ -1592,7 +1597,7 @@ static alens_status step_resident(alens_ctx *ctx, const double *f_ext, alens_sol
         // the plain redo starts from the same previous-step impulses
         drop_graph(ctx);
         for (int f = 0; f < 2; ++f)
-            if ((unfit & (1 << f)) && !(f == 0 && ctx->route.alone)) ctx->resident_limit[f] = 0.9 * (double)cnt[2];
+            if ((unfit & (1 << f)) && !(f == 0 && ctx->route.alone)) ctx->resident_limit[f] = retry_slots(ctx, (double)cnt[2]);
         ++ctx->graph_overflows;
         return step_plain(ctx, f_ext, rep_out);
     }

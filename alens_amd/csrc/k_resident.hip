@@ -27,15 +27,16 @@
 // Sums, products and their order are those of the general kernel: results are bit-identical.
 //
 // An iteration is bound by its chain of round trips past the L2 (about 1 us each: velocities, then (x, g) and
-// the partials together), by the lane requests of a CU (about one per ns) and, with one or two waves per SIMD, by
-// the number of instructions.  So words travel 16 B at a time; velocities are held by slice position (a share's
+// the partials together) and by the lane requests of a CU (about one per ns): waves wait for data or for other blocks
+// in 63-67% of their cycles, and for their turn to issue in 12% (FP64, one group) to 22% (FP32, four groups).  So words travel 16 B at a time; velocities are held by slice position (a share's
 // are consecutive) and fetched once per block; strides of the LDS are constants; what only the start needs stays
 // out of the loop's registers.  Microseconds per iteration, general kernel -> here (slab and box systems in their
 // sorted order, FP64 unless noted): 22.8k rows 29 -> 8.1, 107k 29 -> 10.6, 183k in FP32 33 -> 12.6, 472k in FP32
 // 31 -> 22.9; 64 systems of 1.37M rows together (each waits only for itself) 10.8 -> 8.1 ms.
 //
 // Systems do not meet each other at all: a block belongs to one system at a time, takes (system, share)
-// pairs from a counter in order, and so the blocks of the first unfinished system are always running.
+// pairs from a counter in order, and so the blocks of the first unfinished system are always running.  A batch in
+// which too few systems can run at a time is left to the general kernel (turns_ok).
 #include <algorithm>
 #include <type_traits>
 
